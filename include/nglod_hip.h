@@ -413,8 +413,13 @@ int nglod_sdf_bwd(const nglod_model_t* model, const float* x, int64_t n, int32_t
 /* ---- training targets and samples ------------------------------------- */
 
 /* Workspace bytes nglod_mesh2sdf_f64 needs for nf triangles (per-triangle
- * FP64 table). */
+ * FP64 table, sort buffers and the tree over the triangles). */
 size_t nglod_mesh2sdf_workspace_size(int64_t nf);
+
+/* Workspace bytes with which nglod_mesh2sdf_f64 also visits n points in
+ * spatial order (the same results; the points of a wave then need the same
+ * triangles). */
+size_t nglod_mesh2sdf_ordered_workspace_size(int64_t n, int64_t nf);
 
 /* Signed distance from points [n][3] to a closed triangle mesh [nf][3][3],
  * computed in FP64.  Replaces mesh2sdf.mesh2sdf_gpu
@@ -422,7 +427,9 @@ size_t nglod_mesh2sdf_workspace_size(int64_t nf);
  * :1009, called from sdf-net/lib/torchgp/compute_sdf.py:38): unsigned distance
  * by the edge/face rule of :423-445, negative iff all 13 stab directions
  * (:341-353) have a hit on both sides of the point (:479-529, :584-602).
- * dist [n] fp32; dist64 [n] fp64 (may be NULL). */
+ * dist [n] fp32; dist64 [n] fp64 (may be NULL).  workspace: 8-byte aligned, at
+ * least nglod_mesh2sdf_workspace_size(nf) bytes; the points are ordered when it
+ * has nglod_mesh2sdf_ordered_workspace_size(n, nf). */
 int nglod_mesh2sdf_f64(const float* points, int64_t n, const float* mesh, int64_t nf, float* dist,
                        double* dist64, void* workspace, size_t workspace_bytes, void* stream);
 

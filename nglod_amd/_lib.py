@@ -150,6 +150,7 @@ SIGNATURES = {
                                            _p, _p, _sz, ctypes.POINTER(_sz), _p]),
     "nglod_mark_unique_rays": (ctypes.c_int, [_p, _i64, _p, _p]),
     "nglod_mesh2sdf_workspace_size": (_sz, [_i64]),
+    "nglod_mesh2sdf_ordered_workspace_size": (_sz, [_i64, _i64]),
     "nglod_mesh2sdf_f64": (ctypes.c_int, [_p, _i64, _p, _i64, _p, _p, _p, _sz, _p]),
     "nglod_sample_uniform": (ctypes.c_int, [_i64, ctypes.c_uint64, _p, _p]),
     "nglod_sample_surface": (ctypes.c_int, [_p, _p, _i64, _i64, ctypes.c_uint64, ctypes.c_double, _p, _p, _p]),

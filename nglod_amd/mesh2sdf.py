@@ -30,7 +30,7 @@ def mesh2sdf_gpu(points, mesh):
     dist = torch.empty(n, dtype=torch.float32, device=p.device)
     if n:
         lib = _lib.load()
-        ws = torch.empty(max(1, lib.nglod_mesh2sdf_workspace_size(nf)), dtype=torch.uint8, device=p.device)
+        ws = torch.empty(max(1, lib.nglod_mesh2sdf_ordered_workspace_size(n, nf)), dtype=torch.uint8, device=p.device)
         _lib.check(lib.nglod_mesh2sdf_f64(_lib.ptr(p), n, _lib.ptr(tris), nf, _lib.ptr(dist), None, _lib.ptr(ws),
                                           ws.numel(), _lib.stream_of(p)), "nglod_mesh2sdf_f64")
     return [dist]

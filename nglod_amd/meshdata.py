@@ -14,7 +14,7 @@ from . import _lib, mesh as _mesh
 
 
 class MeshData:
-    """Triangles, face-area CDF and the mesh2sdf workspace on one device."""
+    """Triangles and face-area CDF on one device."""
 
     def __init__(self, V, F, device="cuda"):
         V = np.asarray(V, dtype=np.float32)
@@ -26,9 +26,6 @@ class MeshData:
         self.tris = torch.from_numpy(np.ascontiguousarray(tris)).to(self.device)
         self.cdf = torch.from_numpy(_mesh.face_cdf(tris)).to(self.device)
         self.nf = tris.shape[0]
-        lib = _lib.load()
-        self._ws = torch.empty(max(1, lib.nglod_mesh2sdf_workspace_size(self.nf)), dtype=torch.uint8,
-                               device=self.device)
 
     def sdf(self, pts, with_f64=False):
         """Signed distance of pts [N, 3] (FP64 arithmetic); [N] fp32 (and fp64)."""
@@ -38,9 +35,11 @@ class MeshData:
         out = torch.empty(n, dtype=torch.float32, device=p.device)
         out64 = torch.empty(n, dtype=torch.float64, device=p.device) if with_f64 else None
         lib = _lib.load()
+        ws = torch.empty(max(1, lib.nglod_mesh2sdf_ordered_workspace_size(n, self.nf)), dtype=torch.uint8,
+                         device=p.device)
         _lib.check(lib.nglod_mesh2sdf_f64(_lib.ptr(p), n, _lib.ptr(self.tris), self.nf, _lib.ptr(out),
-                                          _lib.ptr(out64), _lib.ptr(self._ws), self._ws.numel(),
-                                          _lib.stream_of(p)), "nglod_mesh2sdf_f64")
+                                          _lib.ptr(out64), _lib.ptr(ws), ws.numel(), _lib.stream_of(p)),
+                   "nglod_mesh2sdf_f64")
         return (out, out64) if with_f64 else out
 
     def sample_uniform(self, n, seed):
