@@ -410,6 +410,23 @@ int nglod_sdf_bwd(const nglod_model_t* model, const float* x, int64_t n, int32_t
                   const float* grad_out, int32_t level_mask, const nglod_model_grads_t* grads,
                   void* workspace, size_t workspace_bytes, void* stream);
 
+/* The training forward: nglod_sdf_fwd_all's predictions (the same bits), and
+ * in `saved` (nglod_sdf_fwd_save_bytes bytes, 16-byte aligned: 164 bytes per
+ * query and level at most) what nglod_sdf_bwd_saved then need not compute again:
+ * the spatial order of the queries, their features and the signs of the
+ * decoders' pre-activations.  n <= 2^28. */
+size_t nglod_sdf_fwd_save_bytes(const nglod_model_t* model, int64_t n, int32_t lod);
+size_t nglod_sdf_fwd_save_workspace_size(int64_t n);
+int nglod_sdf_fwd_save(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, float* out, void* saved,
+                       size_t saved_bytes, void* workspace, size_t workspace_bytes, void* stream);
+
+/* nglod_sdf_bwd on what nglod_sdf_fwd_save left for the same model, x, n and
+ * lod; the same gradients, bit for bit. */
+size_t nglod_sdf_bwd_saved_workspace_size(const nglod_model_t* model, int64_t n, int32_t lod);
+int nglod_sdf_bwd_saved(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, const float* grad_out,
+                        int32_t level_mask, const nglod_model_grads_t* grads, void* saved, size_t saved_bytes,
+                        void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- training targets and samples ------------------------------------- */
 
 /* Workspace bytes nglod_mesh2sdf_f64 needs for nf triangles (per-triangle

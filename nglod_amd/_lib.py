@@ -140,6 +140,12 @@ SIGNATURES = {
     "nglod_sdf_bwd_workspace_size": (_sz, [ctypes.POINTER(NglodModel), _i64, _i32]),
     "nglod_sdf_bwd": (ctypes.c_int, [ctypes.POINTER(NglodModel), _p, _i64, _i32, _p, _i32,
                                       ctypes.POINTER(NglodModelGrads), _p, _sz, _p]),
+    "nglod_sdf_fwd_save_bytes": (_sz, [ctypes.POINTER(NglodModel), _i64, _i32]),
+    "nglod_sdf_fwd_save_workspace_size": (_sz, [_i64]),
+    "nglod_sdf_fwd_save": (ctypes.c_int, [ctypes.POINTER(NglodModel), _p, _i64, _i32, _p, _p, _sz, _p, _sz, _p]),
+    "nglod_sdf_bwd_saved_workspace_size": (_sz, [ctypes.POINTER(NglodModel), _i64, _i32]),
+    "nglod_sdf_bwd_saved": (ctypes.c_int, [ctypes.POINTER(NglodModel), _p, _i64, _i32, _p, _i32,
+                                            ctypes.POINTER(NglodModelGrads), _p, _sz, _p, _sz, _p]),
     "nglod_spc_occupancy": (ctypes.c_int, [_p, _i64, _i32, _p, _i64, ctypes.POINTER(_i64), _p, _sz,
                                             ctypes.POINTER(_sz), _p]),
     "nglod_spc_from_codes": (ctypes.c_int, [_p, _i64, _i32, _p, _i64, ctypes.POINTER(_i64), _p, _p, _sz,

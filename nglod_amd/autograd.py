@@ -26,6 +26,15 @@ def _param_slots(net):
     return slots
 
 
+# The forward of every level keeps its features for the backward (164 bytes per
+# query and level) up to this many bytes; a larger batch computes them again.
+SAVE_LIMIT = 4 << 30
+
+
+def _versions(net):
+    return tuple((p.data_ptr(), p._version) for p in net.parameters())
+
+
 class _SdfFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, net, x, lod, all_levels, *params):
@@ -35,6 +44,20 @@ class _SdfFunction(torch.autograd.Function):
         xf = x.detach().reshape(-1, 3).float().contiguous()
         ctx.x_shape = x.shape
         ctx.x_dtype = x.dtype
+        n = xf.shape[0]
+        if all_levels and n > 0 and any(ctx.needs_input_grad[4:]):
+            lib = _lib.load()
+            m = net.descriptor(_lib.FP32)
+            nbytes = lib.nglod_sdf_fwd_save_bytes(m, n, lod)
+            if nbytes <= SAVE_LIMIT and n <= 1 << 28:
+                out = torch.empty(lod + 1, n, 1, device=x.device, dtype=torch.float32)
+                saved = torch.empty(nbytes, device=x.device, dtype=torch.uint8)
+                ws = torch.empty(lib.nglod_sdf_fwd_save_workspace_size(n), device=x.device, dtype=torch.uint8)
+                _lib.check(lib.nglod_sdf_fwd_save(m, _lib.ptr(xf), n, lod, _lib.ptr(out), _lib.ptr(saved), nbytes,
+                                                  _lib.ptr(ws), ws.numel(), _lib.stream_of(x)), "nglod_sdf_fwd_save")
+                ctx.versions = _versions(net)
+                ctx.save_for_backward(xf, saved)
+                return out
         ctx.save_for_backward(xf)
         if all_levels:
             return torch.stack(net.sdf_all_hip(xf, lod), 0)
@@ -43,7 +66,7 @@ class _SdfFunction(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, grad_out):
-        (x,) = ctx.saved_tensors
+        x, *saved = ctx.saved_tensors
         net, L = ctx.net, ctx.lod
         n = x.shape[0]
         dev = x.device
@@ -79,10 +102,18 @@ class _SdfFunction(torch.autograd.Function):
                 getattr(G, key)[d] = t.data_ptr()
         m = net.descriptor(_lib.FP32)
         lib = _lib.load()
-        nbytes = lib.nglod_sdf_bwd_workspace_size(m, n, L)
-        ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=dev)
-        _lib.check(lib.nglod_sdf_bwd(m, _lib.ptr(x), n, L, _lib.ptr(g), mask, G, _lib.ptr(ws), ws.numel(),
-                                     _lib.stream_of(x)), "nglod_sdf_bwd")
+        # features of other weights are not the features of these: computed again
+        if saved and ctx.versions == _versions(net):
+            nbytes = lib.nglod_sdf_bwd_saved_workspace_size(m, n, L)
+            ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=dev)
+            _lib.check(lib.nglod_sdf_bwd_saved(m, _lib.ptr(x), n, L, _lib.ptr(g), mask, G, _lib.ptr(saved[0]),
+                                               saved[0].numel(), _lib.ptr(ws), ws.numel(), _lib.stream_of(x)),
+                       "nglod_sdf_bwd_saved")
+        else:
+            nbytes = lib.nglod_sdf_bwd_workspace_size(m, n, L)
+            ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=dev)
+            _lib.check(lib.nglod_sdf_bwd(m, _lib.ptr(x), n, L, _lib.ptr(g), mask, G, _lib.ptr(ws), ws.numel(),
+                                         _lib.stream_of(x)), "nglod_sdf_bwd")
         grads = []
         for kind, idx, _ in _param_slots(net):
             if kind == "grid":

@@ -1,6 +1,9 @@
 // Hand-written backward of the fused query (OctreeSDF.sdf, every level up
 // to lod) for training, deterministic by construction (no float atomics):
 //
+// The training forward (nglod_sdf_fwd_save) runs steps 1 and 2 with the
+// predictions and leaves their results for the backward.
+//
 //   1. the queries are visited in the Morton order of their cell in the
 //      finest grid ("positions"), so that neighbouring lanes share corners;
 //   2. features: per position and level the running trilinear features E
@@ -112,9 +115,13 @@ __device__ __forceinline__ float layer2_tile_bits(const f32x16_t& c, int h, uint
 // Features and pre-activation signs of 64 positions per wave, a persistent
 // block: the decoders of its levels stay in LDS (dynamic: one Fp32Lds each).
 // Block y takes levels l0 .. l1 of the split: all of them, or for few queries
-// one (its features still start at level 0).  decode_fp32_wave's arithmetic.
-template <bool POSINV>
-__global__ __launch_bounds__(512) void bwd_features_kernel(BwdArgs a, int split) {
+// one (its features still start at level 0).  decode_fp32_wave's arithmetic;
+// PRED: the levels' predictions too (the training forward), out [lod+1][n].
+//
+// 2^19 queries, 5 levels: the forward in query order 0.50 ms and the features
+// again in the backward 0.30 ms -> 0.34 ms for both.
+template <bool POSINV, bool PRED>
+__global__ __launch_bounds__(512) void train_features_kernel(BwdArgs a, int split, float* __restrict__ out) {
     extern __shared__ __align__(16) char dyn[];
     Fp32Lds* lds = reinterpret_cast<Fp32Lds*>(dyn);
     const int l0 = split ? (int)blockIdx.y : 0, l1 = split ? (int)blockIdx.y : a.lod;
@@ -162,8 +169,9 @@ __global__ __launch_bounds__(512) void bwd_features_kernel(BwdArgs a, int split)
                 B0[kk] = __uint_as_float(sw[0]);
                 B1[kk] = __uint_as_float(sw[1]);
             }
-            uint32_t word[4];
-#pragma unroll
+            uint32_t* word = reinterpret_cast<uint32_t*>(a.bits + (size_t)l * a.n + (valid ? pos : 0));
+            float part[2] = {0.0f, 0.0f};
+#pragma unroll 1
             for (int h = 0; h < 4; ++h) {
                 uint32_t b[2] = {0u, 0u};
 #pragma unroll
@@ -179,13 +187,17 @@ __global__ __launch_bounds__(512) void bwd_features_kernel(BwdArgs a, int split)
                         c = __builtin_amdgcn_mfma_f32_32x32x2f32(w.z, B[4 * kq + 2], c, 0, 0, 0);
                         c = __builtin_amdgcn_mfma_f32_32x32x2f32(w.w, B[4 * kq + 3], c, 0, 0, 0);
                     }
-                    (void)layer2_tile_bits(c, h, half, s, !POSINV, u == 0 ? qx0 : qx1, u == 0 ? qy0 : qy1,
-                                           u == 0 ? qz0 : qz1, b[u]);
+                    const float sum = layer2_tile_bits(c, h, half, s, !POSINV, u == 0 ? qx0 : qx1,
+                                                       u == 0 ? qy0 : qy1, u == 0 ? qz0 : qz1, b[u]);
+                    if (PRED) part[u] += sum;
                 }
                 const auto sw = __builtin_amdgcn_permlane32_swap(b[0], b[1], false, false);
-                word[h] = sw[0] | sw[1];
+                if (valid) word[h] = sw[0] | sw[1];
             }
-            if (valid) a.bits[(size_t)l * a.n + pos] = make_uint4(word[0], word[1], word[2], word[3]);
+            if (PRED) {
+                const float d = halves_sum(part[0], part[1]) + a.m.b1[joint ? 0 : l][0];
+                if (valid) out[(size_t)l * a.n + q] = d;
+            }
         }
     }
 }
@@ -500,7 +512,7 @@ __global__ __launch_bounds__(256) void bwd_runs_kernel(const uint32_t* __restric
     if (i == m - 1 || keys[i + 1] != k) runs[k].y = i + 1;
 }
 
-// Sums of the pieces that start in a window of kWindow sorted entries: piece p
+// Sums of the pieces that start in a window of `size` sorted entries: piece p
 // of a run covers its entries 64 p .. 64 p + 63, each contribution
 // w_c(x) * dg one FMA per channel, in order.  8 lanes take a piece (a float4 of
 // channels each, so a row of dg is one coalesced 128-byte access); their
@@ -511,10 +523,12 @@ __global__ __launch_bounds__(256) void bwd_runs_kernel(const uint32_t* __restric
 //
 // 2^19 queries, 5 levels: 1.13 ms with a lane per piece and the rows in query
 // order -> 0.45 ms.
+// A window is smaller where the entries would not fill the GPU (512 queries, 10
+// windows of 2048: 123 us, 80 of 256: 18 us).
 constexpr int kWindow = 2048;
 
 __global__ __launch_bounds__(256) void bwd_pieces_kernel(BwdArgs a, CornerLevels L, const uint32_t* __restrict__ keys,
-                                                         const uint32_t* __restrict__ vals, uint32_t m,
+                                                         const uint32_t* __restrict__ vals, uint32_t m, uint32_t size,
                                                          const uint2* __restrict__ runs, float* __restrict__ partial) {
     __shared__ uint32_t starts[kWindow];
     __shared__ uint32_t count;
@@ -523,9 +537,9 @@ __global__ __launch_bounds__(256) void bwd_pieces_kernel(BwdArgs a, CornerLevels
     // consecutive windows on one XCD (blocks go to the XCDs in turn): their rows share its L2
     const uint32_t per = (gridDim.x + 7) / 8;
     const uint32_t window = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
-    const uint64_t w0 = (uint64_t)window * kWindow;
+    const uint64_t w0 = (uint64_t)window * size;
     const uint32_t lane = lane_id();
-    for (int r = 0; r < kWindow / 256; ++r) {
+    for (uint32_t r = 0; r < size / 256; ++r) {
         const uint64_t i = w0 + r * 256 + threadIdx.x;
         const bool first = i < m && (((uint32_t)i - runs[keys[i]].x) & (kRunPiece - 1)) == 0;
         const uint64_t mask = __ballot(first);
@@ -663,8 +677,13 @@ __global__ __launch_bounds__(256) void bwd_fill_kernel(FillList l) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = 0.0f;
 }
 
+// What the training forward leaves for the backward.
+struct SavedLayout {
+    size_t order, rank, xs, E, bits, total;
+};
+
 struct BwdLayout {
-    size_t rank, xs, E, bits, dg, part, gpart, order, keys_in, keys_out, vals_in, vals_out, sort_tmp, runs, partial, total;
+    size_t saved, order_ws, dg, part, gpart, keys_in, keys_out, vals_in, vals_out, sort_tmp, runs, partial, total;
     size_t sort_bytes;
     int64_t nchunks, ngroups;
     bool together;  // the contributions of all levels in one sort
@@ -691,7 +710,24 @@ static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 // with 2^19.
 constexpr int64_t kTogether = (int64_t)1 << 31;
 
-static int bwd_layout(int64_t n, int lod, int din, const int32_t* res, BwdLayout* L) {
+static void saved_layout(int64_t n, int lod, SavedLayout* L) {
+    const size_t levels = (size_t)lod + 1;
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = off;
+        off += align256(bytes);
+        return at;
+    };
+    L->order = take((size_t)n * 4);
+    L->rank = take((size_t)n * 4);
+    L->xs = take((size_t)n * 3 * sizeof(float));
+    L->bits = take(levels * n * sizeof(uint4));
+    L->E = take(levels * n * kC * sizeof(float));
+    L->total = off;
+}
+
+// saved: the features come from a training forward, else the call computes them.
+static int bwd_layout(int64_t n, int lod, int din, const int32_t* res, bool saved, BwdLayout* L) {
     const size_t levels = (size_t)lod + 1;
     L->nchunks = (n + kChunk - 1) / kChunk;
     L->ngroups = (L->nchunks + kGroup - 1) / kGroup;
@@ -709,14 +745,13 @@ static int bwd_layout(int64_t n, int lod, int din, const int32_t* res, BwdLayout
     }
     L->together = (int64_t)levels * n * 8 <= kTogether && corners < ((uint64_t)1 << 31);
     const size_t m = (size_t)n * 8 * (L->together ? levels : 1);
-    L->rank = take((size_t)n * 4);
-    L->xs = take((size_t)n * 3 * sizeof(float));
-    L->E = take(levels * n * kC * sizeof(float));
-    L->bits = take(levels * n * sizeof(uint4));
+    SavedLayout S;
+    saved_layout(n, lod, &S);
+    L->saved = saved ? 0 : take(S.total);
+    L->order_ws = saved ? 0 : take(sort_workspace_bytes(n));
     L->dg = take(levels * n * kC * sizeof(float));
     L->part = take(levels * L->nchunks * outs * sizeof(float));
     L->gpart = take(levels * L->ngroups * outs * sizeof(float));
-    L->order = take(sort_workspace_bytes(n));
     L->keys_in = take(m * 4);
     L->keys_out = take(m * 4);
     L->vals_in = take(m * 4);
@@ -739,29 +774,82 @@ static int bwd_layout(int64_t n, int lod, int din, const int32_t* res, BwdLayout
     return NGLOD_OK;
 }
 
-}  // namespace nglod
-
-using namespace nglod;
-
-extern "C" {
-
-size_t nglod_sdf_bwd_workspace_size(const nglod_model_t* model, int64_t n, int32_t lod) {
-    if (!model || n < 0 || lod < 0) return 0;
-    if (lod >= model->num_lods || lod >= NGLOD_MAX_LODS) return 0;
-    BwdLayout L;
-    const int din = model->pos_invariant ? kC : kC + 3;
-    if (bwd_layout(n, lod, din, model->res, &L)) return 0;
-    return L.total;
+static BwdArgs bwd_args(const ModelArgs& m, const float* x, int64_t n, int lod, int mask, const float* g, void* saved) {
+    SavedLayout S;
+    saved_layout(n, lod, &S);
+    char* w = (char*)saved;
+    BwdArgs a;
+    a.m = m;
+    a.lod = lod;
+    a.din = m.pos_inv ? kC : kC + 3;
+    a.off = m.pos_inv ? 0 : 3;
+    a.mask = mask;
+    a.n = n;
+    a.x = x;
+    a.g = g;
+    a.order = (const uint32_t*)(w + S.order);
+    a.rank = (uint32_t*)(w + S.rank);
+    a.xs = (float*)(w + S.xs);
+    a.bits = (uint4*)(w + S.bits);
+    a.E = (float*)(w + S.E);
+    a.dg = nullptr;
+    return a;
 }
 
-int nglod_sdf_bwd(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, const float* grad_out,
-                  int32_t level_mask, const nglod_model_grads_t* grads, void* workspace, size_t workspace_bytes,
-                  void* stream) {
+// Fewer 64-query tiles than CUs: a level per block, so that the levels'
+// latencies run side by side (512 queries: 92 -> 41 us for the features); else
+// a block per CU with every level's decoder in LDS.
+struct Split {
+    int on, held, threads, cus;
+    Split(int64_t n, const ModelArgs& m, int lod) {
+        cus = device_cu_count();
+        on = (n + 63) / 64 < (int64_t)cus ? 1 : 0;
+        held = on || m.num_dec == 1 ? 1 : lod + 1;
+        threads = on ? 256 : 512;
+    }
+    dim3 grid(int64_t waves, int lod) const {
+        const int64_t want = (waves + threads / 64 - 1) / (threads / 64);
+        return dim3((unsigned)(on || want < cus ? want : cus), on ? lod + 1 : 1);
+    }
+};
+
+// Positions, features and signs of the levels in a.mask, and the predictions
+// into `out` unless NULL.
+static int launch_features(const BwdArgs& a, float* out, void* sort_ws, hipStream_t s) {
+    SortBuffers sb = sort_buffers(sort_ws, a.n);
+    const int bits = cell_bits(a.m.res[a.lod]);
+    sb.vals[sort_result(bits)] = const_cast<uint32_t*>(a.order);
+    hipLaunchKernelGGL(bwd_cell_keys_kernel, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, s, a.x, a.n,
+                       a.m.res[a.lod], sb.keys[0]);
+    launch_sort(sb, a.n, bits, s);
+    const Split sp(a.n, a.m, a.lod);
+    auto k = a.m.pos_inv ? (out ? train_features_kernel<true, true> : train_features_kernel<true, false>)
+                         : (out ? train_features_kernel<false, true> : train_features_kernel<false, false>);
+    hipLaunchKernelGGL(k, sp.grid((a.n + 63) / 64, a.lod), dim3(sp.threads), sp.held * sizeof(Fp32Lds), s, a, sp.on, out);
+    return check_launch("train_features_kernel");
+}
+
+static bool bwd_sizes_ok(const nglod_model_t* model, int64_t n, int32_t lod) {
+    return model && n >= 0 && lod >= 0 && lod < model->num_lods && lod < NGLOD_MAX_LODS;
+}
+
+static size_t bwd_workspace(const nglod_model_t* model, int64_t n, int32_t lod, bool saved) {
+    if (!bwd_sizes_ok(model, n, lod)) return 0;
+    BwdLayout L;
+    return bwd_layout(n, lod, model->pos_invariant ? kC : kC + 3, model->res, saved, &L) ? 0 : L.total;
+}
+
+constexpr int64_t kMaxQueries = (int64_t)1 << 28;
+
+// The backward; saved NULL: the features are computed here.
+static int backward(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, const float* grad_out,
+                    int32_t level_mask, const nglod_model_grads_t* grads, void* saved, size_t saved_bytes,
+                    void* workspace, size_t workspace_bytes, void* stream) {
     ModelArgs m;
     int rc = make_model_args(model, lod, NGLOD_FP32, &m);
     if (rc) return rc;
     if (n < 0) return fail(NGLOD_ERR_ARG, "n < 0");
-    if (n > ((int64_t)1 << 28)) return fail(NGLOD_ERR_ARG, "n too large for 32-bit sort values");
+    if (n > kMaxQueries) return fail(NGLOD_ERR_ARG, "n too large for 32-bit sort values");
     if (!grads) return fail(NGLOD_ERR_ARG, "grads is NULL");
     const int din = m.pos_inv ? kC : kC + 3;
     hipStream_t s = (hipStream_t)stream;
@@ -797,10 +885,14 @@ int nglod_sdf_bwd(const nglod_model_t* model, const float* x, int64_t n, int32_t
     if (!work) return fill();
     if (!x || !grad_out) return fail(NGLOD_ERR_ARG, "NULL pointer");
     BwdLayout L;
-    rc = bwd_layout(n, lod, din, model->res, &L);
+    rc = bwd_layout(n, lod, din, model->res, saved != nullptr, &L);
     if (rc) return rc;
     if (!workspace || workspace_bytes < L.total || !aligned16(workspace))
         return fail(NGLOD_ERR_WORKSPACE, "workspace too small or misaligned");
+    SavedLayout S;
+    saved_layout(n, lod, &S);
+    if (saved && (saved_bytes < S.total || !aligned16(saved)))
+        return fail(NGLOD_ERR_WORKSPACE, "saved features too small or misaligned");
     char* ws = (char*)workspace;
     uint2* runs = (uint2*)(ws + L.runs);
     if (L.together) {
@@ -811,46 +903,20 @@ int nglod_sdf_bwd(const nglod_model_t* model, const float* x, int64_t n, int32_t
     rc = fill();
     if (rc) return rc;
     const unsigned qblocks = (unsigned)((n + 255) / 256);
-    const SortBuffers sb = sort_buffers(ws + L.order, n);
-    hipLaunchKernelGGL(bwd_cell_keys_kernel, dim3(qblocks), dim3(256), 0, s, x, n, m.res[lod], sb.keys[0]);
-    const int sorted = launch_sort(sb, n, cell_bits(m.res[lod]), s);
-    BwdArgs a;
-    a.m = m;
-    a.lod = lod;
-    a.din = din;
-    a.off = m.pos_inv ? 0 : 3;
-    a.mask = level_mask;
-    a.n = n;
-    a.x = x;
-    a.g = grad_out;
-    a.order = sb.vals[sorted];
-    a.rank = (uint32_t*)(ws + L.rank);
-    a.xs = (float*)(ws + L.xs);
-    a.E = (float*)(ws + L.E);
-    a.bits = (uint4*)(ws + L.bits);
+    BwdArgs a = bwd_args(m, x, n, lod, level_mask, grad_out, saved ? saved : ws + L.saved);
     a.dg = (float*)(ws + L.dg);
     float* part = (float*)(ws + L.part);
-    // Fewer 64-query tiles than CUs: a level per block, so that the levels'
-    // latencies run side by side (512 queries: 92 -> 41 us for the features);
-    // else a block per CU with every level's decoder in LDS.
-    const int cus = device_cu_count();
-    const int64_t tiles = (n + 63) / 64;
-    const int split = tiles < (int64_t)cus ? 1 : 0;
-    const int held = split || m.num_dec == 1 ? 1 : lod + 1;
-    const int threads = split ? 256 : 512;
-    const auto blocks_for = [&](int64_t waves) {
-        const int64_t want = (waves + threads / 64 - 1) / (threads / 64);
-        return (unsigned)(split || want < cus ? want : cus);
-    };
-    const dim3 fgrid(blocks_for(tiles), split ? lod + 1 : 1), dgrid(blocks_for((n + 31) / 32), split ? lod + 1 : 1);
-    auto fk = m.pos_inv ? bwd_features_kernel<true> : bwd_features_kernel<false>;
-    hipLaunchKernelGGL(fk, fgrid, dim3(threads), held * sizeof(Fp32Lds), s, a, split);
-    rc = check_launch("bwd_features_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(bwd_ds_kernel, dgrid, dim3(threads), held * sizeof(BwdLds), s, a, split);
+    if (!saved) {
+        rc = launch_features(a, nullptr, ws + L.order_ws, s);
+        if (rc) return rc;
+    }
+    const Split sp(n, m, lod);
+    const int cus = sp.cus;
+    hipLaunchKernelGGL(bwd_ds_kernel, sp.grid((n + 31) / 32, lod), dim3(sp.threads), sp.held * sizeof(BwdLds), s, a,
+                       sp.on);
     rc = check_launch("bwd_ds_kernel");
     if (rc) return rc;
-    if (split && lod > 0)
+    if (sp.on && lod > 0)
         hipLaunchKernelGGL(bwd_suffix_kernel, dim3((unsigned)((n * (kC / 4) + 255) / 256)), dim3(256), 0, s, a);
     // decoder gradients
     auto pk = m.pos_inv ? bwd_decoder_partial_kernel<true> : bwd_decoder_partial_kernel<false>;
@@ -901,9 +967,11 @@ int nglod_sdf_bwd(const nglod_model_t* model, const float* x, int64_t n, int32_t
             hipSuccess)
             return fail(NGLOD_ERR_HIP, "radix sort failed");
         hipLaunchKernelGGL(bwd_runs_kernel, dim3((mm + 255) / 256), dim3(256), 0, s, kout, mm, runs);
-        const uint32_t windows = (mm + kWindow - 1) / kWindow;
-        hipLaunchKernelGGL(bwd_pieces_kernel, dim3((windows + 7) / 8 * 8), dim3(256), 0, s, a, C, kout, vout, mm, runs,
-                           partial);
+        uint32_t size = kWindow;
+        while (size > 256 && mm / size < 4u * (uint32_t)cus) size /= 2;
+        const uint32_t windows = (mm + size - 1) / size;
+        hipLaunchKernelGGL(bwd_pieces_kernel, dim3((windows + 7) / 8 * 8), dim3(256), 0, s, a, C, kout, vout, mm, size,
+                           runs, partial);
         if (C.strided != (1u << C.count) - 1u)
             hipLaunchKernelGGL(bwd_run_final_kernel, dim3((unsigned)(((uint64_t)corners * kC + 255) / 256)), dim3(256),
                                0, s, C, runs, partial);
@@ -920,6 +988,59 @@ int nglod_sdf_bwd(const nglod_model_t* model, const float* x, int64_t n, int32_t
         if (rc) return rc;
     }
     return NGLOD_OK;
+}
+
+}  // namespace nglod
+
+using namespace nglod;
+
+extern "C" {
+
+size_t nglod_sdf_bwd_workspace_size(const nglod_model_t* model, int64_t n, int32_t lod) {
+    return bwd_workspace(model, n, lod, false);
+}
+
+size_t nglod_sdf_bwd_saved_workspace_size(const nglod_model_t* model, int64_t n, int32_t lod) {
+    return bwd_workspace(model, n, lod, true);
+}
+
+size_t nglod_sdf_fwd_save_bytes(const nglod_model_t* model, int64_t n, int32_t lod) {
+    if (!bwd_sizes_ok(model, n, lod)) return 0;
+    SavedLayout S;
+    saved_layout(n, lod, &S);
+    return S.total;
+}
+
+size_t nglod_sdf_fwd_save_workspace_size(int64_t n) { return n > 0 ? sort_workspace_bytes(n) : 0; }
+
+int nglod_sdf_fwd_save(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, float* out, void* saved,
+                       size_t saved_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+    ModelArgs m;
+    int rc = make_model_args(model, lod, NGLOD_FP32, &m);
+    if (rc) return rc;
+    if (n < 0 || n > kMaxQueries) return fail(NGLOD_ERR_ARG, "n out of range");
+    if (n == 0) return NGLOD_OK;
+    if (!x || !out || !saved) return fail(NGLOD_ERR_ARG, "NULL pointer");
+    if (saved_bytes < nglod_sdf_fwd_save_bytes(model, n, lod) || !aligned16(saved))
+        return fail(NGLOD_ERR_WORKSPACE, "saved features too small or misaligned");
+    if (!workspace || workspace_bytes < sort_workspace_bytes(n) || !aligned16(workspace))
+        return fail(NGLOD_ERR_WORKSPACE, "workspace too small or misaligned");
+    const BwdArgs a = bwd_args(m, x, n, lod, (1 << (lod + 1)) - 1, nullptr, saved);
+    return launch_features(a, out, workspace, (hipStream_t)stream);
+}
+
+int nglod_sdf_bwd(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, const float* grad_out,
+                  int32_t level_mask, const nglod_model_grads_t* grads, void* workspace, size_t workspace_bytes,
+                  void* stream) {
+    return backward(model, x, n, lod, grad_out, level_mask, grads, nullptr, 0, workspace, workspace_bytes, stream);
+}
+
+int nglod_sdf_bwd_saved(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, const float* grad_out,
+                        int32_t level_mask, const nglod_model_grads_t* grads, void* saved, size_t saved_bytes,
+                        void* workspace, size_t workspace_bytes, void* stream) {
+    if (n > 0 && !saved) return fail(NGLOD_ERR_ARG, "NULL pointer");
+    return backward(model, x, n, lod, grad_out, level_mask, grads, saved, saved_bytes, workspace, workspace_bytes,
+                    stream);
 }
 
 }  // extern "C"

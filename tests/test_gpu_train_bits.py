@@ -80,3 +80,42 @@ def test_last_level_alone_is_the_call_at_its_lod(dev):
         assert torch.equal(a[f"features.{i}.fm"], b[f"features.{i}.fm"])
     for k in ("louts.2.0.weight", "louts.2.0.bias", "louts.2.2.weight", "louts.2.2.bias"):
         assert torch.equal(a[k], b[k])
+
+
+@pytest.mark.parametrize("n", [300, 40000])
+@pytest.mark.parametrize("pos_invariant", [True, False])
+def test_saved_features_give_the_same_bits(dev, n, pos_invariant, monkeypatch):
+    """The backward on the forward's saved features against one that computes
+    them again (a batch above the limit, or weights changed in between), and
+    the predictions against the plain call's."""
+    from nglod_amd import autograd
+
+    net = workloads.make_model(num_lods=4, pos_invariant=pos_invariant, seed=7, device=dev)
+    g = torch.Generator().manual_seed(8)
+    x, gt = (torch.rand(n, 3, generator=g) * 2 - 1).to(dev), torch.rand(n, 1, generator=g).to(dev)
+    a = _grads(net, x, gt)
+    preds = net.sdf(x, return_lst=True)
+    with torch.no_grad():
+        for p, q in zip(preds, net.sdf(x, return_lst=True)):
+            assert torch.equal(p, q)
+    monkeypatch.setattr(autograd, "SAVE_LIMIT", 0)
+    b = _grads(net, x, gt)
+    for k in a:
+        assert torch.equal(a[k], b[k]), k
+    monkeypatch.undo()
+    loss = sum(((p - gt) ** 2).sum() for p in net.sdf(x, return_lst=True))
+    net.zero_grad()
+    with torch.no_grad():
+        net.louts[0][0].weight.mul_(2.0)
+    loss.backward()  # on the new weights' features
+    c = {k: v.grad.clone() for k, v in net.named_parameters()}
+    monkeypatch.setattr(autograd, "SAVE_LIMIT", 0)
+    with torch.no_grad():
+        net.louts[0][0].weight.div_(2.0)
+    loss = sum(((p - gt) ** 2).sum() for p in net.sdf(x, return_lst=True))
+    net.zero_grad()
+    with torch.no_grad():
+        net.louts[0][0].weight.mul_(2.0)
+    loss.backward()
+    for k, v in net.named_parameters():
+        assert torch.equal(c[k], v.grad), k
