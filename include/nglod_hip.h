@@ -427,6 +427,19 @@ int nglod_sdf_bwd_saved(const nglod_model_t* model, const float* x, int64_t n, i
                         int32_t level_mask, const nglod_model_grads_t* grads, void* saved, size_t saved_bytes,
                         void* workspace, size_t workspace_bytes, void* stream);
 
+/* Loss of Trainer.step_geometry (sdf-net/lib/trainer.py:325-337): loss [1] = sum
+ * over the levels l of level_mask of sum_i (pred[l][i] - gt[i])^2 / n, and
+ * grad [levels][n] = its gradient (0 for the other levels). */
+size_t nglod_geometry_loss_workspace_size(void);
+int nglod_geometry_loss(const float* pred, const float* gt, int64_t n, int32_t levels, uint32_t level_mask, float* grad,
+                        float* loss, void* workspace, size_t workspace_bytes, void* stream);
+
+/* torch.optim.Adam's update (no weight decay, no amsgrad) of `count` tensors of
+ * n[i] floats, given by HOST arrays of device pointers: parameters, gradients
+ * and both moments; `step` counts from 1. */
+int nglod_adam_step(float* const* p, const float* const* g, float* const* m, float* const* v, const int64_t* n,
+                    int32_t count, double beta1, double beta2, double eps, double lr, int64_t step, void* stream);
+
 /* ---- training targets and samples ------------------------------------- */
 
 /* Workspace bytes nglod_mesh2sdf_f64 needs for nf triangles (per-triangle

@@ -146,6 +146,10 @@ SIGNATURES = {
     "nglod_sdf_bwd_saved_workspace_size": (_sz, [ctypes.POINTER(NglodModel), _i64, _i32]),
     "nglod_sdf_bwd_saved": (ctypes.c_int, [ctypes.POINTER(NglodModel), _p, _i64, _i32, _p, _i32,
                                             ctypes.POINTER(NglodModelGrads), _p, _sz, _p, _sz, _p]),
+    "nglod_geometry_loss_workspace_size": (_sz, []),
+    "nglod_geometry_loss": (ctypes.c_int, [_p, _p, _i64, _i32, ctypes.c_uint32, _p, _p, _p, _sz, _p]),
+    "nglod_adam_step": (ctypes.c_int, [_p, _p, _p, _p, _p, _i32, ctypes.c_double, ctypes.c_double, ctypes.c_double,
+                                       ctypes.c_double, _i64, _p]),
     "nglod_spc_occupancy": (ctypes.c_int, [_p, _i64, _i32, _p, _i64, ctypes.POINTER(_i64), _p, _sz,
                                             ctypes.POINTER(_sz), _p]),
     "nglod_spc_from_codes": (ctypes.c_int, [_p, _i64, _i32, _p, _i64, ctypes.POINTER(_i64), _p, _p, _sz,

@@ -125,9 +125,10 @@ class _SdfFunction(torch.autograd.Function):
         return (None, grad_x, None, None, *grads)
 
 
-def sdf_with_grad(net, x, lod, all_levels):
+def sdf_with_grad(net, x, lod, all_levels, stacked=False):
+    """stacked: the levels' predictions as one [lod + 1, n, 1] tensor."""
     params = list(net.parameters())
     out = _SdfFunction.apply(net, x, lod, all_levels, *params)
-    if all_levels:
+    if all_levels and not stacked:
         return [out[i] for i in range(out.shape[0])]
     return out

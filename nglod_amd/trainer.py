@@ -4,28 +4,58 @@ produces the benchmark model.
 
 step_geometry: zero_grad; predictions of every LOD in loss_lods from one
 fused forward (the reference's return_lst branch, :317-319); loss =
-sum over LODs of sum (pred - gt)^2, divided by the batch size (:325-337);
-backward through nglod_sdf_bwd; Adam (lr 1e-3, :184-185).
+sum over LODs of sum (pred - gt)^2, divided by the batch size (:325-337), and
+its gradient from one kernel (nglod_geometry_loss); backward through
+nglod_sdf_bwd_saved; Adam (lr 1e-3, :184-185) by nglod_adam_step.
 """
 import torch
 
-from . import workloads
+from . import _lib, workloads
+from .autograd import sdf_with_grad
 from .meshdata import MeshData
+from .octree_sdf import OctreeSDF
+from .optim import Adam
 from . import mesh as _mesh
 
 
 class Trainer:
     def __init__(self, net, lr=1e-3, loss_lods=None):
         self.net = net
-        self.optimizer = torch.optim.Adam(net.parameters(), lr=lr)
+        self.optimizer = Adam(net.parameters(), lr=lr)
         self.loss_lods = list(range(net.num_lods)) if loss_lods is None else list(loss_lods)
         self.last_loss = None
+
+    def _fused(self, pts, gts):
+        """Whether loss and gradient can come from nglod_geometry_loss: a plain
+        OctreeSDF's every-level predictions against one FP32 value per point."""
+        net = self.net
+        return (type(net) is OctreeSDF and net.lod is None and pts.dim() == 2 and pts.is_cuda and pts.shape[0] > 0
+                and torch.is_tensor(gts) and gts.shape == (pts.shape[0], 1) and gts.dtype == torch.float32
+                and gts.device == pts.device and not gts.requires_grad and torch.is_grad_enabled()
+                and all(0 <= i < net.num_lods for i in self.loss_lods)
+                and len(set(self.loss_lods)) == len(self.loss_lods) > 0
+                and all(p.requires_grad for p in net.parameters()))
 
     def step_geometry(self, pts, gts):
         net = self.net
         net.train()
         batch_size = pts.shape[0]
         net.zero_grad()
+        if self._fused(pts, gts):
+            stacked = sdf_with_grad(net, pts, net.num_lods - 1, all_levels=True, stacked=True)
+            net.loss_preds = list(stacked.unbind(0))
+            gt = gts.contiguous()
+            grad = torch.empty_like(stacked)
+            loss = torch.empty((), dtype=torch.float32, device=pts.device)
+            lib = _lib.load()
+            ws = torch.empty(lib.nglod_geometry_loss_workspace_size(), dtype=torch.uint8, device=pts.device)
+            _lib.check(lib.nglod_geometry_loss(_lib.ptr(stacked), _lib.ptr(gt), batch_size, net.num_lods,
+                                               sum(1 << i for i in self.loss_lods), _lib.ptr(grad), _lib.ptr(loss),
+                                               _lib.ptr(ws), ws.numel(), _lib.stream_of(pts)), "nglod_geometry_loss")
+            torch.autograd.backward(stacked, grad)
+            self.optimizer.step()
+            self.last_loss = loss
+            return self.last_loss
         preds = net.sdf(pts, return_lst=True)
         preds = [preds[i] for i in self.loss_lods]
         loss = 0.0
