@@ -2,16 +2,14 @@
 //
 // Uniformly scattered query points put unrelated grid cells in neighbouring
 // lanes, so a wave's corner loads touch as many cache lines as it has lanes.
-// Sorting the points by the Morton code of their position (10 bits per axis)
-// first makes a wave's 64 points a compact cluster: its loads share lines in
-// L1 and L2.  Keys are 30 bits, sorted with their indices by rocPRIM's radix
-// sort; the batch kernels then evaluate point order[t] in thread t and write
-// out[order[t]].
+// Sorting the points by the Morton code of their cell first gives a wave few
+// cells: the FP32 kernel then interpolates cell by cell (cell_gather.hpp), the
+// mixed one finds its lines in L1 and L2.  The batch kernels evaluate point
+// order[t] in thread t and write out[order[t]].
 #include <cstring>
 
-#include <rocprim/rocprim.hpp>
-
 #include "api_common.hpp"
+#include "radix_sort.hpp"
 
 namespace nglod {
 
@@ -25,28 +23,28 @@ __device__ __forceinline__ uint32_t spread3(uint32_t v) {
     return v;
 }
 
-__device__ __forceinline__ uint32_t quantize10(float p) {
-    const float q = (p + 1.0f) * 512.0f;  // [-1, 1] -> [0, 1024]
-    return q <= 0.0f ? 0u : (q >= 1023.0f ? 1023u : (uint32_t)q);  // NaN -> 0
-}
-
-__global__ void morton_keys_kernel(const float* __restrict__ x, int64_t n, uint32_t* __restrict__ keys,
-                                   uint32_t* __restrict__ idx) {
+// Key of a point: the Morton code of its cell in a grid of resolution r, less
+// its low `drop` bits.
+__global__ void morton_keys_kernel(const float* __restrict__ x, int64_t n, int r, int drop,
+                                   uint32_t* __restrict__ keys) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const uint32_t qx = quantize10(x[3 * i]), qy = quantize10(x[3 * i + 1]), qz = quantize10(x[3 * i + 2]);
-    keys[i] = (spread3(qz) << 2) | (spread3(qy) << 1) | spread3(qx);
-    idx[i] = (uint32_t)i;
+    const uint32_t qx = (uint32_t)axis_weights(x[3 * i], r).i0, qy = (uint32_t)axis_weights(x[3 * i + 1], r).i0,
+                   qz = (uint32_t)axis_weights(x[3 * i + 2], r).i0;
+    keys[i] = ((spread3(qz) << 2) | (spread3(qy) << 1) | spread3(qx)) >> drop;
 }
 
-static inline size_t up256(size_t b) { return (b + 255) / 256 * 256; }
-
-static size_t sort_temp_bytes(int64_t n) {
-    size_t t = 0;
-    if (rocprim::radix_sort_pairs((void*)nullptr, t, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr,
-                                  (uint32_t*)nullptr, (size_t)n, 0, 30, (hipStream_t)0) != hipSuccess)
-        return 0;
-    return t;
+// Sorted bits: the finest grid's cells as far as a bin of the order still holds
+// about a wave's 64 points (the cells of a wave need not be in runs).  Each 8
+// bits are a pass over the pairs: 2^22 points at LOD 4 take two passes instead
+// of the four of a 30-bit position code.
+static int order_bits(int64_t n, int r, int* drop) {
+    int axis = 0, want = 1;
+    while ((1 << axis) < r) ++axis;
+    while (((int64_t)64 << want) < n) ++want;
+    const int all = 3 * axis > 0 ? 3 * axis : 1;
+    *drop = all > want ? all - want : 0;
+    return all - *drop;
 }
 
 }  // namespace nglod
@@ -55,10 +53,7 @@ using namespace nglod;
 
 extern "C" {
 
-size_t nglod_sdf_fwd_ordered_workspace_size(int64_t n) {
-    if (n < 1) n = 1;
-    return 4 * up256((size_t)n * 4) + up256(sort_temp_bytes(n));
-}
+size_t nglod_sdf_fwd_ordered_workspace_size(int64_t n) { return sort_workspace_bytes(n < 1 ? 1 : n); }
 
 int nglod_sdf_fwd_ordered(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, int32_t form, float* out,
                           void* workspace, size_t workspace_bytes, void* stream) {
@@ -68,26 +63,21 @@ int nglod_sdf_fwd_ordered(const nglod_model_t* model, const float* x, int64_t n,
     if (n < 0 || n > (int64_t)0x7fff0000) return fail(NGLOD_ERR_ARG, "n out of range");
     if (n == 0) return NGLOD_OK;
     if (!x || !out) return fail(NGLOD_ERR_ARG, "NULL pointer");
-    const size_t seg = up256((size_t)n * 4);
-    size_t tmp = sort_temp_bytes(n);
-    if (tmp == 0) return fail(NGLOD_ERR_HIP, "sort size query failed");
-    if (!workspace || workspace_bytes < 4 * seg + up256(tmp)) return fail(NGLOD_ERR_WORKSPACE, "workspace too small");
+    if (!workspace || workspace_bytes < sort_workspace_bytes(n))
+        return fail(NGLOD_ERR_WORKSPACE, "workspace too small");
     if (!aligned16(workspace)) return fail(NGLOD_ERR_ARG, "workspace not 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
-    char* w = (char*)workspace;
-    uint32_t* k_in = (uint32_t*)w;
-    uint32_t* k_out = (uint32_t*)(w + seg);
-    uint32_t* i_in = (uint32_t*)(w + 2 * seg);
-    uint32_t* i_out = (uint32_t*)(w + 3 * seg);
-    hipLaunchKernelGGL(morton_keys_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, n, k_in, i_in);
-    rc = check_launch("morton_keys_kernel");
+    const SortBuffers sb = sort_buffers(workspace, n);
+    int drop = 0;
+    const int bits = order_bits(n, model->res[lod], &drop);
+    hipLaunchKernelGGL(morton_keys_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, n, model->res[lod],
+                       drop, sb.keys[0]);
+    const uint32_t* order = sb.vals[launch_sort(sb, n, bits, s)];
+    rc = check_launch("sort_scatter_kernel");
     if (rc) return rc;
-    if (rocprim::radix_sort_pairs((void*)(w + 4 * seg), tmp, k_in, k_out, i_in, i_out, (size_t)n, 0, 30, s) !=
-        hipSuccess)
-        return fail(NGLOD_ERR_HIP, "sort failed");
     const int dec = decoder_of(model, lod);
-    if (form == NGLOD_MIXED) return launch_sdf_mixed(m, 0, dec, x, n, out, i_out, s);
-    return launch_sdf_fp32(m, lod, dec, x, n, out, i_out, s);
+    if (form == NGLOD_MIXED) return launch_sdf_mixed(m, 0, dec, x, n, out, order, s);
+    return launch_sdf_ordered_fp32(m, lod, dec, x, n, out, order, s);
 }
 
 }  // extern "C"
