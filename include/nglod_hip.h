@@ -131,8 +131,8 @@ size_t nglod_sdf_fwd_ordered_workspace_size(int64_t n);
 
 /* nglod_sdf_fwd (the same reference interface, OctreeSDF.sdf) for large,
  * spatially scattered query sets: the points are first sorted by the Morton
- * code of their position (10 bits per axis over [-1, 1]) and evaluated in that
- * order, so the lanes of a wave gather neighbouring grid corners; out is in
+ * code of their cell at `lod` and evaluated in that order, so the lanes of a
+ * wave share cells or gather neighbouring grid corners; out is in
  * input order and bit-identical to nglod_sdf_fwd's (each point's arithmetic
  * does not depend on the other points of its wave).  n < 2^31.  workspace:
  * device memory of nglod_sdf_fwd_ordered_workspace_size(n) bytes, 16-byte
@@ -272,6 +272,15 @@ int nglod_normals_fd(const nglod_model_t* model, const float* x, int64_t n, int3
  * 0 returns the raw gradient as diffutils.gradient and get_min do. */
 int nglod_gradient(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, int32_t form,
                    int32_t method, const uint8_t* mask, int32_t normalize, float* grad, void* stream);
+
+/* nglod_gradient for large, spatially scattered point sets: the points are
+ * evaluated in the order of their cells, as nglod_sdf_fwd_ordered does, with the
+ * same workspace (nglod_sdf_fwd_ordered_workspace_size(n) bytes, 16-byte
+ * aligned).  grad is in input order; each point's arithmetic does not depend on
+ * the other points of its wave. */
+int nglod_gradient_ordered(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, int32_t form,
+                           int32_t method, const uint8_t* mask, int32_t normalize, float* grad, void* workspace,
+                           size_t workspace_bytes, void* stream);
 
 /* OctreeSDF.sdf(x, lod) and its autodiff gradient in one pass (sdf [n], may
  * be NULL; grad [n][3]): the position gradient of the reference's autograd

@@ -133,6 +133,8 @@ SIGNATURES = {
     "nglod_normals_fd": (ctypes.c_int, [ctypes.POINTER(NglodModel), _p, _i64, _i32, _i32, _p, _p]),
     "nglod_pack_mixed": (ctypes.c_int, [ctypes.POINTER(NglodModel), _p]),
     "nglod_gradient": (ctypes.c_int, [ctypes.POINTER(NglodModel), _p, _i64, _i32, _i32, _i32, _p, _i32, _p, _p]),
+    "nglod_gradient_ordered": (ctypes.c_int, [ctypes.POINTER(NglodModel), _p, _i64, _i32, _i32, _i32, _p, _i32, _p, _p,
+                                              _sz, _p]),
     "nglod_sdf_grad": (ctypes.c_int, [ctypes.POINTER(NglodModel), _p, _i64, _i32, _i32, _p, _p, _p]),
     "nglod_trace_min_workspace_size": (_sz, [_i64]),
     "nglod_trace_min": (ctypes.c_int, [ctypes.POINTER(NglodModel), _p, _p, _i64, _i32, ctypes.POINTER(NglodTraceParams),

@@ -143,6 +143,8 @@ struct TraceArgs;
 int launch_sdf_fp32(const ModelArgs& m, int lod, int dec, const float* x, int64_t n, float* out, hipStream_t s);
 int launch_sdf_ordered_fp32(const ModelArgs& m, int lod, int dec, const float* x, int64_t n, float* out,
                             const uint32_t* order, hipStream_t s);
+int launch_cell_order(const float* x, int64_t n, int r, void* workspace, size_t workspace_bytes,
+                      const uint32_t** order, hipStream_t s);
 int launch_sdf_mixed(const ModelArgs& m, int lod, int dec, const float* x, int64_t n, float* out,
                      const uint32_t* order, hipStream_t s);
 int launch_trace_mixed(const TraceArgs& a, int64_t n, hipStream_t s, PassTimer& timer);

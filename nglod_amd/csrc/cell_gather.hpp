@@ -36,6 +36,11 @@ struct CellFeatures {
 
 __device__ __forceinline__ CellFeatures zero_cell_features() { return CellFeatures{{{}, {}}}; }
 
+// Channel of row n of the A operand.
+__device__ __forceinline__ uint32_t cell_row(uint32_t n) {
+    return 2u * (4u * (n >> 3) + (n & 3u)) + ((n >> 2) & 1u);
+}
+
 // One more level onto f.  Every lane of the wave calls this with a position
 // (lanes without a query: any position); use1: tile 1 holds a query.
 __device__ __forceinline__ void gather_cells(const float* __restrict__ grid, int r, float px, float py, float pz,
@@ -95,8 +100,7 @@ __device__ __forceinline__ void gather_cells(const float* __restrict__ grid, int
         w[1][s] = __uint_as_float(sw[1]);
     }
     const uint32_t n = lane & 31u, half = lane >> 5;
-    const uint32_t row = 2u * (4u * (n >> 3) + (n & 3u)) + ((n >> 2) & 1u);  // channel of A row n
-    const float* mine = grid + half * kC + row;  // corner 2 s + half: x = half
+    const float* mine = grid + half * kC + cell_row(n);  // corner 2 s + half: x = half
     const size_t sy = (size_t)S * kC, sz = (size_t)S * S * kC;
     for (uint64_t m = all; m != 0;) {
         const uint32_t cell = (uint32_t)__builtin_amdgcn_readlane((int)base, __ffsll((unsigned long long)m) - 1);

@@ -47,6 +47,22 @@ static int order_bits(int64_t n, int r, int* drop) {
     return all - *drop;
 }
 
+// The evaluation order of n points over a grid of resolution r, in a checked
+// workspace of sort_workspace_bytes(n).
+int launch_cell_order(const float* x, int64_t n, int r, void* workspace, size_t workspace_bytes,
+                      const uint32_t** order, hipStream_t s) {
+    if (!workspace || workspace_bytes < sort_workspace_bytes(n))
+        return fail(NGLOD_ERR_WORKSPACE, "workspace too small");
+    if (!aligned16(workspace)) return fail(NGLOD_ERR_ARG, "workspace not 16-byte aligned");
+    const SortBuffers sb = sort_buffers(workspace, n);
+    int drop = 0;
+    const int bits = order_bits(n, r, &drop);
+    hipLaunchKernelGGL(morton_keys_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, n, r, drop,
+                       sb.keys[0]);
+    *order = sb.vals[launch_sort(sb, n, bits, s)];
+    return check_launch("sort_scatter_kernel");
+}
+
 }  // namespace nglod
 
 using namespace nglod;
@@ -63,17 +79,9 @@ int nglod_sdf_fwd_ordered(const nglod_model_t* model, const float* x, int64_t n,
     if (n < 0 || n > (int64_t)0x7fff0000) return fail(NGLOD_ERR_ARG, "n out of range");
     if (n == 0) return NGLOD_OK;
     if (!x || !out) return fail(NGLOD_ERR_ARG, "NULL pointer");
-    if (!workspace || workspace_bytes < sort_workspace_bytes(n))
-        return fail(NGLOD_ERR_WORKSPACE, "workspace too small");
-    if (!aligned16(workspace)) return fail(NGLOD_ERR_ARG, "workspace not 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
-    const SortBuffers sb = sort_buffers(workspace, n);
-    int drop = 0;
-    const int bits = order_bits(n, model->res[lod], &drop);
-    hipLaunchKernelGGL(morton_keys_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, n, model->res[lod],
-                       drop, sb.keys[0]);
-    const uint32_t* order = sb.vals[launch_sort(sb, n, bits, s)];
-    rc = check_launch("sort_scatter_kernel");
+    const uint32_t* order = nullptr;
+    rc = launch_cell_order(x, n, model->res[lod], workspace, workspace_bytes, &order, s);
     if (rc) return rc;
     const int dec = decoder_of(model, lod);
     if (form == NGLOD_MIXED) return launch_sdf_mixed(m, 0, dec, x, n, out, order, s);

@@ -240,12 +240,17 @@ class OctreeSDF(nn.Module):
                    "nglod_sdf_fwd")
         return out
 
-    def gradient_hip(self, x, lod, method="autodiff", mask=None, normalize=False, form=_lib.FP32):
+    def gradient_hip(self, x, lod, method="autodiff", mask=None, normalize=False, form=_lib.FP32, ordered=None):
         """d sdf(x, lod) / d x [N, 3] (diffutils.gradient, sdf-net/lib/diffutils.py:29-84)
         by 'finitediff', 'tetrahedron' or 'autodiff' (the derivative torch
         autograd computes), FP32.  mask: optional bool [N]; rows where it is
         False are 0.  normalize: F.normalize(eps=1e-5) of each row, as
-        SphereTracer.forward applies to its normals.  No autograd graph."""
+        SphereTracer.forward applies to its normals.  No autograd graph.
+        ordered: None picks by batch size, True / False forces the evaluation in
+        cell / input order (the same results; a frame's points are neighbours
+        already).  Uniform points at LOD 4, both ways in us: autodiff 117 / 105
+        with 2^16 points, 140 / 174 with 2^17; finite differences 212 / 251 with
+        2^13, at LOD 1 148 / 221 with 2^17; tetrahedron 181 / 185 with 2^15."""
         if method not in _lib.GRAD_METHODS:
             raise NotImplementedError(f"gradient method {method!r}")
         xf = x.detach().reshape(-1, 3).float().contiguous()
@@ -258,8 +263,17 @@ class OctreeSDF(nn.Module):
                 raise ValueError("mask must hold one flag per point")
         m = self.descriptor(form)
         lib = _lib.load()
-        _lib.check(lib.nglod_gradient(m, _lib.ptr(xf), n, int(lod), form, _lib.GRAD_METHODS[method], _lib.ptr(mk),
-                                      1 if normalize else 0, _lib.ptr(out), _lib.stream_of(x)), "nglod_gradient")
+        args = (m, _lib.ptr(xf), n, int(lod), form, _lib.GRAD_METHODS[method], _lib.ptr(mk), 1 if normalize else 0,
+                _lib.ptr(out))
+        if ordered is None:
+            ordered = n >= (1 << 17 if method == "autodiff" else 1 << 15)
+        if ordered and n > 0:
+            nbytes = int(lib.nglod_sdf_fwd_ordered_workspace_size(n))
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+            _lib.check(lib.nglod_gradient_ordered(*args, _lib.ptr(ws), nbytes, _lib.stream_of(x)),
+                       "nglod_gradient_ordered")
+        else:
+            _lib.check(lib.nglod_gradient(*args, _lib.stream_of(x)), "nglod_gradient")
         return out
 
     def sdf_grad_hip(self, x, lod):

@@ -236,7 +236,8 @@ class SphereTracer(BaseTracer):
                                          _lib.ptr(hit), _lib.ptr(normal), _lib.ptr(ws), ws.numel(), _lib.ptr(evals),
                                          _lib.ptr(ray_steps), _lib.stream_of(o)), "nglod_trace_dense")
         if not fused_normals:
-            normal = net.gradient_hip(x, lod, self.grad_method, mask=hit, normalize=True, form=form)
+            normal = net.gradient_hip(x, lod, self.grad_method, mask=hit, normalize=True, form=form,
+                                      ordered=False)
         self.last_evals = evals
         self.last_pass_ms = list(pass_ms) if pass_ms is not None else None
         return RenderBuffer(x=x, depth=t, hit=hit, normal=normal)
@@ -275,7 +276,7 @@ class SphereTracer(BaseTracer):
         _lib.check(lib.nglod_trace_min(net.descriptor(_lib.FP32), _lib.ptr(o), _lib.ptr(d), n, lod, p, _lib.ptr(x),
                                        _lib.ptr(t), _lib.ptr(hit), _lib.ptr(min_x), _lib.ptr(ws), ws.numel(),
                                        _lib.stream_of(o)), "nglod_trace_min")
-        normal = net.gradient_hip(x, lod, self.grad_method, mask=hit, normalize=False)
+        normal = net.gradient_hip(x, lod, self.grad_method, mask=hit, normalize=False, ordered=False)
         return RenderBuffer(x=x, depth=t, hit=hit, normal=normal, min_x=min_x)
 
     def sample_surface(self, n, net, seed=0, max_batches=1000):
