@@ -147,6 +147,7 @@ int launch_cell_order(const float* x, int64_t n, int r, void* workspace, size_t 
                       const uint32_t** order, hipStream_t s);
 int launch_sdf_mixed(const ModelArgs& m, int lod, int dec, const float* x, int64_t n, float* out,
                      const uint32_t* order, hipStream_t s);
+int launch_trace_fp32(const TraceArgs& a, int64_t n, hipStream_t s);
 int launch_trace_mixed(const TraceArgs& a, int64_t n, hipStream_t s, PassTimer& timer);
 
 // Pooled trace (several requests, one launch per pass): the request table is

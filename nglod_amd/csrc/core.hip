@@ -178,69 +178,6 @@ __global__ __launch_bounds__(256) void normals_fp32_kernel(ModelArgs m, int lod,
     normalize_grad(g[0], g[1], g[2], nrm[3 * i], nrm[3 * i + 1], nrm[3 * i + 2]);
 }
 
-template <bool POSINV>
-__global__ __launch_bounds__(kMarchBlock) void trace_dense_fp32_kernel(TraceArgs a) {
-    __shared__ Fp32Lds lds;
-    __shared__ CoarseLds32 coarse;
-    __shared__ __align__(16) float solo_sv[kMarchBlock / 64][kH];
-    __shared__ SoloLevels solo_lv;
-    stage_fp32_lds(a.m, a.dec, &lds);
-    stage_coarse32(a.m, a.coarse, &coarse);
-    stage_solo_levels(a.m, &solo_lv);
-    __syncthreads();
-    const float b1 = a.m.b1[a.dec][0];
-    const uint32_t lane = lane_id();
-    float* sv = solo_sv[threadIdx.x >> 6];
-    RayFeed feed;
-    feed.init(a.nrays, a.queue_stride);
-    RayState s;
-    s.ray = -1;
-    s.phase = PH_IDLE;
-    uint32_t nevals = 0;
-    bool tail = false;
-    for (;;) {
-        feed.refill<0>(s, a, lane);
-        const uint64_t act = __ballot(s.phase != PH_IDLE);
-        if (act == 0) break;
-        if (feed.empty() && __popcll(act) <= a.solo_lanes) {
-            tail = true;
-            break;
-        }
-        const bool busy = s.phase != PH_IDLE;
-        const float d = sdf_fp32_wave<POSINV>(a.m, a.lod, &lds, b1, lane, busy, s.qx, s.qy, s.qz, a.coarse, &coarse);
-        if (busy) {
-            ++nevals;
-            s.consume(a, d);
-        }
-    }
-    // the wave's last few rays, one query at a time (fp32_solo_step)
-    while (tail) {
-        const uint64_t act = __ballot(s.phase != PH_IDLE);
-        if (act == 0) break;
-        const float d = fp32_solo_step<POSINV>(a, &lds, &coarse, a.coarse, &solo_lv, sv, b1, lane, act, s.qx, s.qy,
-                                               s.qz);
-        if (s.phase != PH_IDLE) {
-            ++nevals;
-            s.consume(a, d);
-        }
-    }
-    if (a.evals) {
-        unsigned long long tot = nevals;
-        for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off);
-        if (lane == 0) atomicAdd(a.evals, tot);
-    }
-}
-
-template <typename K>
-static int persistent_grid(K kernel, int64_t n, int block) {
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess || per_cu <= 0) per_cu = 4;
-    const int64_t want = (n + block - 1) / block;
-    const int64_t cap = (int64_t)device_cu_count() * per_cu;
-    return (int)(want < cap ? (want < 1 ? 1 : want) : cap);
-}
-
-
 }  // namespace nglod
 
 using namespace nglod;
@@ -417,14 +354,7 @@ static int trace_dense_run(const nglod_model_t* model, const ModelArgs& m, const
         rc = launch_trace_mixed(a, n, s, timer);
         return rc ? rc : timer.finish();
     }
-    if (m.pos_inv) {
-        const int grid = persistent_grid(trace_dense_fp32_kernel<true>, n, kMarchBlock);
-        hipLaunchKernelGGL(trace_dense_fp32_kernel<true>, dim3(grid), dim3(kMarchBlock), 0, s, a);
-    } else {
-        const int grid = persistent_grid(trace_dense_fp32_kernel<false>, n, kMarchBlock);
-        hipLaunchKernelGGL(trace_dense_fp32_kernel<false>, dim3(grid), dim3(kMarchBlock), 0, s, a);
-    }
-    rc = check_launch("trace_dense_fp32_kernel");
+    rc = launch_trace_fp32(a, n, s);
     if (rc) return rc;
     timer.mark(kPassMarch);
     return timer.finish();

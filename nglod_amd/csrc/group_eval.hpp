@@ -1,0 +1,155 @@
+// The SDF of a group of 32 queries by one block of four waves, FP32: every wave
+// holds the same 32 queries (lanes n and n + 32: query n) and does a part of each.
+//
+//  1. A thread per (level, query) computes the cell and the eight corner weights.
+//  2. Eight threads per query gather: thread q of a query owns channels 4 q .. 4 q + 3,
+//     so the eight threads read a corner's row of 128 bytes in one piece (15 cycles
+//     of the vector L1 per load instruction; one query per lane, 64 rows at a time:
+//     25).
+//  3. Wave h multiplies hidden units 32 h .. 32 h + 31 (its rows of W0 stay in 16
+//     registers) by the features of all 32 queries and takes its units' share of the
+//     second layer; the four shares are added in the order of h.
+//
+// The sums have the order of sdf_fp32_wave's, so the bits are the same.  A grid of
+// 5^3 corners (level 0) is kept in LDS: one fifth of a 5-level gather leaves the
+// L1 (1280x720: 3.82 -> 3.43 ms); with 34 KB of LDS a CU holds four blocks.
+// Interpolating the cells that neighbouring rays share on the matrix cores (as
+// cell_gather.hpp does for sorted points) cut the L1's traffic to a quarter but
+// was slower (5.5 ms; only cells shared by most rays: 5.1): a group's rays lie in
+// four cells per level and 16 rays on average, one dependent product each.
+#pragma once
+
+#include "fp32_wave.hpp"
+
+namespace nglod {
+
+constexpr int kGroup = 32;            // queries of a block
+constexpr int kGroupThreads = 256;
+constexpr int kFeatStride = 20;       // floats between queries: 16-byte aligned, spread over the banks
+
+struct GroupLds {
+    float4 w[NGLOD_MAX_LODS][kGroup][2];  // corner weights, corner = 4 z + 2 y + x
+    uint32_t base[NGLOD_MAX_LODS][kGroup];
+    float feat[2][kGroup][kFeatStride];   // [half][query][kk] = channel 2 kk + half
+    float part[4][64];
+    float b0[kH];
+    float w1[kH];
+    float wxyz[kH][4];
+    float4 coarse[125 * (kC / 4)];  // level 0's grid when it has at most 5^3 corners
+};
+
+struct GroupWeights {
+    float a[kC / 2];  // A operands: W0[32 h + n][2 kk + half]
+};
+
+// Every thread of the block; the caller's next barrier comes before group_sdf.
+__device__ __forceinline__ GroupWeights stage_group(const ModelArgs& m, int dec, GroupLds* s) {
+    const int din = m.pos_inv ? kC : kC + 3, off = m.pos_inv ? 0 : 3;
+    const float* W0 = m.w0[dec];
+    const int lane = threadIdx.x & 63, h = threadIdx.x >> 6;
+    const float* row = W0 + (32 * h + (lane & 31)) * din + off + (lane >> 5);
+    GroupWeights g;
+#pragma unroll
+    for (int kk = 0; kk < kC / 2; ++kk) g.a[kk] = row[2 * kk];
+    for (int j = threadIdx.x; j < kH; j += kGroupThreads) {
+        s->b0[j] = m.b0[dec][j];
+        s->w1[j] = m.w1[dec][j];
+        for (int k = 0; k < 3; ++k) s->wxyz[j][k] = m.pos_inv ? 0.0f : W0[j * din + k];
+        s->wxyz[j][3] = 0.0f;
+    }
+    if (m.res[0] <= 4) {
+        const int S = m.res[0] + 1;
+        const float4* g4 = reinterpret_cast<const float4*>(m.grid[0]);
+        for (int j = threadIdx.x; j < S * S * S * (kC / 4); j += kGroupThreads) s->coarse[j] = g4[j];
+    }
+    return g;
+}
+
+// Eight corner rows' float4 of this thread.
+__device__ __forceinline__ void group_rows(const float* __restrict__ grid, int S, uint32_t base, uint32_t q,
+                                           float4 (&g)[8]) {
+    const float* b = grid + (size_t)base * kC + 4 * q;
+    const size_t sy = (size_t)S * kC, sz = (size_t)S * S * kC;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        g[k] = *reinterpret_cast<const float4*>(b + (k & 1) * kC + (k & 2 ? sy : 0) + (k & 4 ? sz : 0));
+}
+
+__device__ __forceinline__ void group_corners(const float4 (&g)[8], const float4* w, float4& f) {
+    const float4 w0 = w[0], w1 = w[1];
+    const float ww[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        f.x = __builtin_fmaf(g[k].x, ww[k], f.x);
+        f.y = __builtin_fmaf(g[k].y, ww[k], f.y);
+        f.z = __builtin_fmaf(g[k].z, ww[k], f.z);
+        f.w = __builtin_fmaf(g[k].w, ww[k], f.w);
+    }
+}
+
+// Every thread of the block, with the position of query lane % 32 (the same in
+// all four waves; any position for queries whose result is not used).
+template <bool POSINV>
+__device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds* s, const GroupWeights& gw, float b1,
+                                           float px, float py, float pz) {
+    const uint32_t lane = lane_id(), n = lane & 31u, half = lane >> 5;
+    const int h = (int)(threadIdx.x >> 6);
+    {
+        const int l = 2 * h + (int)half;  // NGLOD_MAX_LODS = 8 levels
+        if (l <= lod) {
+            const int r = m.res[l], S = r + 1;
+            const AxisW ax = axis_weights(px, r);
+            const AxisW ay = axis_weights(py, r);
+            const AxisW az = axis_weights(pz, r);
+            const float wxy00 = ax.w0 * ay.w0, wxy10 = ax.w1 * ay.w0;
+            const float wxy01 = ax.w0 * ay.w1, wxy11 = ax.w1 * ay.w1;
+            s->base[l][n] = (uint32_t)((az.i0 * S + ay.i0) * S + ax.i0);
+            s->w[l][n][0] = make_float4(wxy00 * az.w0, wxy10 * az.w0, wxy01 * az.w0, wxy11 * az.w0);
+            s->w[l][n][1] = make_float4(wxy00 * az.w1, wxy10 * az.w1, wxy01 * az.w1, wxy11 * az.w1);
+        }
+    }
+    __syncthreads();
+    {
+        const uint32_t ray = threadIdx.x >> 3, q = threadIdx.x & 7u;
+        float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        float4 g[8];
+        int l = 0;
+        if (m.res[0] <= 4) {
+            const int S = m.res[0] + 1;
+            const float4* b = s->coarse + s->base[0][ray] * (kC / 4) + q;
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                g[k] = b[((k & 1) + (k & 2 ? S : 0) + (k & 4 ? S * S : 0)) * (kC / 4)];
+            group_corners(g, s->w[0][ray], f);
+            l = 1;
+        }
+#pragma unroll 1
+        for (; l <= lod; ++l) {
+            group_rows(m.grid[l], m.res[l] + 1, s->base[l][ray], q, g);
+            group_corners(g, s->w[l][ray], f);
+        }
+        *reinterpret_cast<float2*>(&s->feat[0][ray][2 * q]) = make_float2(f.x, f.z);
+        *reinterpret_cast<float2*>(&s->feat[1][ray][2 * q]) = make_float2(f.y, f.w);
+    }
+    __syncthreads();
+    f32x16_t c = {};
+    {
+        const float4* b4 = reinterpret_cast<const float4*>(s->feat[half][n]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float4 b = b4[k];
+            c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 0], b.x, c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 1], b.y, c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 2], b.z, c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 3], b.w, c, 0, 0, 0);
+        }
+    }
+    s->part[h][lane] = layer2_tile(c, h, half, s, !POSINV, px, py, pz);
+    __syncthreads();
+    float p = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) p += s->part[k][lane];
+    return halves_sum(p, p) + b1;
+}
+
+}  // namespace nglod

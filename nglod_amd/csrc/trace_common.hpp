@@ -34,11 +34,9 @@ __device__ __forceinline__ void normalize_grad(float g0, float g1, float g2, flo
 // (workgroups are dispatched to XCDs round-robin, so blockIdx % 8 picks the
 // XCD-local range and its L2 sees one band of the image); a wave that drains
 // its own range moves on to the next ones.
-// Threads per block of the FP32 march: one block of 8
-// waves per CU (the 128 KB of decoder and coarse-level tables in LDS leave room
-// for one), sharing those tables.  Measured on the 1280x720 LOD-4 frame: 512
-// threads 4.66 ms, 768 4.99, 384 5.10, 1024 5.36, 256 5.68 (more waves per CU
-// evict each other's cells from the L1).
+// Threads per block of the FP32 ambient occlusion: one block of 8 waves per CU (the
+// 128 KB of decoder and coarse-level tables in LDS leave room for one), sharing
+// those tables.
 constexpr int kMarchBlock = 512;
 constexpr int kQueues = 8;  // a multiple of 8 (one share per XCD)
 static_assert(kQueues % 8 == 0 && kQueues <= 256, "kQueues: a multiple of 8, at most 256");
@@ -94,9 +92,8 @@ struct TraceArgs {
     float return_dist;        // FP32 step length above which a ray goes back to mixed
     int defer_normals;        // 0: a finished hit takes its normal taps in-lane; 1: it is handed to the FP32
                               // pass (hand-off record in phase PH_N0), which takes the taps
-    int solo_lanes;           // FP32 passes: a wave with no rays left to claim and at most this many busy
-                              // lanes evaluates them one at a time with the whole wave (sdf_fp32_solo);
-                              // the mixed passes' cooperative tails use min(this, 4), pass 1's 8 unless 0
+    int solo_lanes;           // mixed passes: a wave with no rays left to claim and at most min(this, 4) busy
+                              // lanes (pass 1: 8 unless 0) spreads their gathers over the idle lanes
     int64_t nrays;  // the frame is split into kQueues ranges [nrays*q/kQueues, nrays*(q+1)/kQueues)
 };
 
@@ -122,17 +119,20 @@ struct RayState {
     float t, D, Dp;
     float qx, qy, qz;  // next query point
     float fplus, g0, g1, g2;
+    bool writes = true;  // false: another lane holds the same ray and writes it out
 
     __device__ __forceinline__ void retire(const TraceArgs& a, bool hit, float n0, float n1, float n2) {
-        a.x[3 * ray] = x0;
-        a.x[3 * ray + 1] = x1;
-        a.x[3 * ray + 2] = x2;
-        a.t[ray] = t;
-        a.hit[ray] = hit ? 1 : 0;
-        a.normal[3 * ray] = n0;
-        a.normal[3 * ray + 1] = n1;
-        a.normal[3 * ray + 2] = n2;
-        if (a.ray_steps) a.ray_steps[ray] = steps;
+        if (writes) {
+            a.x[3 * ray] = x0;
+            a.x[3 * ray + 1] = x1;
+            a.x[3 * ray + 2] = x2;
+            a.t[ray] = t;
+            a.hit[ray] = hit ? 1 : 0;
+            a.normal[3 * ray] = n0;
+            a.normal[3 * ray + 1] = n1;
+            a.normal[3 * ray + 2] = n2;
+            if (a.ray_steps) a.ray_steps[ray] = steps;
+        }
         phase = PH_IDLE;
         ray = -1;
     }
@@ -338,31 +338,6 @@ __device__ __forceinline__ int64_t claim_hits(uint32_t* counter, const uint8_t* 
         if (base + (uint32_t)cnt >= total) drained = true;
     }
     return id;
-}
-
-// The tail of a persistent FP32 pass: a wave with nothing left to claim and
-// at most TraceArgs::solo_lanes busy lanes leaves its main loop (its busy
-// count can only fall from there) and evaluates the remaining queries one at
-// a time with the whole wave (sdf_fp32_solo), the same bits as the wave-wide
-// path.  A separate loop after the main one, so that its registers do not
-// weigh on the main loop's (inlined into the main loop, the unused solo code
-// made the pass 25% slower).
-template <bool POSINV>
-__device__ __forceinline__ float fp32_solo_step(const TraceArgs& a, const Fp32Lds* lds, const CoarseLds32* coarse,
-                                                CoarsePlan cp, const SoloLevels* lv, float* sv, float b1,
-                                                uint32_t lane, uint64_t act, float qx, float qy, float qz) {
-    float d = 0.0f;
-    uint64_t mm = act;
-    while (mm) {
-        const int r = __ffsll((unsigned long long)mm) - 1;
-        mm &= mm - 1ull;
-        // broadcast through a lane shuffle: the address arithmetic of the
-        // solo gather then stays in vector registers
-        const float px = __shfl(qx, r), py = __shfl(qy, r), pz = __shfl(qz, r);
-        const float dr = sdf_fp32_solo<POSINV>(lv, a.lod, lds, b1, lane, sv, px, py, pz, cp, coarse);
-        if ((int)lane == r) d = dr;
-    }
-    return d;
 }
 
 // Hands ray ids to the lanes of one wave.  The frame is split into kQueues

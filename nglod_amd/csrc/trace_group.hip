@@ -1,0 +1,91 @@
+// The FP32 dense sphere trace: launch_trace_fp32 (nglod_trace_dense).  A file of
+// its own: it is built with MFMA results in ordinary VGPRs, which the ReLU reads.
+#include "api_common.hpp"
+#include "group_eval.hpp"
+#include "trace_common.hpp"
+
+namespace nglod {
+
+// A block of four waves marches 32 rays, one evaluation of all of them a trip
+// (group_sdf).  Every wave keeps the state of all 32 rays (lanes n and n + 32: ray
+// n) and steps it by the same results, so the state is never exchanged; the first
+// 32 threads write the rays out.  Persistent: a block claims 32 consecutive rays
+// at a time and hands them to its idle lanes in order.
+//
+// Bound: small frames by the length of the longest ray times a trip's latency
+// (about 2 us: the dependent loads, three barriers, 16 MFMAs in a row), large ones
+// by the corner rows through the vector L1 (56% of its cycles at 1280x720, vector
+// ALU 50%, matrix cores 27%) and by the four blocks a CU that the registers
+// allow: three measured a quarter slower, also with a second level's rows in
+// flight.  A whole frame, 5 LODs, against one ray per lane and 64 rays a wave:
+// 64x48 1339 -> 365 us, 128x96 1367 -> 430, 320x180 1445 -> 677, 1280x720 4091 ->
+// 3430.
+template <bool POSINV>
+__global__ __launch_bounds__(kGroupThreads, 4) void trace_dense_fp32_kernel(TraceArgs a) {
+    __shared__ GroupLds lds;
+    __shared__ int64_t claimed[2];
+    __shared__ int claims_left;
+    const GroupWeights gw = stage_group(a.m, a.dec, &lds);
+    const float b1 = a.m.b1[a.dec][0];
+    const uint32_t lane = lane_id();
+    const bool first = threadIdx.x < 64;
+    RayFeed feed;
+    feed.init(a.nrays, a.queue_stride);
+    RayState s;
+    s.ray = -1;
+    s.phase = PH_IDLE;
+    s.writes = threadIdx.x < kGroup;
+    uint32_t nevals = 0;
+    for (;;) {
+        // refill: block-uniform, every wave sees the same idle lanes
+        for (;;) {
+            const uint32_t need = (uint32_t)__ballot(s.phase == PH_IDLE);
+            if (need == 0 || feed.empty()) break;
+            if (feed.cb >= feed.ce) {
+                if (first) {
+                    feed.claim<true>(a.queue, lane, 0, kGroup);
+                    if (lane == 0) {
+                        claimed[0] = feed.cb;
+                        claimed[1] = feed.ce;
+                        claims_left = feed.drained ? 0 : 1;
+                    }
+                }
+                __syncthreads();
+                feed.cb = claimed[0];
+                feed.ce = claimed[1];
+                feed.drained = claims_left == 0;
+                __syncthreads();
+                continue;
+            }
+            const int64_t id = feed.cb + __popc(need & ((1u << (lane & 31u)) - 1u));
+            const int64_t end = feed.cb + __popc(need);
+            if (s.phase == PH_IDLE && id < feed.ce) s.start(a, id);
+            feed.cb = end < feed.ce ? end : feed.ce;
+        }
+        if (__ballot(s.phase != PH_IDLE) == 0) break;
+        const bool busy = s.phase != PH_IDLE;
+        const float d = group_sdf<POSINV>(a.m, a.lod, &lds, gw, b1, busy ? s.qx : 0.0f, busy ? s.qy : 0.0f,
+                                          busy ? s.qz : 0.0f);
+        if (busy) {
+            ++nevals;
+            s.consume(a, d);
+        }
+    }
+    if (a.evals && first) {
+        unsigned long long tot = lane < kGroup ? nevals : 0;
+        for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off);
+        if (lane == 0) atomicAdd(a.evals, tot);
+    }
+}
+
+int launch_trace_fp32(const TraceArgs& a, int64_t n, hipStream_t s) {
+    const int64_t blocks = (n + kGroup - 1) / kGroup, cap = (int64_t)device_cu_count() * 4;
+    const dim3 grid((unsigned)(blocks < cap ? blocks : cap));
+    if (a.m.pos_inv)
+        hipLaunchKernelGGL(trace_dense_fp32_kernel<true>, grid, dim3(kGroupThreads), 0, s, a);
+    else
+        hipLaunchKernelGGL(trace_dense_fp32_kernel<false>, grid, dim3(kGroupThreads), 0, s, a);
+    return check_launch("trace_dense_fp32_kernel");
+}
+
+}  // namespace nglod
