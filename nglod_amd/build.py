@@ -34,6 +34,7 @@ FLAGS = [
 # it and keep the default).
 EXTRA = {
     "mixed.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "sol_march.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "trace_group.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "query_cells.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }

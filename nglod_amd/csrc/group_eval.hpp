@@ -27,42 +27,83 @@ constexpr int kGroup = 32;            // queries of a block
 constexpr int kGroupThreads = 256;
 constexpr int kFeatStride = 20;       // floats between queries: 16-byte aligned, spread over the banks
 
-struct GroupLds {
-    float4 w[NGLOD_MAX_LODS][kGroup][2];  // corner weights, corner = 4 z + 2 y + x
-    uint32_t base[NGLOD_MAX_LODS][kGroup];
-    float feat[2][kGroup][kFeatStride];   // [half][query][kk] = channel 2 kk + half
+struct alignas(16) GroupDecoder {
+    float feat[2][kGroup][kFeatStride];  // [half][query][kk] = channel 2 kk + half
     float part[4][64];
     float b0[kH];
     float w1[kH];
     float wxyz[kH][4];
+};
+
+struct GroupLds {
+    float4 w[NGLOD_MAX_LODS][kGroup][2];  // corner weights, corner = 4 z + 2 y + x
+    uint32_t base[NGLOD_MAX_LODS][kGroup];
     float4 coarse[125 * (kC / 4)];  // level 0's grid when it has at most 5^3 corners
+    GroupDecoder dec;
 };
 
 struct GroupWeights {
     float a[kC / 2];  // A operands: W0[32 h + n][2 kk + half]
 };
 
-// Every thread of the block; the caller's next barrier comes before group_sdf.
-__device__ __forceinline__ GroupWeights stage_group(const ModelArgs& m, int dec, GroupLds* s) {
-    const int din = m.pos_inv ? kC : kC + 3, off = m.pos_inv ? 0 : 3;
-    const float* W0 = m.w0[dec];
+// Every thread of the block (W0 [128][din], din = 32, or 35 with xyz first); a
+// barrier comes before the first group_decode.
+__device__ __forceinline__ GroupWeights stage_group_decoder(const float* W0, int din, const float* b0, const float* w1,
+                                                            GroupDecoder* s) {
+    const int off = din - kC;
     const int lane = threadIdx.x & 63, h = threadIdx.x >> 6;
     const float* row = W0 + (32 * h + (lane & 31)) * din + off + (lane >> 5);
     GroupWeights g;
 #pragma unroll
     for (int kk = 0; kk < kC / 2; ++kk) g.a[kk] = row[2 * kk];
     for (int j = threadIdx.x; j < kH; j += kGroupThreads) {
-        s->b0[j] = m.b0[dec][j];
-        s->w1[j] = m.w1[dec][j];
-        for (int k = 0; k < 3; ++k) s->wxyz[j][k] = m.pos_inv ? 0.0f : W0[j * din + k];
+        s->b0[j] = b0[j];
+        s->w1[j] = w1[j];
+        for (int k = 0; k < 3; ++k) s->wxyz[j][k] = off == 0 ? 0.0f : W0[j * din + k];
         s->wxyz[j][3] = 0.0f;
     }
+    return g;
+}
+
+__device__ __forceinline__ GroupWeights stage_group(const ModelArgs& m, int dec, GroupLds* s) {
     if (m.res[0] <= 4) {
         const int S = m.res[0] + 1;
         const float4* g4 = reinterpret_cast<const float4*>(m.grid[0]);
         for (int j = threadIdx.x; j < S * S * S * (kC / 4); j += kGroupThreads) s->coarse[j] = g4[j];
     }
-    return g;
+    return stage_group_decoder(m.w0[dec], m.pos_inv ? kC : kC + 3, m.b0[dec], m.w1[dec], &s->dec);
+}
+
+// Channels 4 q .. 4 q + 3 of a query.
+__device__ __forceinline__ void store_features(GroupDecoder* s, uint32_t query, uint32_t q, const float4& f) {
+    *reinterpret_cast<float2*>(&s->feat[0][query][2 * q]) = make_float2(f.x, f.z);
+    *reinterpret_cast<float2*>(&s->feat[1][query][2 * q]) = make_float2(f.y, f.w);
+}
+
+// The decoder on the stored features: every thread, with the position of query
+// lane % 32.
+template <bool POSINV>
+__device__ __forceinline__ float group_decode(GroupDecoder* s, const GroupWeights& gw, float b1, float px, float py,
+                                              float pz) {
+    const uint32_t lane = lane_id(), n = lane & 31u, half = lane >> 5;
+    const int h = (int)(threadIdx.x >> 6);
+    __syncthreads();
+    f32x16_t c = {};
+    const float4* b4 = reinterpret_cast<const float4*>(s->feat[half][n]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float4 b = b4[k];
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 0], b.x, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 1], b.y, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 2], b.z, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 3], b.w, c, 0, 0, 0);
+    }
+    s->part[h][lane] = layer2_tile(c, h, half, s, !POSINV, px, py, pz);
+    __syncthreads();
+    float p = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) p += s->part[k][lane];
+    return halves_sum(p, p) + b1;
 }
 
 // Eight corner rows' float4 of this thread.
@@ -93,9 +134,8 @@ template <bool POSINV>
 __device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds* s, const GroupWeights& gw, float b1,
                                            float px, float py, float pz) {
     const uint32_t lane = lane_id(), n = lane & 31u, half = lane >> 5;
-    const int h = (int)(threadIdx.x >> 6);
     {
-        const int l = 2 * h + (int)half;  // NGLOD_MAX_LODS = 8 levels
+        const int l = 2 * (int)(threadIdx.x >> 6) + (int)half;  // NGLOD_MAX_LODS = 8 levels
         if (l <= lod) {
             const int r = m.res[l], S = r + 1;
             const AxisW ax = axis_weights(px, r);
@@ -128,28 +168,9 @@ __device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds
             group_rows(m.grid[l], m.res[l] + 1, s->base[l][ray], q, g);
             group_corners(g, s->w[l][ray], f);
         }
-        *reinterpret_cast<float2*>(&s->feat[0][ray][2 * q]) = make_float2(f.x, f.z);
-        *reinterpret_cast<float2*>(&s->feat[1][ray][2 * q]) = make_float2(f.y, f.w);
+        store_features(&s->dec, ray, q, f);
     }
-    __syncthreads();
-    f32x16_t c = {};
-    {
-        const float4* b4 = reinterpret_cast<const float4*>(s->feat[half][n]);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float4 b = b4[k];
-            c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 0], b.x, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 1], b.y, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 2], b.z, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x2f32(gw.a[4 * k + 3], b.w, c, 0, 0, 0);
-        }
-    }
-    s->part[h][lane] = layer2_tile(c, h, half, s, !POSINV, px, py, pz);
-    __syncthreads();
-    float p = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) p += s->part[k][lane];
-    return halves_sum(p, p) + b1;
+    return group_decode<POSINV>(&s->dec, gw, b1, px, py, pz);
 }
 
 }  // namespace nglod

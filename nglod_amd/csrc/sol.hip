@@ -6,8 +6,9 @@
 //                        by binary search instead of the reference's O(n*m) scan
 //   nglod_trace_sparse   SDF::sphereTrace + getNormal (sol-renderer/SDF.cu:218-472)
 //
-// The march is one persistent kernel: each lane owns a ray (refilled from a
-// queue when it retires) and runs the reference's per-ray recurrence: enter
+// The march is one persistent kernel (sol_march.hip; here, for tables that one
+// does not take, with a lane per ray): each ray, refilled from a queue when it
+// retires, runs the reference's per-ray recurrence: enter
 // the first voxel of its nugget list that contains or lies ahead of the
 // current point, evaluate the sparse SDF there (features summed over the
 // voxel's ancestors, decoder in registers), step, re-enter, at most 50 times;
@@ -19,7 +20,7 @@
 
 #include "api_common.hpp"
 #include "fp32_wave.hpp"
-#include "trace_common.hpp"
+#include "sol_common.hpp"
 
 namespace nglod {
 
@@ -31,62 +32,6 @@ __host__ __device__ __forceinline__ uint64_t morton_u64(uint32_t x, uint32_t y, 
         m |= (uint64_t)((x >> i) & 1u) << (3 * i + 2);
     }
     return m;
-}
-
-struct SolArgs {
-    int target, lod, din;
-    const int16_t* points;
-    int64_t psum_target;  // global index of the first point of level `target`
-    const uint32_t* tv;   // [P][8]
-    const int32_t* parent;
-    const int32_t* cc;    // [Nc][3]
-    const float* cf;      // [Nc][32]
-    const float* w0;
-    const float* b0;
-    const float* w1;
-    const float* b1;
-    // rays
-    const float* o;
-    const float* d;
-    int64_t n;
-    const int32_t* offs;  // [n+1] CSR over nuggets
-    const int32_t* nug;   // [M][2]
-    float* x;
-    float* t;
-    uint8_t* hit;
-    float* normal;
-    int32_t* iters;
-    uint32_t* queue;
-    unsigned long long* evals;
-    float r;  // voxel half size at `target`
-};
-
-__device__ __forceinline__ float sol_ray_aabb(float qx, float qy, float qz, float dx, float dy, float dz, float ivx,
-                                              float ivy, float ivz, float sx_, float sy_, float sz_, float cx, float cy,
-                                              float cz, float r) {
-    const float ox = qx - cx, oy = qy - cy, oz = qz - cz;
-    const float cmax = fmaxf(fmaxf(fabsf(ox), fabsf(oy)), fabsf(oz));
-    float winding = cmax < r ? -1.0f : 1.0f;
-    winding *= r;
-    if (winding < 0) return winding;
-    const float d0 = __builtin_fmaf(winding, sx_, -ox) * ivx;
-    const float d1 = __builtin_fmaf(winding, sy_, -oy) * ivy;
-    const float d2 = __builtin_fmaf(winding, sz_, -oz) * ivz;
-    const float ltxy = __builtin_fmaf(dy, d0, oy), ltxz = __builtin_fmaf(dz, d0, oz);
-    const float ltyx = __builtin_fmaf(dx, d1, ox), ltyz = __builtin_fmaf(dz, d1, oz);
-    const float ltzx = __builtin_fmaf(dx, d2, ox), ltzy = __builtin_fmaf(dy, d2, oy);
-    const bool t0 = (d0 >= 0.0f) && (fabsf(ltxy) < r) && (fabsf(ltxz) < r);
-    const bool t1 = (d1 >= 0.0f) && (fabsf(ltyx) < r) && (fabsf(ltyz) < r);
-    const bool t2 = (d2 >= 0.0f) && (fabsf(ltzx) < r) && (fabsf(ltzy) < r);
-    float ssx = 0.0f, ssy = 0.0f, ssz = 0.0f;
-    if (t0) ssx = sx_;
-    else if (t1) ssy = sy_;
-    else if (t2) ssz = sz_;
-    float dd = 0.0f;
-    if (ssx != 0.0f) dd = d0;
-    else if (ssy != 0.0f) dd = d1;
-    else if (ssz != 0.0f) dd = d2;
-    return dd;
 }
 
 // Sparse features at p, voxel cidx (global point index) and its ancestors,
@@ -313,7 +258,8 @@ struct SolRay {
     }
 };
 
-// Persistent sparse march: one ray per lane (SolRay), refilled from kQueues
+// Persistent sparse march of structures with more than kSolGroupLevels levels or
+// tables off their vectors' alignment (the others: launch_trace_sparse_group): one ray per lane (SolRay), refilled from kQueues
 // ray ranges (RayFeed); the features come from the sparse corner table, the
 // decoder is the FP32 MFMA one of the dense form (fp32_wave.hpp), staged in
 // LDS once per block.  512-thread blocks, as the dense FP32 march.
@@ -675,6 +621,8 @@ int nglod_trace_sparse(const nglod_sol_t* sol, const float* ray_o, const float* 
     rc = check_launch("clear_counters_kernel");
     if (rc) return rc;
     const bool posinv = a.din == kC;
+    if (a.lod < kSolGroupLevels && ((uintptr_t)a.points & 7u) == 0 && aligned16(a.cf))
+        return launch_trace_sparse_group(a, s);
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
             &per_cu, posinv ? trace_sparse_kernel<true> : trace_sparse_kernel<false>, kSparseBlock, 0) != hipSuccess ||
