@@ -366,7 +366,7 @@ int nglod_spc_raytrace(const uint8_t* octree, const uint32_t* prefix, const int1
                        void* workspace, size_t workspace_bytes, size_t* workspace_needed, void* stream);
 
 /* Workspace bytes nglod_spc_raytrace_async needs for n rays (a ticket
- * counter and 8 bytes per tile of 64 rays). */
+ * counter, 8 bytes per tile of 64 rays and 8 KiB per wave: at most 8 waves a CU). */
 size_t nglod_spc_raytrace_async_workspace_size(int64_t n);
 
 /* The same traversal and nugget list as nglod_spc_raytrace (spc_raytrace,

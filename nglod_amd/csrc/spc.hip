@@ -299,6 +299,7 @@ struct SpcBfsArgs {
     uint64_t* tile_state;  // [ntiles] (flag << 32 | count), zeroed before the launch
     uint32_t* status;      // [0] total nuggets, [1] flags: 1 = capacity exceeded, 2 = look-back gave up
     uint32_t* offs;        // [n + 1] CSR offsets of each ray's nuggets
+    uint32_t* kept;        // [gridDim.x][kBfsCap]: a wave's last list, until its place is known
     uint32_t ntiles;
     int64_t cap;           // nugget capacity (entries beyond it are not written)
 };
@@ -329,18 +330,21 @@ __device__ __forceinline__ RayConsts ray_consts(const float* o, const float* d, 
     return c;
 }
 
-__device__ __forceinline__ double shfl_d(double v, int src) {
-    const uint64_t b = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)b, src);
-    const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(b >> 32), src);
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
+// 2^-l, the cell size at level l in the unit cube.
+__device__ __forceinline__ float level_scale(int l) { return __uint_as_float((uint32_t)(127 - l) << 23); }
 
 __device__ __forceinline__ bool cell_hit(const RayConsts& c, int l, uint16_t px, uint16_t py, uint16_t pz) {
-    const float s1 = (float)(1.0 / (double)(float)(1u << l));
+    const float s1 = level_scale(l);
     const float s2 = s1 * s1;
     return face_eval(py, pz, -s2 * c.dz, s2 * c.dy, s1 * c.cx) && face_eval(px, pz, s2 * c.dz, -s2 * c.dx, s1 * c.cy) &&
            face_eval(px, py, -s2 * c.dy, s2 * c.dx, s1 * c.cz);
+}
+
+// face_eval by minima and maxima of the four values (the bounds 1 and -1 it starts
+// from do not decide, and a NaN counts for neither side, as there).
+__device__ __forceinline__ bool face_spans(float i, float j, float a, float b, float c) {
+    const float r0 = a * i + b * j + c, r1 = r0 + a, r2 = r0 + b, r3 = r1 + b;
+    return fminf(fminf(r0, r1), fminf(r2, r3)) <= 0.0f && fmaxf(fmaxf(r0, r1), fmaxf(r2, r3)) >= 0.0f;
 }
 
 // Octant of the ray origin relative to the centre of cell p at level l (the Order row).
@@ -405,22 +409,25 @@ __device__ __forceinline__ uint32_t wave_excl_scan_u32(uint32_t v, uint32_t lane
     return x - v;
 }
 
-// Decoupled look-back: publishes the tile's count, then sums its
-// predecessors' until one has published an inclusive sum; returns the
-// tile's exclusive prefix.  Predecessors took their tickets earlier and
-// publish their count before they wait on anyone, so the wait ends; the
-// spin limit only guards against a broken invariant (status flag 2).  A
+// Decoupled look-back: sums the counts that a tile's predecessors have published
+// until one has published an inclusive sum; returns the
+// tile's exclusive prefix.  Predecessors took their tickets earlier and a wave
+// publishes its tile's count before it waits for that tile or a later one, and
+// waits for an earlier one only once it holds no unpublished count, so the wait
+// ends; the spin limit only guards against a broken invariant (status flag 2).  A
 // state word carries its flag and its value together and no other data is
 // published with it, so the loads and stores are relaxed (device-scope
 // atomics, which bypass the CU's L1): an acquire load would also invalidate
 // the CU's L1 on every poll, under the waves that are still walking the
 // octree.
+__device__ __forceinline__ void publish_tile(const SpcBfsArgs& b, uint32_t tile, uint32_t count, uint32_t lane) {
+    if (lane == 0)
+        __hip_atomic_store(&b.tile_state[tile], (tile == 0 ? kTileInclusive : kTileAggregate) | count, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+
 __device__ uint32_t tile_lookback(const SpcBfsArgs& b, uint32_t tile, uint32_t count, uint32_t lane) {
-    if (tile == 0) {
-        if (lane == 0) __hip_atomic_store(&b.tile_state[0], kTileInclusive | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return 0u;
-    }
-    if (lane == 0) __hip_atomic_store(&b.tile_state[tile], kTileAggregate | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tile == 0) return 0u;
     uint32_t excl = 0;
     int64_t top = (int64_t)tile - 1;
     uint32_t spins = 0;
@@ -449,10 +456,68 @@ __device__ uint32_t tile_lookback(const SpcBfsArgs& b, uint32_t tile, uint32_t c
     return excl;
 }
 
+// A ray's values in the traversal's LDS table, for the children of one level's
+// cells: the face tests' s^2 d and s c at the children's cell size s, and h, the
+// origin in units of the parents' cells (a power of two away from its value in
+// the unit cube: comparing it in float with a cell's centre, a whole number and a
+// half, is exact, as octant_code's FP64 is).
+struct alignas(16) TileRay {
+    float dx, dy, dz, cx, cy, cz, hx, hy, hz, pad[3];
+};
+
+// Groups of eight parents a wave expands at a time: their loads are in flight
+// together.  A parent's point, octree byte and prefix sum do not depend on each
+// other, and a child's point is its parent's, doubled, plus its octant's bits, so
+// that a batch waits for memory once.  Bound: the vector ALU (60% busy; eight
+// waves a CU by LDS).  1280x720 rays, level 6, 3.65 M voxels: one group at a time,
+// the child's point and the order table loaded, FP64 octants 1.63 ms; four groups,
+// coordinates and comparisons in float 1.29; the order by selects 1.02; faces by
+// minima and maxima and lists kept back instead of waiting for their place (a
+// third of the time) 0.57.
+constexpr int kBfsGroups = 4;
+
+// kOrder[code][slot] by selects (as a table in memory it is a load between the
+// parent's and the child's).
+__device__ __forceinline__ uint32_t order_of(uint32_t code, uint32_t slot) {
+    const uint32_t r0 = code & 1u ? 0x67425301u : 0x76534210u, r1 = code & 1u ? 0x46507213u : 0x57416302u;
+    const uint32_t r2 = code & 1u ? 0x26307415u : 0x37216504u, r3 = code & 1u ? 0x04216537u : 0x15307426u;
+    const uint32_t lo = code & 2u ? r1 : r0, hi = code & 2u ? r3 : r2;
+    return ((code & 4u ? hi : lo) >> (4u * slot)) & 7u;
+}
+
 __global__ __launch_bounds__(64) void spc_bfs_kernel(SpcBfsArgs b) {
     __shared__ uint32_t lists[2][kBfsCap];
+    __shared__ TileRay rays[64];
     const SpcArgs& a = b.s;
     const uint32_t lane = threadIdx.x;
+    const bool whole = ((uintptr_t)a.pts & 7u) == 0;  // a point is one 8-byte load
+    // A finished tile's list waits here while the wave walks its next tile: its
+    // predecessors' counts are there by then.
+    uint32_t* kept = b.kept + (size_t)blockIdx.x * kBfsCap;
+    uint32_t kept_tile = b.ntiles, kept_count = 0, kept_lo = 0;
+    auto place_kept = [&]() {
+        if (kept_tile >= b.ntiles) return;
+        const uint32_t base = tile_lookback(b, kept_tile, kept_count, lane);
+        const int64_t r0 = (int64_t)kept_tile * 64;
+        if (r0 + lane < a.n) b.offs[r0 + lane] = base + kept_lo;
+        for (uint32_t j = lane; j < kept_count; j += 64) {
+            const uint32_t e = kept[j];
+            const int64_t pos = (int64_t)base + j;
+            if (pos < b.cap) {
+                int2 v;
+                v.x = (int32_t)(r0 + (e >> 26));
+                v.y = (int32_t)(e & kNodeMask);
+                reinterpret_cast<int2*>(a.nug)[pos] = v;
+            }
+        }
+        if (kept_tile == b.ntiles - 1 && lane == 0) {
+            const uint32_t total = base + kept_count;
+            b.offs[a.n] = total;
+            b.status[0] = total;
+            if ((int64_t)total > b.cap) atomicOr(&b.status[1], 1u);
+        }
+        kept_tile = b.ntiles;
+    };
     for (;;) {
         uint32_t tile = 0;
         if (lane == 0) tile = atomicAdd(b.ticket, 1u);
@@ -474,40 +539,53 @@ __global__ __launch_bounds__(64) void spc_bfs_kernel(SpcBfsArgs b) {
             const uint32_t parents = count;
             uint32_t next = 0;
             const int32_t base_l = a.psum[l], base_n = a.psum[l + 1];
-            for (uint32_t j0 = 0; j0 < parents; j0 += 8) {
-                const uint32_t pi = j0 + (lane >> 3);
-                const uint32_t slot = lane & 7u;
-                const bool act = pi < parents;
-                const uint32_t e = act ? lists[cur][pi] : 0u;
-                const int rl = (int)(e >> 26);
-                const uint32_t k = e & kNodeMask;
-                RayConsts c;
-                c.dx = __shfl(mine.dx, rl);
-                c.dy = __shfl(mine.dy, rl);
-                c.dz = __shfl(mine.dz, rl);
-                c.cx = __shfl(mine.cx, rl);
-                c.cy = __shfl(mine.cy, rl);
-                c.cz = __shfl(mine.cz, rl);
-                c.hx = shfl_d(mine.hx, rl);
-                c.hy = shfl_d(mine.hy, rl);
-                c.hz = shfl_d(mine.hz, rl);
-                bool h = false;
-                uint32_t child = 0;
-                if (act) {
-                    const int16_t* p = a.pts + 4 * ((int64_t)base_l + k);
-                    const uint8_t ob = a.oct[base_l + k];
-                    const uint32_t jj = kOrder[octant_code(c, l, p)][slot];
-                    if (ob & (1u << jj)) {
-                        const uint32_t rank = (uint32_t)__builtin_popcount(ob & ((2u << jj) - 1u));
-                        child = a.S[base_l + k] + rank - (uint32_t)base_n;
-                        const int16_t* q = a.pts + 4 * ((int64_t)base_n + child);
-                        h = cell_hit(c, l + 1, (uint16_t)q[0], (uint16_t)q[1], (uint16_t)q[2]);
+            {
+                const float s1 = level_scale(l + 1), s2 = s1 * s1, up = __uint_as_float((uint32_t)(127 + l) << 23);
+                rays[lane] = TileRay{s2 * mine.dx, s2 * mine.dy, s2 * mine.dz, s1 * mine.cx, s1 * mine.cy, s1 * mine.cz,
+                                     (float)mine.hx * up, (float)mine.hy * up, (float)mine.hz * up, {0.0f, 0.0f, 0.0f}};
+            }
+            __syncthreads();
+            const uint32_t slot = lane & 7u;
+            for (uint32_t j0 = 0; j0 < parents; j0 += 8 * kBfsGroups) {
+                uint32_t e[kBfsGroups], ob[kBfsGroups], sum[kBfsGroups];
+                int2 p[kBfsGroups];
+#pragma unroll
+                for (int u = 0; u < kBfsGroups; ++u) {
+                    const uint32_t pi = j0 + 8 * u + (lane >> 3);
+                    const bool act = pi < parents;
+                    e[u] = lists[cur][act ? pi : j0];
+                    const int64_t k = (int64_t)base_l + (e[u] & kNodeMask);
+                    ob[u] = act ? a.oct[k] : 0u;
+                    sum[u] = a.S[k];
+                    if (whole) {
+                        p[u] = *reinterpret_cast<const int2*>(a.pts + 4 * k);
+                    } else {
+                        const int16_t* q = a.pts + 4 * k;
+                        p[u].x = (int)((uint32_t)(uint16_t)q[0] | ((uint32_t)(uint16_t)q[1] << 16));
+                        p[u].y = (int)(uint16_t)q[2];
                     }
                 }
-                const uint64_t hm = __ballot(h);
-                const uint32_t pos = next + mask_rank(hm);
-                if (h && pos < (uint32_t)kBfsCap) lists[cur ^ 1][pos] = ((uint32_t)rl << 26) | child;
-                next += (uint32_t)__popcll(hm);
+#pragma unroll
+                for (int u = 0; u < kBfsGroups; ++u) {
+                    const TileRay c = rays[e[u] >> 26];
+                    const float px = (float)(int16_t)(p[u].x & 0xffff), py = (float)(int16_t)(p[u].x >> 16),
+                                pz = (float)(int16_t)(p[u].y & 0xffff);
+                    uint32_t code = c.hx > px + 0.5f ? 4u : 0u;
+                    code += c.hy > py + 0.5f ? 2u : 0u;
+                    code += c.hz > pz + 0.5f ? 1u : 0u;
+                    const uint32_t jj = order_of(code, slot);
+                    const float qx = __builtin_fmaf(2.0f, px, jj & 4u ? 1.0f : 0.0f),
+                                qy = __builtin_fmaf(2.0f, py, jj & 2u ? 1.0f : 0.0f),
+                                qz = __builtin_fmaf(2.0f, pz, jj & 1u ? 1.0f : 0.0f);
+                    const uint32_t child = sum[u] + (uint32_t)__builtin_popcount(ob[u] & ((2u << jj) - 1u)) -
+                                           (uint32_t)base_n;
+                    const bool h = ((ob[u] >> jj) & 1u) && face_spans(qy, qz, -c.dz, c.dy, c.cx) &&
+                                   face_spans(qx, qz, c.dz, -c.dx, c.cy) && face_spans(qx, qy, -c.dy, c.dx, c.cz);
+                    const uint64_t hm = __ballot(h);
+                    const uint32_t pos = next + mask_rank(hm);
+                    if (h && pos < (uint32_t)kBfsCap) lists[cur ^ 1][pos] = (e[u] & ~kNodeMask) | child;
+                    next += (uint32_t)__popcll(hm);
+                }
             }
             __syncthreads();  // one wave per block: orders the list writes before the next level's reads
             if (next > (uint32_t)kBfsCap) {
@@ -519,7 +597,8 @@ __global__ __launch_bounds__(64) void spc_bfs_kernel(SpcBfsArgs b) {
         }
         __syncthreads();
         if (!overflow) {
-            const uint32_t base = tile_lookback(b, tile, count, lane);
+            publish_tile(b, tile, count, lane);
+            place_kept();
             // this ray's first entry: lower bound of lane << 26 in the sorted list
             uint32_t lo = 0, hi = count;
             while (lo < hi) {
@@ -527,28 +606,17 @@ __global__ __launch_bounds__(64) void spc_bfs_kernel(SpcBfsArgs b) {
                 if ((lists[cur][mid] >> 26) < lane) lo = mid + 1;
                 else hi = mid;
             }
-            if (valid) b.offs[ray] = base + lo;
-            for (uint32_t j = lane; j < count; j += 64) {
-                const uint32_t e = lists[cur][j];
-                const int64_t pos = (int64_t)base + j;
-                if (pos < b.cap) {
-                    int2 v;
-                    v.x = (int32_t)(r0 + (e >> 26));
-                    v.y = (int32_t)(e & kNodeMask);
-                    reinterpret_cast<int2*>(a.nug)[pos] = v;
-                }
-            }
-            if (tile == b.ntiles - 1 && lane == 0) {
-                const uint32_t total = base + count;
-                b.offs[a.n] = total;
-                b.status[0] = total;
-                if ((int64_t)total > b.cap) atomicOr(&b.status[1], 1u);
-            }
+            for (uint32_t j = lane; j < count; j += 64) kept[j] = lists[cur][j];
+            kept_tile = tile;
+            kept_count = count;
+            kept_lo = lo;
         } else {
             // the per-ray depth-first walk, the two lists as 64 stacks
             uint32_t* st = &lists[0][0] + lane * kBfsStack;
             const uint32_t mycount = valid ? dfs_one<false>(a, mine, ray, st, 0u, 0) : 0u;
             const uint32_t total = wave_sum_u32(mycount);
+            publish_tile(b, tile, total, lane);
+            place_kept();
             const uint32_t base = tile_lookback(b, tile, total, lane);
             const uint32_t w = base + wave_excl_scan_u32(mycount, lane);
             if (valid) {
@@ -564,6 +632,7 @@ __global__ __launch_bounds__(64) void spc_bfs_kernel(SpcBfsArgs b) {
         }
         __syncthreads();  // the next tile rewrites the lists
     }
+    place_kept();
 }
 
 __global__ void spc_bfs_clear_kernel(uint32_t* ticket, uint64_t* state, uint32_t ntiles, uint32_t* status) {
@@ -658,8 +727,17 @@ static int spc_args(const uint8_t* octree, const uint32_t* prefix, const int16_t
 
 static uint32_t bfs_tiles(int64_t n) { return (uint32_t)((n + 63) / 64); }
 
-// Workspace of the single pass: the ticket counter, then the tiles' states.
-static size_t bfs_workspace_size(int64_t n) { return 256 + a256((size_t)bfs_tiles(n) * 8); }
+// Waves of the traversal: eight a CU (its LDS holds no more).
+static unsigned bfs_grid(int64_t n) {
+    const int64_t most = (int64_t)device_cu_count() * 8, tiles = bfs_tiles(n);
+    return (unsigned)(tiles < most ? tiles : most);
+}
+
+// Workspace of the single pass: the ticket counter, the tiles' states, the waves'
+// kept lists.
+static size_t bfs_workspace_size(int64_t n) {
+    return 256 + a256((size_t)bfs_tiles(n) * 8) + (size_t)bfs_grid(n) * kBfsCap * 4;
+}
 
 static int spc_raytrace_bfs(const SpcArgs& a, int32_t* nuggets, int64_t cap, uint32_t* ray_offsets, uint32_t* status,
                             void* workspace, hipStream_t s) {
@@ -668,6 +746,7 @@ static int spc_raytrace_bfs(const SpcArgs& a, int32_t* nuggets, int64_t cap, uin
     b.s.nug = nuggets;
     b.ticket = (uint32_t*)workspace;
     b.tile_state = (uint64_t*)((char*)workspace + 256);
+    b.kept = (uint32_t*)((char*)workspace + 256 + a256((size_t)bfs_tiles(a.n) * 8));
     b.status = status;
     b.offs = ray_offsets;
     b.ntiles = bfs_tiles(a.n);
@@ -676,12 +755,7 @@ static int spc_raytrace_bfs(const SpcArgs& a, int32_t* nuggets, int64_t cap, uin
                        b.ntiles, b.status);
     int rc = check_launch("spc_bfs_clear_kernel");
     if (rc) return rc;
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, spc_bfs_kernel, 64, 0) != hipSuccess || per_cu <= 0)
-        per_cu = 8;
-    const int64_t cap_blocks = (int64_t)device_cu_count() * per_cu;
-    const unsigned grid = (unsigned)((int64_t)b.ntiles < cap_blocks ? (int64_t)b.ntiles : cap_blocks);
-    hipLaunchKernelGGL(spc_bfs_kernel, dim3(grid), dim3(64), 0, s, b);
+    hipLaunchKernelGGL(spc_bfs_kernel, dim3(bfs_grid(a.n)), dim3(64), 0, s, b);
     return check_launch("spc_bfs_kernel");
 }
 
