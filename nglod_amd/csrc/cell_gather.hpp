@@ -43,6 +43,8 @@ __device__ __forceinline__ uint32_t cell_row(uint32_t n) {
 
 // One more level onto f.  Every lane of the wave calls this with a position
 // (lanes without a query: any position); use1: tile 1 holds a query.
+// ONLY: f is this level alone (what it holds is not read).
+template <bool ONLY = false>
 __device__ __forceinline__ void gather_cells(const float* __restrict__ grid, int r, float px, float py, float pz,
                                              uint32_t lane, bool use1, CellFeatures& f) {
     const int S = r + 1;
@@ -65,6 +67,10 @@ __device__ __forceinline__ void gather_cells(const float* __restrict__ grid, int
         float v[kC];
 #pragma unroll
         for (int kk = 0; kk < kC / 2; ++kk) {
+            if (ONLY) {
+                v[2 * kk] = v[2 * kk + 1] = 0.0f;
+                continue;
+            }
             const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(f.t[0][kk]), __float_as_uint(f.t[1][kk]),
                                                              false, false);
             v[2 * kk] = __uint_as_float(sw[0]);
@@ -102,6 +108,7 @@ __device__ __forceinline__ void gather_cells(const float* __restrict__ grid, int
     const uint32_t n = lane & 31u, half = lane >> 5;
     const float* mine = grid + half * kC + cell_row(n);  // corner 2 s + half: x = half
     const size_t sy = (size_t)S * kC, sz = (size_t)S * S * kC;
+    uint64_t left = ONLY ? all : 0;  // queries of a tile whose features are not set yet: all or none
     for (uint64_t m = all; m != 0;) {
         const uint32_t cell = (uint32_t)__builtin_amdgcn_readlane((int)base, __ffsll((unsigned long long)m) - 1);
         const uint64_t same = __ballot(base == cell) & all;
@@ -112,11 +119,12 @@ __device__ __forceinline__ void gather_cells(const float* __restrict__ grid, int
         for (int t = 0; t < 2; ++t) {
             const uint32_t here = (uint32_t)(same >> (32 * t));
             if (here == 0) continue;
-            f32x16_t d = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, w[t][0], f.t[t], 0, 0, 0);
+            f32x16_t d = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, w[t][0], ONLY ? f32x16_t{} : f.t[t], 0, 0, 0);
             d = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, w[t][1], d, 0, 0, 0);
             d = __builtin_amdgcn_mfma_f32_32x32x2f32(a2, w[t][2], d, 0, 0, 0);
             d = __builtin_amdgcn_mfma_f32_32x32x2f32(a3, w[t][3], d, 0, 0, 0);
-            if (here == 0xffffffffu) {
+            if (here == 0xffffffffu || (ONLY && (uint32_t)(left >> (32 * t)) != 0u)) {
+                left &= ~(0xffffffffull << (32 * t));
                 f.t[t] = d;
             } else {
                 const bool in = (here >> n) & 1u;
@@ -130,28 +138,29 @@ __device__ __forceinline__ void gather_cells(const float* __restrict__ grid, int
 // The decoder on such features (decode_fp32_wave from its B operands on).
 template <bool POSINV>
 __device__ __forceinline__ float decode_cells(const CellFeatures& f, const Fp32Lds* s, float b1, uint32_t lane,
-                                              bool use1, float px, float py, float pz) {
+                                              float px, float py, float pz) {
     const uint32_t half = lane >> 5;
     float qx0, qy0, qz0, qx1, qy1, qz1;
     tile_coords(px, py, pz, qx0, qy0, qz0, qx1, qy1, qz1);
     float part[2] = {0.0f, 0.0f};
 #pragma unroll 1
     for (int h = 0; h < 4; ++h) {
+        // both tiles whether used or not: one block, so that a tile's ReLU runs beside
+        // the other's products
+        f32x16_t c[2] = {{}, {}};
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            if (t == 1 && !use1) continue;
-            f32x16_t c = {};
 #pragma unroll
             for (int kq = 0; kq < 4; ++kq) {
                 const float4 a = s->afrag[(h * 4 + kq) * 64 + lane];
-                c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, f.t[t][4 * kq + 0], c, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, f.t[t][4 * kq + 1], c, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, f.t[t][4 * kq + 2], c, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, f.t[t][4 * kq + 3], c, 0, 0, 0);
+                c[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, f.t[t][4 * kq + 0], c[t], 0, 0, 0);
+                c[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, f.t[t][4 * kq + 1], c[t], 0, 0, 0);
+                c[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, f.t[t][4 * kq + 2], c[t], 0, 0, 0);
+                c[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, f.t[t][4 * kq + 3], c[t], 0, 0, 0);
             }
-            part[t] += layer2_tile(c, h, half, s, !POSINV, t == 0 ? qx0 : qx1, t == 0 ? qy0 : qy1,
-                                   t == 0 ? qz0 : qz1);
         }
+        part[0] += layer2_tile(c[0], h, half, s, !POSINV, qx0, qy0, qz0);
+        part[1] += layer2_tile(c[1], h, half, s, !POSINV, qx1, qy1, qz1);
     }
     return halves_sum(part[0], part[1]) + b1;
 }

@@ -28,7 +28,7 @@ __global__ __launch_bounds__(256) void sdf_ordered_fp32_kernel(ModelArgs m, int 
         const bool use1 = w * 64 + 32 < n;
         CellFeatures f = zero_cell_features();
         for (int l = 0; l <= lod; ++l) gather_cells(m.grid[l], m.res[l], px, py, pz, lane, use1, f);
-        const float d = decode_cells<POSINV>(f, &lds, b1, lane, use1, px, py, pz);
+        const float d = decode_cells<POSINV>(f, &lds, b1, lane, px, py, pz);
         if (valid) out[i] = d;
     }
 }

@@ -9,8 +9,10 @@
 // matcap bilinear lookup and the blur run in FP64 as SciPy does.
 #include <math.h>
 
+#include <type_traits>
+
 #include "api_common.hpp"
-#include "fp32_wave.hpp"
+#include "cell_gather.hpp"
 #include "split_wave.hpp"
 #include "trace_common.hpp"
 
@@ -77,12 +79,15 @@ __global__ __launch_bounds__(256) void shadow_rays_kernel(const float* __restric
 // dist[i] = 0.1 * 0.25 * ((i + 1) / 41)^1.6 along the normal, r = sdf(x + n *
 // dist[i]) (a plane hit takes min(r, dist[i])), acc += 3.5 * relu(dist[i] - r -
 // 0.0015); ao = clamp(1 - acc, 0.1, 1)^2, and 1 where neither hit is set.
-// Persistent: lanes claim the marked rays in frame order (claim_hits), each
-// runs its 40 taps through the FP32 MFMA decoder, LODs 0-1 from LDS.
+// A wave takes `chunk` (at most kAoRays) rays at a time and spreads the (hit,
+// tap) pairs over its lanes, 64 a round: the taps of a hit lie within 0.025 of each
+// other, so a round's 64 points fall into few cells, which are interpolated cell
+// by cell on the matrix cores (cell_gather.hpp), and no lane waits for another's
+// hit.  A hit's taps are added in their order afterwards.
 struct AoArgs {
     ModelArgs m;
     int lod, dec;
-    CoarsePlan coarse;
+    int chunk;
     const float* x;
     const float* normal;
     const uint8_t* hit;
@@ -101,91 +106,117 @@ __global__ __launch_bounds__(256) void ao_fill_kernel(const uint8_t* __restrict_
     if (!hit[i] && !(plane && plane[i])) ao[i] = 1.0f;
 }
 
-template <bool POSINV>
-__global__ __launch_bounds__(kMarchBlock) void ao_kernel(AoArgs a) {
-    __shared__ Fp32Lds lds;
-    __shared__ CoarseLds32 coarse;
-    stage_fp32_lds(a.m, a.dec, &lds);
-    stage_coarse32(a.m, a.coarse, &coarse);
+constexpr int kAoRays = 32;
+constexpr int kAoBlock = 256;
+
+// A wave's rays of the current claim.
+struct AoWaveLds {
+    float p[kAoRays][3], n[kAoRays][3];
+    uint32_t id[kAoRays];
+    uint32_t on_plane[kAoRays];
+    float u[kAoRays * (kAoTaps + 1)];  // [hit][tap], one float apart from the next hit's bank
+};
+
+template <bool SPLIT>
+struct AoLds {
+    typename std::conditional<SPLIT, SplitLds, Fp32Lds>::type dec;
+    float dist[kAoTaps];
+    AoWaveLds wave[kAoBlock / 64];
+};
+
+// SPLIT: the mixed form, on the FP32 cumulative grid (one level) with the decoder
+// of the mixed trace's FP32 pass (exact three-term BF16 splits, FP32-level
+// results); else every level and the FP32 decoder.  Bound: the matrix cores (60% of
+// the cycles in the mixed form, three waves a SIMD by registers) and the vector
+// ALU (45%).  0.69 M hits at LOD 4, against a lane per hit and its taps in a row:
+// mixed 1.44 -> 1.25 ms, with xyz inputs 1.74 -> 1.42, FP32 3.84 -> 3.31; 3000 hits:
+// 454 -> 88 us and 1012 -> 97.  Rays a claim: eight (five full rounds of 64
+// pairs) while that fills the GPU's waves, 32 from four claims a wave on.
+template <bool POSINV, bool SPLIT>
+__global__ __launch_bounds__(kAoBlock, 3) void ao_kernel(AoArgs a) {
+    __shared__ AoLds<SPLIT> lds;
+    if constexpr (SPLIT)
+        stage_split_lds(a.m, a.dec, &lds.dec);
+    else
+        stage_fp32_lds(a.m, a.dec, &lds.dec);
+    for (int j = threadIdx.x; j < kAoTaps; j += kAoBlock) lds.dist[j] = a.dist[j];
     __syncthreads();
     const float b1 = a.m.b1[a.dec][0];
     const uint32_t lane = lane_id();
-    bool drained = false;
+    AoWaveLds& w = lds.wave[threadIdx.x >> 6];
+    auto wave_sync = [] {  // orders this wave's LDS writes before its later reads
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
     for (;;) {
-        const int64_t id = claim_hits(a.counter, a.hit, (uint32_t)a.n, lane, drained, a.plane);
-        const bool valid = id >= 0;
-        if (__ballot(valid) == 0) break;
-        float p0 = 0.0f, p1 = 0.0f, p2 = 0.0f, n0 = 0.0f, n1 = 0.0f, n2 = 0.0f;
-        bool on_plane = false;
-        if (valid) {
-            p0 = a.x[3 * id];
-            p1 = a.x[3 * id + 1];
-            p2 = a.x[3 * id + 2];
-            n0 = a.normal[3 * id];
-            n1 = a.normal[3 * id + 1];
-            n2 = a.normal[3 * id + 2];
-            on_plane = !a.hit[id];
+        uint32_t claim = 0;
+        if (lane == 0) claim = atomicAdd(a.counter, 1u);
+        const int64_t first = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)claim) * a.chunk;
+        if (first >= a.n) break;
+        const int64_t id = first + lane;
+        const bool have = lane < (uint32_t)a.chunk && id < a.n;
+        const bool hit = have && a.hit[id] != 0;
+        const bool marked = hit || (have && a.plane && a.plane[id]);
+        const uint64_t m = __ballot(marked);
+        if (m == 0) continue;
+        wave_sync();
+        if (marked) {
+            const uint32_t s = mask_rank(m);
+            for (int k = 0; k < 3; ++k) {
+                w.p[s][k] = a.x[3 * id + k];
+                w.n[s][k] = a.normal[3 * id + k];
+            }
+            w.id[s] = (uint32_t)id;
+            w.on_plane[s] = hit ? 0u : 1u;
         }
-        float acc = 0.0f;
+        wave_sync();
+        const int hits = __popcll(m), pairs = hits * kAoTaps;
 #pragma unroll 1
-        for (int k = 0; k < kAoTaps; ++k) {
-            const float dk = a.dist[k];
-            const float q0 = p0 + n0 * dk, q1 = p1 + n1 * dk, q2 = p2 + n2 * dk;
-            float r = sdf_fp32_wave<POSINV>(a.m, a.lod, &lds, b1, lane, valid, q0, q1, q2, a.coarse, &coarse);
-            if (on_plane) r = fminf(r, dk);
+        for (int j = 0; j < pairs; j += 64) {
+            const int i = j + (int)lane < pairs ? j + (int)lane : pairs - 1;  // no cells of their own past the end
+            const int s = i / kAoTaps, k = i - s * kAoTaps;
+            const float dk = lds.dist[k];
+            const float q0 = w.p[s][0] + w.n[s][0] * dk, q1 = w.p[s][1] + w.n[s][1] * dk,
+                        q2 = w.p[s][2] + w.n[s][2] * dk;
+            const bool use1 = j + 32 < pairs;
+            CellFeatures f;
+            float r;
+            if constexpr (SPLIT) {
+                gather_cells<true>(a.m.grid[0], a.m.res[0], q0, q1, q2, lane, use1, f);
+                r = decode_split_tiles<POSINV>(f.t, &lds.dec, b1, lane, q0, q1, q2);
+            } else {
+                f = zero_cell_features();
+                for (int l = 0; l <= a.lod; ++l) gather_cells(a.m.grid[l], a.m.res[l], q0, q1, q2, lane, use1, f);
+                r = decode_cells<POSINV>(f, &lds.dec, b1, lane, q0, q1, q2);
+            }
+            if (w.on_plane[s]) r = fminf(r, dk);
             const float u = (dk - r) - 0.0015f;
-            acc = acc + 3.5f * (u > 0.0f ? u : 0.0f);
+            if (j + (int)lane < pairs) w.u[s * (kAoTaps + 1) + k] = u > 0.0f ? u : 0.0f;
         }
-        if (valid) {
+        wave_sync();
+        if ((int)lane < hits) {
+            float acc = 0.0f;
+            for (int k = 0; k < kAoTaps; ++k) acc = acc + 3.5f * w.u[lane * (kAoTaps + 1) + k];
             float v = 1.0f - acc;
             v = v < 0.1f ? 0.1f : (v > 1.0f ? 1.0f : v);
-            a.ao[id] = v * v;
+            a.ao[w.id[lane]] = v * v;
         }
     }
 }
 
-// The mixed form's AO: the same loop on the FP32 cumulative grid (one level,
-// no coarse levels to stage) with the decoder of the mixed trace's FP32 pass
-// (exact three-term BF16 splits on the matrix cores, FP32-level results).
-template <bool POSINV>
-__global__ __launch_bounds__(kMarchBlock) void ao_split_kernel(AoArgs a) {
-    __shared__ SplitLds lds;
-    stage_split_lds(a.m, a.dec, &lds);
-    __syncthreads();
-    const float b1 = a.m.b1[a.dec][0];
-    const uint32_t lane = lane_id();
-    bool drained = false;
-    for (;;) {
-        const int64_t id = claim_hits(a.counter, a.hit, (uint32_t)a.n, lane, drained, a.plane);
-        const bool valid = id >= 0;
-        if (__ballot(valid) == 0) break;
-        float p0 = 0.0f, p1 = 0.0f, p2 = 0.0f, n0 = 0.0f, n1 = 0.0f, n2 = 0.0f;
-        bool on_plane = false;
-        if (valid) {
-            p0 = a.x[3 * id];
-            p1 = a.x[3 * id + 1];
-            p2 = a.x[3 * id + 2];
-            n0 = a.normal[3 * id];
-            n1 = a.normal[3 * id + 1];
-            n2 = a.normal[3 * id + 2];
-            on_plane = !a.hit[id];
-        }
-        float acc = 0.0f;
-#pragma unroll 1
-        for (int k = 0; k < kAoTaps; ++k) {
-            const float dk = a.dist[k];
-            const float q0 = p0 + n0 * dk, q1 = p1 + n1 * dk, q2 = p2 + n2 * dk;
-            float r = sdf_split_wave<POSINV>(a.m, &lds, b1, lane, valid, q0, q1, q2);
-            if (on_plane) r = fminf(r, dk);
-            const float u = (dk - r) - 0.0015f;
-            acc = acc + 3.5f * (u > 0.0f ? u : 0.0f);
-        }
-        if (valid) {
-            float v = 1.0f - acc;
-            v = v < 0.1f ? 0.1f : (v > 1.0f ? 1.0f : v);
-            a.ao[id] = v * v;
-        }
-    }
+template <bool POSINV, bool SPLIT>
+static int launch_ao(AoArgs& a, hipStream_t s) {
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ao_kernel<POSINV, SPLIT>, kAoBlock, 0) != hipSuccess ||
+        per_cu <= 0)
+        per_cu = 1;
+    const int64_t cap = (int64_t)device_cu_count() * per_cu, waves = cap * (kAoBlock / 64);
+    // eight rays make five full rounds; fewer claims where they still fill the waves
+    a.chunk = a.n >= 4 * kAoRays * waves ? kAoRays : (a.n >= 64 * waves ? 16 : 8);
+    const int64_t want = (a.n + (int64_t)a.chunk * (kAoBlock / 64) - 1) / ((int64_t)a.chunk * (kAoBlock / 64));
+    hipLaunchKernelGGL((ao_kernel<POSINV, SPLIT>), dim3((unsigned)(want < cap ? want : cap)), dim3(kAoBlock), 0, s, a);
+    return check_launch("ao_kernel");
 }
 
 // ---------------------------------------------------------------------------
@@ -364,7 +395,6 @@ extern "C" int nglod_ao(const nglod_model_t* model, const float* x, const float*
     // the mixed AO kernel gathers one level, the cumulative grid of the LOD
     if (form == NGLOD_MIXED && (a.lod != 0 || a.m.num_lods != 1))
         return fail(NGLOD_ERR_ARG, "mixed form: one cumulative level (gather lod 0)");
-    a.coarse = coarse_plan(a.m, a.lod);
     a.x = x;
     a.normal = normal;
     a.hit = hit;
@@ -378,16 +408,8 @@ extern "C" int nglod_ao(const nglod_model_t* model, const float* x, const float*
     hipLaunchKernelGGL(ao_fill_kernel, dim3(blocks_for(n)), dim3(256), 0, s, hit, plane_hit, n, ao, a.counter);
     rc = check_launch("ao_fill_kernel");
     if (rc) return rc;
-    int per_cu = 0;
-    auto kern = form == NGLOD_MIXED ? (a.m.pos_inv ? ao_split_kernel<true> : ao_split_kernel<false>)
-                                    : (a.m.pos_inv ? ao_kernel<true> : ao_kernel<false>);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kMarchBlock, 0) != hipSuccess || per_cu <= 0)
-        per_cu = 1;
-    const int64_t want = (n + kMarchBlock - 1) / kMarchBlock;
-    const int64_t cap = (int64_t)device_cu_count() * per_cu;
-    const unsigned grid = (unsigned)(want < cap ? want : cap);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(kMarchBlock), 0, s, a);
-    return check_launch("ao_kernel");
+    if (form == NGLOD_MIXED) return a.m.pos_inv ? launch_ao<true, true>(a, s) : launch_ao<false, true>(a, s);
+    return a.m.pos_inv ? launch_ao<true, false>(a, s) : launch_ao<false, false>(a, s);
 }
 
 // SciPy's _gaussian_kernel1d(sigma = 2, radius 8): phi = exp(-0.5 / sigma^2 *

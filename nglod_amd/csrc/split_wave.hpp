@@ -37,17 +37,23 @@ struct SplitLds {
 };
 
 // x = h + m + l exactly (finite x; the grids and weights are far from the
-// BF16 underflow range).
-__device__ __forceinline__ void split3(float x, __bf16& h, __bf16& m, __bf16& l) {
-    h = (__bf16)x;
-    const float r = x - (float)h;
-    m = (__bf16)r;
-    l = (__bf16)(r - (float)m);
-}
-
-__device__ __forceinline__ uint32_t bf16_pair(__bf16 lo, __bf16 hi) {
-    const bf16x2v v = {lo, hi};
-    return __builtin_bit_cast(uint32_t, v);
+// BF16 underflow range), of two values, each part as a pair: a pair's residuals come from its own
+// bits (one conversion per pair and part instead of one per value and one to
+// pack them).
+__device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+    const auto pair = [](float a, float b) {
+        const bf16x2v v = {(__bf16)a, (__bf16)b};
+        return __builtin_bit_cast(uint32_t, v);
+    };
+    const auto rest = [](uint32_t p, float& a, float& b) {
+        a = a - __uint_as_float(p << 16);
+        b = b - __uint_as_float(p & 0xffff0000u);
+    };
+    h = pair(x0, x1);
+    rest(h, x0, x1);
+    m = pair(x0, x1);
+    rest(m, x0, x1);
+    l = pair(x0, x1);
 }
 
 // Stage decoder (W0 [128][din], din = 32 or 35 with xyz first; b0; w1) into
@@ -65,13 +71,9 @@ __device__ __forceinline__ void stage_split_lds_raw(const float* W0, int din, co
         uint32_t ph[4], pm[4], pl[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            __bf16 h0, m0, l0, h1, m1, l1;
             // elements e = 2q, 2q + 1: channels 2*(8kb + e) + lane/32
-            split3(W0[row * din + off + 2 * (8 * kb + 2 * q) + (lane >> 5)], h0, m0, l0);
-            split3(W0[row * din + off + 2 * (8 * kb + 2 * q + 1) + (lane >> 5)], h1, m1, l1);
-            ph[q] = bf16_pair(h0, h1);
-            pm[q] = bf16_pair(m0, m1);
-            pl[q] = bf16_pair(l0, l1);
+            split3_pair(W0[row * din + off + 2 * (8 * kb + 2 * q) + (lane >> 5)],
+                        W0[row * din + off + 2 * (8 * kb + 2 * q + 1) + (lane >> 5)], ph[q], pm[q], pl[q]);
         }
         s->wfrag[0][j] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
         s->wfrag[1][j] = make_uint4(pm[0], pm[1], pm[2], pm[3]);
@@ -107,12 +109,7 @@ __device__ __forceinline__ void split_afrag(const Fp32Lds* s, int h, int kb, uin
     uint32_t ph[4], pm[4], pl[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        __bf16 h0, m0, l0, h1, m1, l1;
-        split3(v[2 * q], h0, m0, l0);
-        split3(v[2 * q + 1], h1, m1, l1);
-        ph[q] = bf16_pair(h0, h1);
-        pm[q] = bf16_pair(m0, m1);
-        pl[q] = bf16_pair(l0, l1);
+        split3_pair(v[2 * q], v[2 * q + 1], ph[q], pm[q], pl[q]);
     }
     ah = __builtin_bit_cast(bf16x8, make_uint4(ph[0], ph[1], ph[2], ph[3]));
     am = __builtin_bit_cast(bf16x8, make_uint4(pm[0], pm[1], pm[2], pm[3]));
@@ -165,21 +162,14 @@ __device__ __forceinline__ float decode_split_wave(const float (&f)[kC], const L
         uint32_t th[2][4], tm[2][4], tl[2][4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            __bf16 h[2][2], m[2][2], l[2][2];  // [tile][element parity]
+            const int kk = 8 * kb + 2 * q;  // channel pairs kk, kk + 1
+            const auto s0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(f[2 * kk]), __float_as_uint(f[2 * kk + 1]),
+                                                             false, false);
+            const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(f[2 * kk + 2]),
+                                                             __float_as_uint(f[2 * kk + 3]), false, false);
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                const int kk = 8 * kb + 2 * q + p;  // channel pair
-                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(f[2 * kk]),
-                                                                 __float_as_uint(f[2 * kk + 1]), false, false);
-                split3(__uint_as_float(sw[0]), h[0][p], m[0][p], l[0][p]);
-                split3(__uint_as_float(sw[1]), h[1][p], m[1][p], l[1][p]);
-            }
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                th[t][q] = bf16_pair(h[t][0], h[t][1]);
-                tm[t][q] = bf16_pair(m[t][0], m[t][1]);
-                tl[t][q] = bf16_pair(l[t][0], l[t][1]);
-            }
+            for (int t = 0; t < 2; ++t)
+                split3_pair(__uint_as_float(s0[t]), __uint_as_float(s1[t]), th[t][q], tm[t][q], tl[t][q]);
         }
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -208,6 +198,65 @@ __device__ __forceinline__ float decode_split_wave(const float (&f)[kC], const L
     return halves_sum(part0, part1) + b1;
 }
 
+// The decoder from the tiles' operands on: register kk of tile t holds channel
+// 2 kk + half of query n (the channel map above, and that of the cell-by-cell
+// gather, cell_gather.hpp).
+template <bool POSINV>
+__device__ __forceinline__ float decode_split_tiles(const f32x16_t (&t)[2], const SplitLds* s, float b1, uint32_t lane,
+                                                    float px, float py, float pz) {
+    const uint32_t half = lane >> 5;
+    bf16x8 Bh[2][2], Bm[2][2], Bl[2][2];  // [tile][kb]
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            uint32_t ph[4], pm[4], pl[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                split3_pair(t[i][8 * kb + 2 * q], t[i][8 * kb + 2 * q + 1], ph[q], pm[q], pl[q]);
+            }
+            Bh[i][kb] = __builtin_bit_cast(bf16x8, make_uint4(ph[0], ph[1], ph[2], ph[3]));
+            Bm[i][kb] = __builtin_bit_cast(bf16x8, make_uint4(pm[0], pm[1], pm[2], pm[3]));
+            Bl[i][kb] = __builtin_bit_cast(bf16x8, make_uint4(pl[0], pl[1], pl[2], pl[3]));
+        }
+    }
+    // the position's columns: two FP32 MFMAs on (x, y) and (z, 0), half the cost of
+    // three FMAs per hidden unit and query
+    float bxy[2] = {0.0f, 0.0f}, bz[2] = {0.0f, 0.0f};
+    if (!POSINV) {
+        float q[2][3];
+        tile_coords(px, py, pz, q[0][0], q[0][1], q[0][2], q[1][0], q[1][1], q[1][2]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            bxy[i] = half ? q[i][1] : q[i][0];
+            bz[i] = half ? 0.0f : q[i][2];
+        }
+    }
+    float part[2] = {0.0f, 0.0f};
+#pragma unroll 1
+    for (int h = 0; h < 4; ++h) {
+        bf16x8 ah[2], am[2], al[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) split_afrag(s, h, kb, lane, ah[kb], am[kb], al[kb]);
+        // both tiles whether used or not: one block, so that a tile's ReLU runs
+        // beside the other's products
+        f32x16 c[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            c[i] = bias_tile(h, half, s);
+            if (!POSINV) {
+                const float* w = s->wxyz[32 * h + (int)(lane & 31u)];
+                c[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[half], bxy[i], c[i], 0, 0, 0);
+                c[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[2 + half], bz[i], c[i], 0, 0, 0);
+            }
+            c[i] = split_tile(ah, am, al, Bh[i], Bm[i], Bl[i], c[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) part[i] += layer2_partial(c[i], h, half, s, false, 0.0f, 0.0f, 0.0f);
+    }
+    return halves_sum(part[0], part[1]) + b1;
+}
+
 // decode_split_wave for a wave with few busy lanes (latency-bound): a used
 // tile's four hidden tiles are independent and issued together instead of
 // one after another.  Per output the same MFMA chain on the same operands and
@@ -230,17 +279,12 @@ __device__ __forceinline__ float decode_split_wave_few(const float (&f)[kC], con
             uint32_t th[4], tm[4], tl[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                __bf16 h[2], m[2], l[2];
-#pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    const int kk = 8 * kb + 2 * q + p;
-                    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(f[2 * kk]),
-                                                                     __float_as_uint(f[2 * kk + 1]), false, false);
-                    split3(__uint_as_float(sw[t]), h[p], m[p], l[p]);
-                }
-                th[q] = bf16_pair(h[0], h[1]);
-                tm[q] = bf16_pair(m[0], m[1]);
-                tl[q] = bf16_pair(l[0], l[1]);
+                const int kk = 8 * kb + 2 * q;
+                const auto s0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(f[2 * kk]),
+                                                                 __float_as_uint(f[2 * kk + 1]), false, false);
+                const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(f[2 * kk + 2]),
+                                                                 __float_as_uint(f[2 * kk + 3]), false, false);
+                split3_pair(__uint_as_float(s0[t]), __uint_as_float(s1[t]), th[q], tm[q], tl[q]);
             }
             Bh[kb] = __builtin_bit_cast(bf16x8, make_uint4(th[0], th[1], th[2], th[3]));
             Bm[kb] = __builtin_bit_cast(bf16x8, make_uint4(tm[0], tm[1], tm[2], tm[3]));
