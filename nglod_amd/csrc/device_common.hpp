@@ -270,6 +270,25 @@ __device__ __forceinline__ void tile_coords(float px, float py, float pz, float&
     qz1 = __uint_as_float(sz[1]);
 }
 
+__device__ __forceinline__ uint32_t lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+// The position's share of a 32x32 tile of pre-activations (hidden units 32 h ..):
+// wxyz[row] . xyz onto v as two FP32 MFMAs on (z, y) and (x, 0), the chain fma(x,
+// fma(y, fma(z, v))) bit for bit (exact products, k = 0 first).  On the vector ALU
+// the three FMAs per unit and query, and the rows' LDS reads, were a third of a
+// mixed evaluation: 1280x720, LOD 4: mixed frame 1.52 -> 1.24 ms (with both of a wave's tiles decoded in one
+// block, 1.37 before).
+// px, py, pz: the tile's queries (tile_coords); wxyz[row][3] is 0.
+template <typename LDS>
+__device__ __forceinline__ f32x16_t add_xyz(f32x16_t v, int h, uint32_t half, const LDS* s, float px, float py,
+                                            float pz) {
+    const float* w = s->wxyz[32 * h + (int)(lane_id() & 31u)];
+    v = __builtin_amdgcn_mfma_f32_32x32x2f32(w[2 - half], half ? py : pz, v, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(w[3 * half], half ? 0.0f : px, v, 0, 0, 0);
+}
+
 // A lane's query result from the two half-sums of its tile: part0 (tile 0)
 // on lanes 0..31 and part1 (tile 1) on lanes 32..63 hold one half each; the
 // swap brings the other half, and the sum is the same whichever operand
@@ -278,8 +297,6 @@ __device__ __forceinline__ float halves_sum(float part0, float part1) {
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(part0), __float_as_uint(part1), false, false);
     return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
 }
-
-__device__ __forceinline__ uint32_t lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 
 // Number of set bits of `mask` below this lane.
 // Position of the r-th (0-based) set bit of m; r < popcount(m).

@@ -19,7 +19,6 @@
 
 namespace nglod {
 
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 // Per-workgroup constants of the FP32 MFMA decoder, staged once in LDS
 // (18.5 KB): A fragments [h tile 0..3][channel-pair quad 0..3][lane] (4
@@ -74,27 +73,24 @@ __device__ __forceinline__ void stage_fp32_lds(const ModelArgs& m, int dec, Fp32
 template <typename LDS>
 __device__ __forceinline__ float layer2_tile(const f32x16_t& c, int h, uint32_t half, const LDS* s, bool xyz,
                                              float px, float py, float pz) {
+    f32x16_t v;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const float4 b = *reinterpret_cast<const float4*>(&s->b0[32 * h + 8 * g + 4 * (int)half]);
+        v[4 * g + 0] = c[4 * g + 0] + b.x;
+        v[4 * g + 1] = c[4 * g + 1] + b.y;
+        v[4 * g + 2] = c[4 * g + 2] + b.z;
+        v[4 * g + 3] = c[4 * g + 3] + b.w;
+    }
+    if (xyz) v = add_xyz(v, h, half, s, px, py, pz);
     float acc = 0.0f;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-        const int row0 = 32 * h + 8 * g + 4 * (int)half;
-        const float4 b = *reinterpret_cast<const float4*>(&s->b0[row0]);
-        const float4 w = *reinterpret_cast<const float4*>(&s->w1[row0]);
-        float v0 = c[4 * g + 0] + b.x, v1 = c[4 * g + 1] + b.y, v2 = c[4 * g + 2] + b.z, v3 = c[4 * g + 3] + b.w;
-        if (xyz) {
-            const float4 q0 = *reinterpret_cast<const float4*>(s->wxyz[row0 + 0]);
-            const float4 q1 = *reinterpret_cast<const float4*>(s->wxyz[row0 + 1]);
-            const float4 q2 = *reinterpret_cast<const float4*>(s->wxyz[row0 + 2]);
-            const float4 q3 = *reinterpret_cast<const float4*>(s->wxyz[row0 + 3]);
-            v0 = __builtin_fmaf(q0.x, px, __builtin_fmaf(q0.y, py, __builtin_fmaf(q0.z, pz, v0)));
-            v1 = __builtin_fmaf(q1.x, px, __builtin_fmaf(q1.y, py, __builtin_fmaf(q1.z, pz, v1)));
-            v2 = __builtin_fmaf(q2.x, px, __builtin_fmaf(q2.y, py, __builtin_fmaf(q2.z, pz, v2)));
-            v3 = __builtin_fmaf(q3.x, px, __builtin_fmaf(q3.y, py, __builtin_fmaf(q3.z, pz, v3)));
-        }
-        acc = __builtin_fmaf(w.x, fmaxf(v0, 0.0f), acc);
-        acc = __builtin_fmaf(w.y, fmaxf(v1, 0.0f), acc);
-        acc = __builtin_fmaf(w.z, fmaxf(v2, 0.0f), acc);
-        acc = __builtin_fmaf(w.w, fmaxf(v3, 0.0f), acc);
+        const float4 w = *reinterpret_cast<const float4*>(&s->w1[32 * h + 8 * g + 4 * (int)half]);
+        acc = __builtin_fmaf(w.x, fmaxf(v[4 * g + 0], 0.0f), acc);
+        acc = __builtin_fmaf(w.y, fmaxf(v[4 * g + 1], 0.0f), acc);
+        acc = __builtin_fmaf(w.z, fmaxf(v[4 * g + 2], 0.0f), acc);
+        acc = __builtin_fmaf(w.w, fmaxf(v[4 * g + 3], 0.0f), acc);
     }
     return acc;
 }

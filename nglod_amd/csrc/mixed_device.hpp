@@ -154,28 +154,17 @@ __device__ __forceinline__ float relu_bits(float v) {
 // layer's output with b0 already in it): sum of
 // w1[row] * relu(C + wxyz[row] . xyz) over this lane's 16 rows.
 template <typename LDS>
-__device__ __forceinline__ float layer2_partial(const f32x16& c, int h, uint32_t half, const LDS* s, bool xyz,
-                                                float px, float py, float pz) {
+__device__ __forceinline__ float layer2_partial(f32x16 c, int h, uint32_t half, const LDS* s, bool xyz, float px,
+                                                float py, float pz) {
+    if (xyz) c = add_xyz(c, h, half, s, px, py, pz);
     float acc = 0.0f;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-        const int row0 = 32 * h + 8 * g + 4 * (int)half;
-        const float4 w = *reinterpret_cast<const float4*>(&s->w1[row0]);
-        float v0 = c[4 * g + 0], v1 = c[4 * g + 1], v2 = c[4 * g + 2], v3 = c[4 * g + 3];
-        if (xyz) {
-            const float4 q0 = *reinterpret_cast<const float4*>(s->wxyz[row0 + 0]);
-            const float4 q1 = *reinterpret_cast<const float4*>(s->wxyz[row0 + 1]);
-            const float4 q2 = *reinterpret_cast<const float4*>(s->wxyz[row0 + 2]);
-            const float4 q3 = *reinterpret_cast<const float4*>(s->wxyz[row0 + 3]);
-            v0 = __builtin_fmaf(q0.x, px, __builtin_fmaf(q0.y, py, __builtin_fmaf(q0.z, pz, v0)));
-            v1 = __builtin_fmaf(q1.x, px, __builtin_fmaf(q1.y, py, __builtin_fmaf(q1.z, pz, v1)));
-            v2 = __builtin_fmaf(q2.x, px, __builtin_fmaf(q2.y, py, __builtin_fmaf(q2.z, pz, v2)));
-            v3 = __builtin_fmaf(q3.x, px, __builtin_fmaf(q3.y, py, __builtin_fmaf(q3.z, pz, v3)));
-        }
-        acc = __builtin_fmaf(w.x, relu_bits(v0), acc);
-        acc = __builtin_fmaf(w.y, relu_bits(v1), acc);
-        acc = __builtin_fmaf(w.z, relu_bits(v2), acc);
-        acc = __builtin_fmaf(w.w, relu_bits(v3), acc);
+        const float4 w = *reinterpret_cast<const float4*>(&s->w1[32 * h + 8 * g + 4 * (int)half]);
+        acc = __builtin_fmaf(w.x, relu_bits(c[4 * g + 0]), acc);
+        acc = __builtin_fmaf(w.y, relu_bits(c[4 * g + 1]), acc);
+        acc = __builtin_fmaf(w.z, relu_bits(c[4 * g + 2]), acc);
+        acc = __builtin_fmaf(w.w, relu_bits(c[4 * g + 3]), acc);
     }
     return acc;
 }
@@ -190,8 +179,6 @@ __device__ __forceinline__ float layer2_partial(const f32x16& c, int h, uint32_t
 template <bool POSINV>
 __device__ __forceinline__ float decode_mixed_wave(const __half2 (&acc)[kC / 2], const MixedLds* s, float b1,
                                                    uint32_t lane, bool active, float px, float py, float pz) {
-    const uint64_t am = __ballot(active);
-    const bool use0 = (uint32_t)am != 0u, use1 = (uint32_t)(am >> 32) != 0u;
     const uint32_t half = lane >> 5;
     // own channels 16kb + 0..7 (Y) and 16kb + 8..15 (X) as bf16; one
     // v_permlane32_swap per word gives tile 0 (own Y | X of lane l-32) and
@@ -218,16 +205,12 @@ __device__ __forceinline__ float decode_mixed_wave(const __half2 (&acc)[kC / 2],
     for (int h = 0; h < 4; ++h) {
         const bf16x8 a0 = __builtin_bit_cast(bf16x8, s->wfrag[(h * 2 + 0) * 64 + lane]);
         const bf16x8 a1 = __builtin_bit_cast(bf16x8, s->wfrag[(h * 2 + 1) * 64 + lane]);
-        if (use0) {
-            f32x16 c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, B0[0], bias_tile(h, half, s), 0, 0, 0);
-            c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, B0[1], c0, 0, 0, 0);
-            part0 += layer2_partial(c0, h, half, s, !POSINV, qx0, qy0, qz0);
-        }
-        if (use1) {
-            f32x16 c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, B1[0], bias_tile(h, half, s), 0, 0, 0);
-            c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, B1[1], c1, 0, 0, 0);
-            part1 += layer2_partial(c1, h, half, s, !POSINV, qx1, qy1, qz1);
-        }
+        f32x16 c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, B0[0], bias_tile(h, half, s), 0, 0, 0);
+        f32x16 c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, B1[0], bias_tile(h, half, s), 0, 0, 0);
+        c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, B0[1], c0, 0, 0, 0);
+        c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, B1[1], c1, 0, 0, 0);
+        part0 += layer2_partial(c0, h, half, s, !POSINV, qx0, qy0, qz0);
+        part1 += layer2_partial(c1, h, half, s, !POSINV, qx1, qy1, qz1);
     }
     return halves_sum(part0, part1) + b1;
 }

@@ -152,8 +152,6 @@ __device__ __forceinline__ f32x16 split_tile(const bf16x8 (&ah)[2], const bf16x8
 template <bool POSINV, typename LDS>
 __device__ __forceinline__ float decode_split_wave(const float (&f)[kC], const LDS* s, float b1, uint32_t lane,
                                                    bool active, float px, float py, float pz) {
-    const uint64_t am_ = __ballot(active);
-    const bool use0 = (uint32_t)am_ != 0u, use1 = (uint32_t)(am_ >> 32) != 0u;
     const uint32_t half = lane >> 5;
     // [tile][kb] B operands of the three parts
     bf16x8 Bh[2][2], Bm[2][2], Bl[2][2];
@@ -186,14 +184,10 @@ __device__ __forceinline__ float decode_split_wave(const float (&f)[kC], const L
         bf16x8 ah[2], am[2], al[2];
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) split_afrag(s, h, kb, lane, ah[kb], am[kb], al[kb]);
-        if (use0) {
-            const f32x16 c = split_tile(ah, am, al, Bh[0], Bm[0], Bl[0], bias_tile(h, half, s));
-            part0 += layer2_partial(c, h, half, s, !POSINV, qx0, qy0, qz0);
-        }
-        if (use1) {
-            const f32x16 c = split_tile(ah, am, al, Bh[1], Bm[1], Bl[1], bias_tile(h, half, s));
-            part1 += layer2_partial(c, h, half, s, !POSINV, qx1, qy1, qz1);
-        }
+        const f32x16 c0 = split_tile(ah, am, al, Bh[0], Bm[0], Bl[0], bias_tile(h, half, s));
+        const f32x16 c1 = split_tile(ah, am, al, Bh[1], Bm[1], Bl[1], bias_tile(h, half, s));
+        part0 += layer2_partial(c0, h, half, s, !POSINV, qx0, qy0, qz0);
+        part1 += layer2_partial(c1, h, half, s, !POSINV, qx1, qy1, qz1);
     }
     return halves_sum(part0, part1) + b1;
 }
@@ -220,18 +214,8 @@ __device__ __forceinline__ float decode_split_tiles(const f32x16_t (&t)[2], cons
             Bl[i][kb] = __builtin_bit_cast(bf16x8, make_uint4(pl[0], pl[1], pl[2], pl[3]));
         }
     }
-    // the position's columns: two FP32 MFMAs on (x, y) and (z, 0), half the cost of
-    // three FMAs per hidden unit and query
-    float bxy[2] = {0.0f, 0.0f}, bz[2] = {0.0f, 0.0f};
-    if (!POSINV) {
-        float q[2][3];
-        tile_coords(px, py, pz, q[0][0], q[0][1], q[0][2], q[1][0], q[1][1], q[1][2]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            bxy[i] = half ? q[i][1] : q[i][0];
-            bz[i] = half ? 0.0f : q[i][2];
-        }
-    }
+    float q[2][3];
+    tile_coords(px, py, pz, q[0][0], q[0][1], q[0][2], q[1][0], q[1][1], q[1][2]);
     float part[2] = {0.0f, 0.0f};
 #pragma unroll 1
     for (int h = 0; h < 4; ++h) {
@@ -242,17 +226,10 @@ __device__ __forceinline__ float decode_split_tiles(const f32x16_t (&t)[2], cons
         // beside the other's products
         f32x16 c[2];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            c[i] = bias_tile(h, half, s);
-            if (!POSINV) {
-                const float* w = s->wxyz[32 * h + (int)(lane & 31u)];
-                c[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[half], bxy[i], c[i], 0, 0, 0);
-                c[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[2 + half], bz[i], c[i], 0, 0, 0);
-            }
-            c[i] = split_tile(ah, am, al, Bh[i], Bm[i], Bl[i], c[i]);
-        }
+        for (int i = 0; i < 2; ++i) c[i] = split_tile(ah, am, al, Bh[i], Bm[i], Bl[i], bias_tile(h, half, s));
 #pragma unroll
-        for (int i = 0; i < 2; ++i) part[i] += layer2_partial(c[i], h, half, s, false, 0.0f, 0.0f, 0.0f);
+        for (int i = 0; i < 2; ++i)
+            part[i] += layer2_partial(c[i], h, half, s, !POSINV, q[i][0], q[i][1], q[i][2]);
     }
     return halves_sum(part[0], part[1]) + b1;
 }
