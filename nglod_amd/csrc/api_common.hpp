@@ -140,7 +140,7 @@ enum : int { kPassMarch = 0, kPassFp32 = 1, kPassUnused = 2, kPassOther = 3, kPa
 struct TraceArgs;
 // Mixed-precision launchers (mixed.hip).
 // Batch queries; order (optional) is the evaluation order, a permutation of [0, n).
-int launch_sdf_fp32(const ModelArgs& m, int lod, int dec, const float* x, int64_t n, float* out, hipStream_t s);
+int launch_sdf_group_fp32(const ModelArgs& m, int lod, int dec, const float* x, int64_t n, float* out, hipStream_t s);
 int launch_sdf_ordered_fp32(const ModelArgs& m, int lod, int dec, const float* x, int64_t n, float* out,
                             const uint32_t* order, hipStream_t s);
 int launch_cell_order(const float* x, int64_t n, int r, void* workspace, size_t workspace_bytes,

@@ -6,7 +6,6 @@
 //   nglod_normals_fd    central-difference normals     (diffutils.py:61-70)
 //   nglod_trace_dense   persistent sphere tracer       (SphereTracer.py:41-132)
 #include <stdio.h>
-#include <stdlib.h>
 
 #include <mutex>
 
@@ -82,32 +81,6 @@ __global__ __launch_bounds__(256) void grid_sample_kernel(const float* __restric
     float4* o4 = reinterpret_cast<float4*>(out + i * kC);
 #pragma unroll
     for (int v = 0; v < kC / 4; ++v) o4[v] = make_float4(f[4 * v], f[4 * v + 1], f[4 * v + 2], f[4 * v + 3]);
-}
-
-// Batch query in input order.
-template <bool POSINV>
-__global__ __launch_bounds__(256) void sdf_fp32_kernel(ModelArgs m, int lod, int dec, const float* __restrict__ x,
-                                                       int64_t n, float* __restrict__ out) {
-    __shared__ Fp32Lds lds;
-    stage_fp32_lds(m, dec, &lds);
-    __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = i < n;
-    if (__ballot(valid) == 0) return;  // whole wave past the end (no barrier follows)
-    const float px = valid ? x[3 * i] : 0.0f;
-    const float py = valid ? x[3 * i + 1] : 0.0f;
-    const float pz = valid ? x[3 * i + 2] : 0.0f;
-    const float d = sdf_fp32_wave<POSINV>(m, lod, &lds, m.b1[dec][0], lane_id(), valid, px, py, pz);
-    if (valid) out[i] = d;
-}
-
-int launch_sdf_fp32(const ModelArgs& m, int lod, int dec, const float* x, int64_t n, float* out, hipStream_t s) {
-    const int64_t blocks = (n + 255) / 256;
-    if (m.pos_inv)
-        hipLaunchKernelGGL(sdf_fp32_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, s, m, lod, dec, x, n, out);
-    else
-        hipLaunchKernelGGL(sdf_fp32_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, s, m, lod, dec, x, n, out);
-    return check_launch("sdf_fp32_kernel");
 }
 
 // Every level's prediction (the training forward): the running FP32 feature
@@ -219,7 +192,7 @@ int nglod_sdf_fwd(const nglod_model_t* model, const float* x, int64_t n, int32_t
     if (!x || !out) return fail(NGLOD_ERR_ARG, "NULL pointer");
     const int dec = decoder_of(model, lod);
     if (form == NGLOD_MIXED) return launch_sdf_mixed(m, 0, dec, x, n, out, nullptr, (hipStream_t)stream);
-    return launch_sdf_fp32(m, lod, dec, x, n, out, (hipStream_t)stream);
+    return launch_sdf_group_fp32(m, lod, dec, x, n, out, (hipStream_t)stream);
 }
 
 int nglod_sdf_fwd_all(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, float* out, void* stream) {
@@ -339,7 +312,6 @@ static int trace_dense_run(const nglod_model_t* model, const ModelArgs& m, const
     // normals pass measured 3-4% slower for the FP32 form.
     a.defer_normals = 0;
     a.solo_lanes = solo_lanes_setting();
-    a.coarse = coarse_plan(m, a.lod);
     a.replay_steps = params->refine_steps < 1 ? 1 : params->refine_steps;
     a.near_dist = (float)params->near_dist;
     a.evals = (unsigned long long*)evals_out;

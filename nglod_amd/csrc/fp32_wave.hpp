@@ -14,7 +14,6 @@
 // both tiles' B operands.
 #pragma once
 
-#include "coarse_lds.hpp"
 #include "device_common.hpp"
 
 namespace nglod {
@@ -95,14 +94,11 @@ __device__ __forceinline__ float layer2_tile(const f32x16_t& c, int h, uint32_t 
     return acc;
 }
 
-// SDF of the 64 lanes' query points in FP32.  Every lane of the wave must
-// call this (no divergent branch around it): the MFMAs and lane swaps are
-// wave-wide.  Lanes without a query pass active = false: they load nothing,
-// and a 32-query tile with no active lane skips its MFMAs.  Each output
-// column depends only on its own query, so a lane's result is the same
-// whatever the other lanes hold.
-// The decoder on the 64 lanes' feature vectors f (zero on inactive lanes).
-// Wave-wide, as sdf_fp32_wave.
+// The decoder on the 64 lanes' feature vectors f (zero on inactive lanes).  Every
+// lane of the wave must call this (no divergent branch around it): the MFMAs and
+// lane swaps are wave-wide.  A 32-query tile with no active lane skips its MFMAs.
+// Each output column depends only on its own query, so a lane's result is the
+// same whatever the other lanes hold.
 template <bool POSINV>
 __device__ __forceinline__ float decode_fp32_wave(const float (&f)[kC], const Fp32Lds* s, float b1, uint32_t lane,
                                                   bool active, float px, float py, float pz) {
@@ -171,23 +167,6 @@ __device__ __forceinline__ void stage_solo_levels(const ModelArgs& m, SoloLevels
             lv->res[l] = m.res[l];
         }
     }
-}
-
-template <bool POSINV>
-__device__ __forceinline__ float sdf_fp32_wave(const ModelArgs& m, int lod, const Fp32Lds* s, float b1,
-                                               uint32_t lane, bool active, float px, float py, float pz,
-                                               CoarsePlan cp = CoarsePlan{0, 0}, const CoarseLds32* cs = nullptr) {
-    // cleared once for both cases (zero on inactive lanes)
-    float f[kC];
-#pragma unroll
-    for (int c = 0; c < kC; ++c) f[c] = 0.0f;
-    if (active) {
-        if (cp.levels > 0)
-            gather_fp32_coarse(m, lod, cp, cs, px, py, pz, f);
-        else
-            gather_fp32_add(m, lod, px, py, pz, f);
-    }
-    return decode_fp32_wave<POSINV>(f, s, b1, lane, active, px, py, pz);
 }
 
 }  // namespace nglod

@@ -10,7 +10,8 @@
 //     registers) by the features of all 32 queries and takes its units' share of the
 //     second layer; the four shares are added in the order of h.
 //
-// The sums have the order of sdf_fp32_wave's, so the bits are the same.  A grid of
+// The sums have the order of the wave-wide decoder's (fp32_wave.hpp), so the bits
+// are the same.  A grid of
 // 5^3 corners (level 0) is kept in LDS: one fifth of a 5-level gather leaves the
 // L1 (1280x720: 3.82 -> 3.43 ms); with 34 KB of LDS a CU holds four blocks.
 // Interpolating the cells that neighbouring rays share on the matrix cores (as
@@ -35,10 +36,11 @@ struct alignas(16) GroupDecoder {
     float wxyz[kH][4];
 };
 
+template <bool COARSE>
 struct GroupLds {
     float4 w[NGLOD_MAX_LODS][kGroup][2];  // corner weights, corner = 4 z + 2 y + x
     uint32_t base[NGLOD_MAX_LODS][kGroup];
-    float4 coarse[125 * (kC / 4)];  // level 0's grid when it has at most 5^3 corners
+    float4 coarse[COARSE ? 125 * (kC / 4) : 1];  // level 0's grid when it has at most 5^3 corners
     GroupDecoder dec;
 };
 
@@ -65,8 +67,10 @@ __device__ __forceinline__ GroupWeights stage_group_decoder(const float* W0, int
     return g;
 }
 
-__device__ __forceinline__ GroupWeights stage_group(const ModelArgs& m, int dec, GroupLds* s) {
-    if (m.res[0] <= 4) {
+// COARSE: with level 0 in LDS (for blocks of many trips).
+template <bool COARSE>
+__device__ __forceinline__ GroupWeights stage_group(const ModelArgs& m, int dec, GroupLds<COARSE>* s) {
+    if (COARSE && m.res[0] <= 4) {
         const int S = m.res[0] + 1;
         const float4* g4 = reinterpret_cast<const float4*>(m.grid[0]);
         for (int j = threadIdx.x; j < S * S * S * (kC / 4); j += kGroupThreads) s->coarse[j] = g4[j];
@@ -130,8 +134,8 @@ __device__ __forceinline__ void group_corners(const float4 (&g)[8], const float4
 
 // Every thread of the block, with the position of query lane % 32 (the same in
 // all four waves; any position for queries whose result is not used).
-template <bool POSINV>
-__device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds* s, const GroupWeights& gw, float b1,
+template <bool POSINV, bool COARSE>
+__device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds<COARSE>* s, const GroupWeights& gw, float b1,
                                            float px, float py, float pz) {
     const uint32_t lane = lane_id(), n = lane & 31u, half = lane >> 5;
     {
@@ -154,7 +158,7 @@ __device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds
         float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         float4 g[8];
         int l = 0;
-        if (m.res[0] <= 4) {
+        if (COARSE && m.res[0] <= 4) {
             const int S = m.res[0] + 1;
             const float4* b = s->coarse + s->base[0][ray] * (kC / 4) + q;
 #pragma unroll

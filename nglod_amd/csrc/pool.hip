@@ -136,7 +136,6 @@ int nglod_trace_pool(const nglod_model_t* models, const void* model_table, int32
     a.return_dist = 0.0f;
     a.defer_normals = 0;  // the pooled passes set their own
     a.solo_lanes = solo_lanes_setting();
-    a.coarse = CoarsePlan{0, 0};
     a.replay_steps = params->refine_steps;
     a.near_dist = (float)params->near_dist;
     a.evals = (unsigned long long*)evals_out;

@@ -4,7 +4,6 @@
 
 #include <stdlib.h>
 
-#include "coarse_lds.hpp"
 #include "device_common.hpp"
 #include "fp32_wave.hpp"
 
@@ -34,10 +33,6 @@ __device__ __forceinline__ void normalize_grad(float g0, float g1, float g2, flo
 // (workgroups are dispatched to XCDs round-robin, so blockIdx % 8 picks the
 // XCD-local range and its L2 sees one band of the image); a wave that drains
 // its own range moves on to the next ones.
-// Threads per block of the FP32 ambient occlusion: one block of 8 waves per CU (the
-// 128 KB of decoder and coarse-level tables in LDS leave room for one), sharing
-// those tables.
-constexpr int kMarchBlock = 512;
 constexpr int kQueues = 8;  // a multiple of 8 (one share per XCD)
 static_assert(kQueues % 8 == 0 && kQueues <= 256, "kQueues: a multiple of 8, at most 256");
 // Stride (in words) of the single-request traces' claim counters: one
@@ -76,7 +71,6 @@ struct TraceArgs {
     uint32_t* queue;
     unsigned long long* evals;  // [0] FP32-form evaluations, [1] mixed-form evaluations
     int32_t* ray_steps;
-    CoarsePlan coarse; // leading levels the march kernels stage in LDS
     // Mixed form.  Records passed between the passes are indexed by ray
     // (record[ray], flag[ray] = 1 when written): no shared append counter, and
     // a pass that reads them claims consecutive ray ids.
@@ -315,30 +309,6 @@ struct RayState {
         }
     }
 };
-
-// Every lane claims the next id in [0, total) whose flag is set (flag2, when
-// not NULL: or whose flag2 is set), from one counter (one atomic per wave per round, as many ids as lanes still
-// looking); -1 once the ids run out (`drained`, wave-uniform).
-__device__ __forceinline__ int64_t claim_hits(uint32_t* counter, const uint8_t* flag, uint32_t total, uint32_t lane,
-                                              bool& drained, const uint8_t* flag2 = nullptr) {
-    int64_t id = -1;
-    for (;;) {
-        const bool want = id < 0 && !drained;
-        const uint64_t mask = __ballot(want);
-        if (mask == 0) break;
-        const int cnt = __popcll(mask);
-        const int leader = __ffsll((unsigned long long)mask) - 1;
-        uint32_t base = 0;
-        if ((int)lane == leader) base = atomicAdd(counter, (uint32_t)cnt);
-        base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);
-        if (want) {
-            const uint32_t idx = base + mask_rank(mask);
-            if (idx < total && (flag[idx] || (flag2 && flag2[idx]))) id = idx;
-        }
-        if (base + (uint32_t)cnt >= total) drained = true;
-    }
-    return id;
-}
 
 // Hands ray ids to the lanes of one wave.  The frame is split into kQueues
 // contiguous ranges with one claim counter each (counters[0..kQueues-1]);

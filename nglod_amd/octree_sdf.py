@@ -211,14 +211,15 @@ class OctreeSDF(nn.Module):
     def _ordered(self, n, lod, form):
         """Whether a batch of n points is evaluated in spatial order
         (nglod_sdf_fwd_ordered; the results are identical either way).  On
-        uniform points, both ways in us: FP32 at LOD 4 52 / 83 with 2^16 points,
-        167 / 131 with 2^18, 2464 / 673 with 2^22, at LOD 0 51 / 58 with 2^18 and
-        177 / 117 with 10^6.  The mixed form gathers one FP16 grid, which the L2s
-        hold below LOD 4 (194 / 250 at LOD 3, 347 / 283 at LOD 4 with 2^22)."""
+        uniform points, both ways in us: FP32 at LOD 4 168 / 146 with 2^19 points,
+        236 / 266 with 10^6, 667 / 1060 with 2^22; at LOD 2 157 / 151 with 10^6, 456 /
+        602 with 2^22; at LOD 0 114 / 101 and 353 / 388.  The mixed form gathers one
+        FP16 grid, which the L2s hold below LOD 4 (194 / 250 at LOD 3, 347 / 283 at
+        LOD 4 with 2^22)."""
         r = self.features[lod].fsize
         if form == _lib.MIXED:
             return n >= 1 << 21 and (r + 1) ** 3 * 64 > 1 << 22
-        return n >= (1 << 18 if r >= 16 else 1 << 19)
+        return n >= (3 << 18 if r >= 32 else 3 << 19)
 
     def sdf_hip(self, x, lod, form=_lib.FP32, ordered=None):
         """ordered: None picks by batch size, LOD and form; True / False forces
