@@ -226,12 +226,31 @@ def check(rc, what):
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    """A tensor's address as a c_void_p argument takes it (None: NULL)."""
+    return t.data_ptr() if t is not None else None
 
 
 def stream_of(t):
     """Raw hipStream_t of torch's current stream on t's device."""
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return torch.cuda.current_stream(t.device).cuda_stream
+
+
+def parameter_list(module):
+    """list(module.parameters()): the same order, without the names that
+    traversal builds (a third of its time)."""
+    out, seen = [], set()
+
+    def walk(m):
+        for p in m._parameters.values():
+            if p is not None and id(p) not in seen:
+                seen.add(id(p))
+                out.append(p)
+        for c in m._modules.values():
+            if c is not None:
+                walk(c)
+
+    walk(module)
+    return out
 
 
 def require_gpu(*tensors):

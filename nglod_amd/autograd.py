@@ -10,20 +10,16 @@ from torch.autograd.function import once_differentiable
 from . import _lib
 
 
-def _param_slots(net):
-    """(kind, index, name) of every parameter in net.parameters() order."""
-    slots = []
-    for name, _ in net.named_parameters():
-        parts = name.split(".")
-        if parts[0] == "features":
-            slots.append(("grid", int(parts[1]), None))
-        elif parts[0] == "louts":
-            key = {("0", "weight"): "w0", ("0", "bias"): "b0", ("2", "weight"): "w1", ("2", "bias"): "b1"}[
-                (parts[2], parts[3])]
-            slots.append((key, int(parts[1]), None))
-        else:
-            slots.append((None, -1, name))
-    return slots
+def _param_slots(net, params):
+    """(kind, index) of each parameter; (None, -1) for one the kernels do not read."""
+    slots = {id(f.fm): ("grid", i) for i, f in enumerate(net.features)}
+    for i, l in enumerate(net.louts):
+        first, _, last = l
+        slots[id(first.weight)] = ("w0", i)
+        slots[id(first.bias)] = ("b0", i)
+        slots[id(last.weight)] = ("w1", i)
+        slots[id(last.bias)] = ("b1", i)
+    return [slots.get(id(p), (None, -1)) for p in params]
 
 
 # The forward of every level keeps its features for the backward (164 bytes per
@@ -31,8 +27,8 @@ def _param_slots(net):
 SAVE_LIMIT = 4 << 30
 
 
-def _versions(net):
-    return tuple((p.data_ptr(), p._version) for p in net.parameters())
+def _versions(params):
+    return [(p.data_ptr(), p._version) for p in params]
 
 
 class _SdfFunction(torch.autograd.Function):
@@ -55,7 +51,7 @@ class _SdfFunction(torch.autograd.Function):
                 ws = torch.empty(lib.nglod_sdf_fwd_save_workspace_size(n), device=x.device, dtype=torch.uint8)
                 _lib.check(lib.nglod_sdf_fwd_save(m, _lib.ptr(xf), n, lod, _lib.ptr(out), _lib.ptr(saved), nbytes,
                                                   _lib.ptr(ws), ws.numel(), _lib.stream_of(x)), "nglod_sdf_fwd_save")
-                ctx.versions = _versions(net)
+                ctx.versions = _versions(params)
                 ctx.save_for_backward(xf, saved)
                 return out
         ctx.save_for_backward(xf)
@@ -102,8 +98,9 @@ class _SdfFunction(torch.autograd.Function):
                 getattr(G, key)[d] = t.data_ptr()
         m = net.descriptor(_lib.FP32)
         lib = _lib.load()
+        params = _lib.parameter_list(net)
         # features of other weights are not the features of these: computed again
-        if saved and ctx.versions == _versions(net):
+        if saved and ctx.versions == _versions(params):
             nbytes = lib.nglod_sdf_bwd_saved_workspace_size(m, n, L)
             ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=dev)
             _lib.check(lib.nglod_sdf_bwd_saved(m, _lib.ptr(x), n, L, _lib.ptr(g), mask, G, _lib.ptr(saved[0]),
@@ -115,7 +112,7 @@ class _SdfFunction(torch.autograd.Function):
             _lib.check(lib.nglod_sdf_bwd(m, _lib.ptr(x), n, L, _lib.ptr(g), mask, G, _lib.ptr(ws), ws.numel(),
                                          _lib.stream_of(x)), "nglod_sdf_bwd")
         grads = []
-        for kind, idx, _ in _param_slots(net):
+        for kind, idx in _param_slots(net, params):
             if kind == "grid":
                 grads.append(out.get(("grid", idx)))
             elif kind is not None and idx in used_dec:
@@ -125,9 +122,11 @@ class _SdfFunction(torch.autograd.Function):
         return (None, grad_x, None, None, *grads)
 
 
-def sdf_with_grad(net, x, lod, all_levels, stacked=False):
-    """stacked: the levels' predictions as one [lod + 1, n, 1] tensor."""
-    params = list(net.parameters())
+def sdf_with_grad(net, x, lod, all_levels, stacked=False, params=None):
+    """stacked: the levels' predictions as one [lod + 1, n, 1] tensor; params:
+    net's parameters, if the caller has them."""
+    if params is None:
+        params = _lib.parameter_list(net)
     out = _SdfFunction.apply(net, x, lod, all_levels, *params)
     if all_levels and not stacked:
         return [out[i] for i in range(out.shape[0])]

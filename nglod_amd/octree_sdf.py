@@ -149,30 +149,36 @@ class OctreeSDF(nn.Module):
     def _needs_grad(self, x):
         if not torch.is_grad_enabled():
             return False
-        return x.requires_grad or any(p.requires_grad for p in self.parameters())
+        return x.requires_grad or any(p.requires_grad for p in _lib.parameter_list(self))
 
     def decoder_index(self, lod):
         return 0 if self.num_decoder == 1 else lod
 
     def descriptor(self, form=_lib.FP32):
         """nglod_model_t for the current parameters (device pointers)."""
-        m = _lib.NglodModel()
-        m.num_lods = self.num_lods
-        m.feature_dim = self.fdim
-        m.hidden_dim = self.hidden_dim
-        m.pos_invariant = 1 if self.pos_invariant else 0
-        m.num_decoders = self.num_decoder
         keep = []
+
+        def address(t, grid):
+            # parameters that are laid out as the kernels read them are read in place
+            if grid:
+                c = t if t.is_contiguous(memory_format=torch.channels_last_3d) else corner_major(t.detach())
+            else:
+                c = t if t.is_contiguous() else t.detach().contiguous()
+            keep.append(c)
+            return c.data_ptr()
+
+        m = _lib.NglodModel(self.num_lods, self.fdim, self.hidden_dim, 1 if self.pos_invariant else 0,
+                            self.num_decoder)
+        res, grid, w0, b0, w1, b1 = m.res, m.grid, m.w0, m.b0, m.w1, m.b1
         for i, f in enumerate(self.features):
-            g = corner_major(f.fm.detach())
-            keep.append(g)
-            m.res[i] = f.fsize
-            m.grid[i] = g.data_ptr()
+            res[i] = f.fsize
+            grid[i] = address(f.fm, True)
         for i, l in enumerate(self.louts):
-            for name, t in (("w0", l[0].weight), ("b0", l[0].bias), ("w1", l[2].weight), ("b1", l[2].bias)):
-                t = t.detach().contiguous()
-                keep.append(t)
-                getattr(m, name)[i] = t.data_ptr()
+            first, _, last = l
+            w0[i] = address(first.weight, False)
+            b0[i] = address(first.bias, False)
+            w1[i] = address(last.weight, False)
+            b1[i] = address(last.bias, False)
         if form == _lib.MIXED:
             grids_c, grids_h, w0s = self.mixed_buffers()
             for i, (gc, gh) in enumerate(zip(grids_c, grids_h)):
@@ -190,7 +196,7 @@ class OctreeSDF(nn.Module):
         that level and every coarser one) in FP32 and its FP16 rounding, and
         the packed BF16 first-layer weights; rebuilt when any parameter changed
         since the last call."""
-        key = tuple((p.data_ptr(), p._version) for p in self.parameters())
+        key = tuple((p.data_ptr(), p._version) for p in _lib.parameter_list(self))
         if self._mixed is not None and self._mixed[0] == key:
             return self._mixed[1], self._mixed[2], self._mixed[3]
         dev = self.features[0].fm.device

@@ -15,7 +15,11 @@ def _dense_like(p, *others):
     """Whether p is laid out without gaps and the others exactly as p."""
     if not (p.is_contiguous() or (p.dim() == 5 and p.is_contiguous(memory_format=torch.channels_last_3d))):
         return False
-    return all(t.stride() == p.stride() and t.shape == p.shape for t in others)
+    shape, stride = p.shape, p.stride()
+    for t in others:
+        if t.shape != shape or t.stride() != stride:
+            return False
+    return True
 
 
 class Adam(torch.optim.Adam):
@@ -37,46 +41,53 @@ class Adam(torch.optim.Adam):
                                            float(beta2), float(group["eps"]), float(group["lr"]), step,
                                            _lib.stream_of(params[0])), "nglod_adam_step")
             # written behind autograd's back: what is keyed by a version must see it
-            torch.autograd.graph.increment_version(params)
+            torch.autograd.graph.increment_version(list(params))
         return None
 
     def _plans(self):
         """[(group, params, grads, exp_avgs, exp_avg_sqs, step)], the states
         created and their steps counted; None where torch's step must run
         (and nothing has been touched)."""
+        current = torch.cuda.current_device() if torch.cuda.is_available() else -1
+        fresh = False
+        found = []
         for group in self.param_groups:
             if (group["amsgrad"] or group["weight_decay"] != 0 or group["maximize"] or group["capturable"]
                     or group["differentiable"] or group.get("fused") or group["foreach"] is False
                     or isinstance(group["lr"], torch.Tensor)
                     or any(isinstance(b, torch.Tensor) for b in group["betas"])):
                 return None
+            rows = []
             for p in group["params"]:
                 g = p.grad
                 if g is None:
                     continue
-                if (g.is_sparse or p.dtype != torch.float32 or g.dtype != torch.float32 or not p.is_cuda
-                        or type(p) is not torch.nn.Parameter or p.device != g.device
-                        or p.device.index != torch.cuda.current_device() or not _dense_like(p, g)):
+                if (type(p) is not torch.nn.Parameter or not p.is_cuda or g.layout != torch.strided
+                        or p.dtype != torch.float32 or g.dtype != torch.float32 or p.get_device() != current
+                        or g.get_device() != current or not _dense_like(p, g)):
                     return None
                 s = self.state.get(p)
-                if s and (not _dense_like(p, s["exp_avg"], s["exp_avg_sq"]) or s["step"].is_cuda
-                          or s["exp_avg"].dtype != torch.float32 or s["exp_avg_sq"].dtype != torch.float32
-                          or s["exp_avg"].device != p.device or s["exp_avg_sq"].device != p.device):
+                if not s:
+                    fresh = True
+                    continue
+                avg, sq, step = s["exp_avg"], s["exp_avg_sq"], s["step"]
+                if (avg.dtype != torch.float32 or sq.dtype != torch.float32 or avg.get_device() != current
+                        or sq.get_device() != current or step.is_cuda or not _dense_like(p, avg, sq)):
                     return None
+                rows.append((p, g, avg, sq, step))
+            found.append((group, rows))
         if torch.cuda.is_current_stream_capturing():
             return None  # torch's step says what capture needs
         plans = []
         with torch.no_grad():
-            for group in self.param_groups:
-                params, grads, avgs, sqs, maxs, steps = [], [], [], [], [], []
-                self._init_group(group, params, grads, avgs, sqs, maxs, steps)
-                if not params:
-                    continue
-                torch._foreach_add_(steps, 1)
+            for group, rows in found:
+                if fresh:
+                    params, grads, avgs, sqs, maxs, steps = [], [], [], [], [], []
+                    self._init_group(group, params, grads, avgs, sqs, maxs, steps)
+                    rows = list(zip(params, grads, avgs, sqs, steps))
                 by_step = {}
-                for i, t in enumerate(steps):
-                    by_step.setdefault(int(t.item()), []).append(i)
+                for row in rows:
+                    by_step.setdefault(int(row[4].add_(1).item()), []).append(row[:4])
                 for step, at in by_step.items():
-                    pick = lambda v: [v[i] for i in at]
-                    plans.append((group, pick(params), pick(grads), pick(avgs), pick(sqs), step))
+                    plans.append((group, *zip(*at), step))
         return plans

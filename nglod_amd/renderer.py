@@ -39,6 +39,18 @@ def normalized_grid(width, height, device="cuda", jitter=False, generator=None):
     return torch.stack((xs[:, None].expand(width, height), ys[None, :].expand(width, height)), dim=-1)
 
 
+def _on_device(rows, device):
+    """FP32 tensors of rows of numbers.  To the GPU by one asynchronous copy from
+    pinned memory: a copy from pageable memory waits for the stream, that is for
+    the frame before."""
+    if (torch.device(device).type == "cuda" and all(type(r) in (list, tuple) and len(r) == len(rows[0]) and
+                                                    all(isinstance(v, (int, float)) for v in r) for r in rows)
+            and not torch.cuda.is_current_stream_capturing()):
+        host = torch.tensor(rows, dtype=torch.float32, pin_memory=True)
+        return host.to(device, non_blocking=True).unbind(0)
+    return [torch.tensor(r, dtype=torch.float32, device=device) for r in rows]
+
+
 def look_at(f, t, width, height, mode="persp", fov=90.0, device="cuda", jitter=False, generator=None):
     """Rays of a camera at `f` looking at `t` with world up +y
     (geoutils.py:180-206), [W*H, 3] origins and unit directions.
@@ -50,9 +62,8 @@ def look_at(f, t, width, height, mode="persp", fov=90.0, device="cuda", jitter=F
     that order (the order fixes the FP32 bits that nglod_camera_rays
     reproduces).  'persp': every ray starts at f towards its plane point;
     'ortho': rays start at the plane points and all run along forward."""
-    eye = torch.tensor(f, dtype=torch.float32, device=device)
-    forward = F.normalize(torch.tensor(t, dtype=torch.float32, device=device) - eye, dim=0)
-    world_up = torch.tensor([0.0, 1.0, 0.0], device=device)
+    eye, at, world_up = _on_device([f, t, (0.0, 1.0, 0.0)], device)
+    forward = F.normalize(at - eye, dim=0)
     side = F.normalize(torch.linalg.cross(forward, world_up), dim=0)
     up = F.normalize(torch.linalg.cross(side, forward), dim=0)
     win = normalized_grid(width, height, device=device, jitter=jitter, generator=generator).reshape(-1, 2)

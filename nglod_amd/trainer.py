@@ -18,6 +18,11 @@ from .optim import Adam
 from . import mesh as _mesh
 
 
+def _training(module):
+    """Whether module and everything in it is in training mode."""
+    return module.training and all(_training(m) for m in module._modules.values() if m is not None)
+
+
 class Trainer:
     def __init__(self, net, lr=1e-3, loss_lods=None):
         self.net = net
@@ -25,7 +30,7 @@ class Trainer:
         self.loss_lods = list(range(net.num_lods)) if loss_lods is None else list(loss_lods)
         self.last_loss = None
 
-    def _fused(self, pts, gts):
+    def _fused(self, pts, gts, params):
         """Whether loss and gradient can come from nglod_geometry_loss: a plain
         OctreeSDF's every-level predictions against one FP32 value per point."""
         net = self.net
@@ -34,15 +39,22 @@ class Trainer:
                 and gts.device == pts.device and not gts.requires_grad and torch.is_grad_enabled()
                 and all(0 <= i < net.num_lods for i in self.loss_lods)
                 and len(set(self.loss_lods)) == len(self.loss_lods) > 0
-                and all(p.requires_grad for p in net.parameters()))
+                and all(p.requires_grad for p in params))
 
     def step_geometry(self, pts, gts):
         net = self.net
-        net.train()
+        params = _lib.parameter_list(net)
+        if type(net) is not OctreeSDF:
+            net.train()
+            net.zero_grad()
+        else:
+            if not _training(net):
+                net.train()
+            for p in params:
+                p.grad = None
         batch_size = pts.shape[0]
-        net.zero_grad()
-        if self._fused(pts, gts):
-            stacked = sdf_with_grad(net, pts, net.num_lods - 1, all_levels=True, stacked=True)
+        if self._fused(pts, gts, params):
+            stacked = sdf_with_grad(net, pts, net.num_lods - 1, all_levels=True, stacked=True, params=params)
             net.loss_preds = list(stacked.unbind(0))
             gt = gts.contiguous()
             grad = torch.empty_like(stacked)
