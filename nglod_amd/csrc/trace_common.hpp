@@ -265,46 +265,40 @@ struct RayState {
     }
 
     __device__ __forceinline__ void consume(const TraceArgs& a, float d, bool replay = false) {
-        if (phase == PH_INIT) {
-            D = d;  // d = net(x) is not scaled by step_size (SphereTracer.py:63)
-            Dp = D;
-            it = 0;
-            check(a, replay);
-        } else if (phase == PH_MARCH) {
-            Dp = D;
-            D = d * a.step;
-            t = t + D;
-            ++it;
-            ++steps;
+        // One path for the entry evaluation and the steps, and one for all taps: the
+        // lanes of a wave are in every phase at once, and each path runs its length.
+        if (phase == PH_INIT || phase == PH_MARCH) {
+            const bool first = phase == PH_INIT;  // d = net(x) is not scaled by step_size (SphereTracer.py:63)
+            Dp = first ? d : D;
+            D = first ? d : d * a.step;
+            t = first ? t : t + D;
+            it = first ? 0 : it + 1;
+            steps = first ? steps : steps + 1;
             check(a, replay);
         } else if (phase < PH_N0 || phase > PH_N5) {
             // not an evaluating phase: end the ray rather than loop on it
             finish(a);
         } else {
             const int k = phase - PH_N0;  // 0..5: axis k/2, + tap then - tap
-            const int axis = k >> 1;
             if ((k & 1) == 0) {
                 fplus = d;
-                qx = axis == 0 ? x0 - kFdH : x0 - 0.0f;
-                qy = axis == 1 ? x1 - kFdH : x1 - 0.0f;
-                qz = axis == 2 ? x2 - kFdH : x2 - 0.0f;
-                ++phase;
             } else {
                 const float g = (fplus - d) / kFdTwoH;
-                if (axis == 0) g0 = g;
-                else if (axis == 1) g1 = g;
-                else g2 = g;
-                if (axis == 2) {
-                    float n0, n1, n2;
-                    normalize_grad(g0, g1, g2, n0, n1, n2);
-                    retire(a, true, n0, n1, n2);
-                } else {
-                    const int na = axis + 1;
-                    qx = na == 0 ? x0 + kFdH : x0 + 0.0f;
-                    qy = na == 1 ? x1 + kFdH : x1 + 0.0f;
-                    qz = na == 2 ? x2 + kFdH : x2 + 0.0f;
-                    ++phase;
-                }
+                g0 = k == 1 ? g : g0;
+                g1 = k == 3 ? g : g1;
+                g2 = k == 5 ? g : g2;
+            }
+            if (k == 5) {
+                float n0, n1, n2;
+                normalize_grad(g0, g1, g2, n0, n1, n2);
+                retire(a, true, n0, n1, n2);
+            } else {
+                const int axis = (k + 1) >> 1;
+                const float h = k & 1 ? kFdH : -kFdH, z = k & 1 ? 0.0f : -0.0f;
+                qx = x0 + (axis == 0 ? h : z);
+                qy = x1 + (axis == 1 ? h : z);
+                qz = x2 + (axis == 2 ? h : z);
+                ++phase;
             }
         }
     }
