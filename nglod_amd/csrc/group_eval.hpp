@@ -132,11 +132,60 @@ __device__ __forceinline__ void group_corners(const float4 (&g)[8], const float4
     }
 }
 
+// The gather for at most eight queries (`act`), as when a march runs out of rays
+// and its trips are all latency: 32 threads per query, a channel each, the rows of
+// four levels on their way at once instead of one level after the other.  Same
+// order of sums.
+template <bool COARSE>
+__device__ __forceinline__ void group_gather_few(const ModelArgs& m, int lod, GroupLds<COARSE>* s, uint32_t act) {
+    const int slot = (int)(threadIdx.x >> 5), c = (int)(threadIdx.x & 31u);
+    if (slot >= __popc(act)) return;
+    const int ray = nth_set_bit(act, slot);
+    float f = 0.0f;
+    auto add = [&](int l, const float (&g)[8]) {
+        const float4* w = s->w[l][ray];
+        const float4 w0 = w[0], w1 = w[1];
+        const float ww[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+        for (int k = 0; k < 8; ++k) f = __builtin_fmaf(g[k], ww[k], f);
+    };
+    int l = 0;
+    if (COARSE && m.res[0] <= 4) {
+        const int S = m.res[0] + 1;
+        const float* b = reinterpret_cast<const float*>(s->coarse) + s->base[0][ray] * kC + c;
+        float g[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) g[k] = b[((k & 1) + (k & 2 ? S : 0) + (k & 4 ? S * S : 0)) * kC];
+        add(0, g);
+        l = 1;
+    }
+#pragma unroll 1
+    for (; l <= lod; l += 4) {
+        float g[4][8];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (l + j <= lod) {
+                const int S = m.res[l + j] + 1;
+                const float* b = m.grid[l + j] + (size_t)s->base[l + j][ray] * kC + c;
+                const size_t sy = (size_t)S * kC, sz = (size_t)S * S * kC;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) g[j][k] = b[(k & 1) * kC + (k & 2 ? sy : 0) + (k & 4 ? sz : 0)];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (l + j <= lod) add(l + j, g[j]);
+    }
+    s->dec.feat[c & 1][ray][c >> 1] = f;
+}
+
 // Every thread of the block, with the position of query lane % 32 (the same in
-// all four waves; any position for queries whose result is not used).
-template <bool POSINV, bool COARSE>
+// all four waves; any position for queries whose result is not used).  act: the
+// queries whose result is used.
+// FEW: with the gather for few queries.
+template <bool POSINV, bool FEW, bool COARSE>
 __device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds<COARSE>* s, const GroupWeights& gw, float b1,
-                                           float px, float py, float pz) {
+                                           uint32_t act, float px, float py, float pz) {
     const uint32_t lane = lane_id(), n = lane & 31u, half = lane >> 5;
     {
         const int l = 2 * (int)(threadIdx.x >> 6) + (int)half;  // NGLOD_MAX_LODS = 8 levels
@@ -153,7 +202,9 @@ __device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds
         }
     }
     __syncthreads();
-    {
+    if (FEW && __popc(act) <= 8) {
+        group_gather_few(m, lod, s, act);
+    } else {
         const uint32_t ray = threadIdx.x >> 3, q = threadIdx.x & 7u;
         float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         float4 g[8];

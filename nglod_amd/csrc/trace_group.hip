@@ -21,7 +21,13 @@ namespace nglod {
 // flight.  A whole frame, 5 LODs, against one ray per lane and 64 rays a wave:
 // 64x48 1339 -> 365 us, 128x96 1367 -> 430, 320x180 1445 -> 677, 1280x720 4091 ->
 // 3430.
-template <bool POSINV>
+//
+// FEW (from LOD 3 on, three levels or more outside LDS): trips of at most eight rays
+// read four levels at once.  A frame ends with rays of up to 128 steps, a few per
+// block: LOD 4, 64x48 348 -> 325 us, 128x96 425 -> 392, 320x180 667 -> 598, 1280x720 the
+// same; at LOD 1 and 2 its instructions cost 2-5% of the large frames and gain
+// nothing.
+template <bool POSINV, bool FEW>
 __global__ __launch_bounds__(kGroupThreads, 4) void trace_dense_fp32_kernel(TraceArgs a) {
     __shared__ GroupLds<true> lds;
     __shared__ int64_t claimed[2];
@@ -63,9 +69,10 @@ __global__ __launch_bounds__(kGroupThreads, 4) void trace_dense_fp32_kernel(Trac
             if (s.phase == PH_IDLE && id < feed.ce) s.start(a, id);
             feed.cb = end < feed.ce ? end : feed.ce;
         }
-        if (__ballot(s.phase != PH_IDLE) == 0) break;
         const bool busy = s.phase != PH_IDLE;
-        const float d = group_sdf<POSINV>(a.m, a.lod, &lds, gw, b1, busy ? s.qx : 0.0f, busy ? s.qy : 0.0f,
+        const uint32_t act = (uint32_t)__ballot(busy);
+        if (act == 0) break;
+        const float d = group_sdf<POSINV, FEW>(a.m, a.lod, &lds, gw, b1, act, busy ? s.qx : 0.0f, busy ? s.qy : 0.0f,
                                           busy ? s.qz : 0.0f);
         if (busy) {
             ++nevals;
@@ -79,13 +86,21 @@ __global__ __launch_bounds__(kGroupThreads, 4) void trace_dense_fp32_kernel(Trac
     }
 }
 
+template <bool POSINV>
+static void launch_dense(const TraceArgs& a, dim3 grid, hipStream_t s) {
+    if (a.lod >= 3)
+        hipLaunchKernelGGL((trace_dense_fp32_kernel<POSINV, true>), grid, dim3(kGroupThreads), 0, s, a);
+    else
+        hipLaunchKernelGGL((trace_dense_fp32_kernel<POSINV, false>), grid, dim3(kGroupThreads), 0, s, a);
+}
+
 int launch_trace_fp32(const TraceArgs& a, int64_t n, hipStream_t s) {
     const int64_t blocks = (n + kGroup - 1) / kGroup, cap = (int64_t)device_cu_count() * 4;
     const dim3 grid((unsigned)(blocks < cap ? blocks : cap));
     if (a.m.pos_inv)
-        hipLaunchKernelGGL(trace_dense_fp32_kernel<true>, grid, dim3(kGroupThreads), 0, s, a);
+        launch_dense<true>(a, grid, s);
     else
-        hipLaunchKernelGGL(trace_dense_fp32_kernel<false>, grid, dim3(kGroupThreads), 0, s, a);
+        launch_dense<false>(a, grid, s);
     return check_launch("trace_dense_fp32_kernel");
 }
 
@@ -104,7 +119,7 @@ __global__ __launch_bounds__(kGroupThreads, 6) void sdf_group_fp32_kernel(ModelA
     const int64_t stride = (int64_t)gridDim.x * kGroup;
     for (int64_t first = (int64_t)blockIdx.x * kGroup; first < n; first += stride) {
         const int64_t i = first + (threadIdx.x & 31u), j = i < n ? i : n - 1;
-        const float d = group_sdf<POSINV>(m, lod, &lds, gw, b1, x[3 * j], x[3 * j + 1], x[3 * j + 2]);
+        const float d = group_sdf<POSINV, false>(m, lod, &lds, gw, b1, ~0u, x[3 * j], x[3 * j + 1], x[3 * j + 2]);
         if (threadIdx.x < kGroup && i < n) out[i] = d;
     }
 }
