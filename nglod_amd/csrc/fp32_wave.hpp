@@ -2,8 +2,9 @@
 // trilinear gather per lane, then the first decoder layer as FP32 MFMA
 // 32x32x2 tiles (v_mfma_f32_32x32x2_f32: exact FP32 products, FP32
 // accumulation), then bias, ReLU and the 128 -> 1 layer in FP32 on the MFMA
-// output registers.  Twice the FP32 rate of the vector FMA decoder, and it
-// runs beside the vector ALU work of the other waves.
+// output registers.  Twice the FP32 rate of the vector FMA decoder (the two do
+// not overlap on a SIMD: 64 cycles per product plus 4.4 per vector FMA, whatever
+// the number of waves).
 //
 // MFMA operand layout (32x32x2, one block): lane l holds A[m = l%32][k = l/32]
 // and B[k = l/32][n = l%32]; output: lane l holds C[m][n = l%32] for

@@ -26,11 +26,13 @@ namespace nglod {
 
 constexpr int kGroup = 32;            // queries of a block
 constexpr int kGroupThreads = 256;
+constexpr int kFewQueries = 16;       // group_decode_few's columns
 constexpr int kFeatStride = 20;       // floats between queries: 16-byte aligned, spread over the banks
 
 struct alignas(16) GroupDecoder {
     float feat[2][kGroup][kFeatStride];  // [half][query][kk] = channel 2 kk + half
     float part[4][64];
+    int col[kGroup];                     // group_decode_few: the query of each column
     float b0[kH];
     float w1[kH];
     float wxyz[kH][4];
@@ -110,6 +112,89 @@ __device__ __forceinline__ float group_decode(GroupDecoder* s, const GroupWeight
     return halves_sum(p, p) + b1;
 }
 
+// From here on this block decodes with group_decode_few: the rows as A operands of
+// v_mfma_f32_16x16x4_f32, gw.a[2 k + s] of lane (m, j) = W0[32 h + 16 s + m][4 k + j]
+// (m = lane % 16, j = lane / 16).
+__device__ __forceinline__ void few_weights(GroupWeights& gw) {
+#pragma unroll
+    for (int k = 0; k < kC / 4; ++k) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(gw.a[2 * k]), __float_as_uint(gw.a[2 * k + 1]),
+                                                        false, false);
+        const auto q = __builtin_amdgcn_permlane16_swap(p[0], p[1], false, false);
+        gw.a[2 * k] = __uint_as_float(q[0]);
+        gw.a[2 * k + 1] = __uint_as_float(q[1]);
+    }
+}
+
+// Column of query n of `act` (the queries of `act` first).  The first 32 threads
+// store it before a barrier that comes before group_decode_few.
+__device__ __forceinline__ uint32_t few_column(uint32_t act, uint32_t n) {
+    const uint32_t rank = (uint32_t)__popc(act & ((1u << n) - 1u));
+    return (act >> n) & 1u ? rank : (uint32_t)__popc(act) + n - rank;
+}
+
+// group_decode for at most 16 queries `act`: half the matrix work, in two chains
+// of eight products instead of one of sixteen of twice the length.  The same sums in
+// the same order: a chain of the second layer takes units 0-3, 8-11, 16-19, 24-27 (or
+// 4-7, ...), which lie in lanes n, n + 32, n, n + 32 here and pass the sum on.
+template <bool POSINV>
+__device__ __forceinline__ float group_decode_few(GroupDecoder* s, const GroupWeights& gw, float b1, uint32_t act,
+                                                  float px, float py, float pz) {
+    typedef float f32x4_t __attribute__((ext_vector_type(4)));
+    const uint32_t lane = lane_id(), m = lane & 15u, j = lane >> 4;
+    const int h = (int)(threadIdx.x >> 6);
+    const int query = s->col[m];
+    float pos = 0.0f;
+    if (!POSINV) {
+        const float x = __shfl(px, query), y = __shfl(py, query), z = __shfl(pz, query);
+        pos = j == 0 ? z : j == 1 ? y : j == 2 ? x : 0.0f;
+    }
+    __syncthreads();
+    f32x4_t c[2] = {{}, {}};
+    const float* b = &s->feat[j & 1u][query][j >> 1];
+#pragma unroll
+    for (int k = 0; k < kC / 4; ++k) {
+        c[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(gw.a[2 * k], b[2 * k], c[0], 0, 0, 0);
+        c[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(gw.a[2 * k + 1], b[2 * k], c[1], 0, 0, 0);
+    }
+    float4 w[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int unit = 32 * h + 16 * t + 4 * (int)j;
+        const float4 bias = *reinterpret_cast<const float4*>(&s->b0[unit]);
+        c[t][0] += bias.x;
+        c[t][1] += bias.y;
+        c[t][2] += bias.z;
+        c[t][3] += bias.w;
+        if (!POSINV)
+            c[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(s->wxyz[32 * h + 16 * t + (int)m][j == 3 ? 3 : 2 - j], pos, c[t],
+                                                        0, 0, 0);
+        w[t] = *reinterpret_cast<const float4*>(&s->w1[unit]);
+    }
+    float acc = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            acc = __builtin_fmaf(w[t].x, fmaxf(c[t][0], 0.0f), acc);
+            acc = __builtin_fmaf(w[t].y, fmaxf(c[t][1], 0.0f), acc);
+            acc = __builtin_fmaf(w[t].z, fmaxf(c[t][2], 0.0f), acc);
+            acc = __builtin_fmaf(w[t].w, fmaxf(c[t][3], 0.0f), acc);
+            if (t + u < 2) {
+                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc), __float_as_uint(acc), false, false);
+                acc = __uint_as_float(sw[u]);
+            }
+        }
+    }
+    if (j >= 2) s->part[h][m + 32u * (j & 1u)] = acc;
+    const uint32_t from = few_column(act, lane & 31u) + (lane & 32u);
+    __syncthreads();
+    float p = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) p += s->part[k][from];
+    return halves_sum(p, p) + b1;
+}
+
 // Eight corner rows' float4 of this thread.
 __device__ __forceinline__ void group_rows(const float* __restrict__ grid, int S, uint32_t base, uint32_t q,
                                            float4 (&g)[8]) {
@@ -182,8 +267,9 @@ __device__ __forceinline__ void group_gather_few(const ModelArgs& m, int lod, Gr
 // Every thread of the block, with the position of query lane % 32 (the same in
 // all four waves; any position for queries whose result is not used).  act: the
 // queries whose result is used.
-// FEW: with the gather for few queries.
-template <bool POSINV, bool FEW, bool COARSE>
+// FEW: group_gather_few for at most eight of them.  DECODE_FEW: at most 16 of them, and
+// few_weights has run.
+template <bool POSINV, bool FEW, bool DECODE_FEW, bool COARSE>
 __device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds<COARSE>* s, const GroupWeights& gw, float b1,
                                            uint32_t act, float px, float py, float pz) {
     const uint32_t lane = lane_id(), n = lane & 31u, half = lane >> 5;
@@ -201,6 +287,7 @@ __device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds
             s->w[l][n][1] = make_float4(wxy00 * az.w1, wxy10 * az.w1, wxy01 * az.w1, wxy11 * az.w1);
         }
     }
+    if (DECODE_FEW && threadIdx.x < kGroup) s->dec.col[few_column(act, n)] = (int)n;
     __syncthreads();
     if (FEW && __popc(act) <= 8) {
         group_gather_few(m, lod, s, act);
@@ -225,6 +312,7 @@ __device__ __forceinline__ float group_sdf(const ModelArgs& m, int lod, GroupLds
         }
         store_features(&s->dec, ray, q, f);
     }
+    if (DECODE_FEW) return group_decode_few<POSINV>(&s->dec, gw, b1, act, px, py, pz);
     return group_decode<POSINV>(&s->dec, gw, b1, px, py, pz);
 }
 

@@ -22,17 +22,25 @@ namespace nglod {
 // 64x48 1339 -> 365 us, 128x96 1367 -> 430, 320x180 1445 -> 677, 1280x720 4091 ->
 // 3430.
 //
-// FEW (from LOD 3 on, three levels or more outside LDS): trips of at most eight rays
-// read four levels at once.  A frame ends with rays of up to 128 steps, a few per
-// block: LOD 4, 64x48 348 -> 325 us, 128x96 425 -> 392, 320x180 667 -> 598, 1280x720 the
-// same; at LOD 1 and 2 its instructions cost 2-5% of the large frames and gain
-// nothing.
-template <bool POSINV, bool FEW>
+// FEW: trips of at most eight rays read four levels at once.  TAIL: once no rays are
+// left to claim, trips of at most 16 rays run in a loop of their own, where
+// group_decode_few takes half the matrix work (0.2 us) and at most eight rays read
+// four levels at once, too.  A frame ends with rays of up to 128 steps, a few per
+// block, whose trips are pure latency.  A whole frame at LOD 1 / 2 / 4, us: 64x48
+// without the loop 275 / 322 / 325 (FEW; 348 without), with it 261 / 279 / 290; 128x96 302 /
+// 385 / 395, 283 / 322 / 346; 320x180 451 / 516 / 593, 415 / 450 / 535; 640x360 800 / 975 / 1165,
+// 816 / 915 / 1135; 960x540 1390 / 1705 / 2096 (2182 without FEW), 1435 / 1685 / 2104; 1280x720
+// 2230 / 2704 / 3382, 2346 / 2761 / 3427: the second loop costs the first one up to 5%,
+// hence the line at kTailRays.  Above it FEW from LOD 3 on: below, its instructions
+// cost 2-5% and there are too few levels to gain by it.
+constexpr int64_t kTailRays = 1 << 18;
+
+template <bool POSINV, bool TAIL, bool FEW>
 __global__ __launch_bounds__(kGroupThreads, 4) void trace_dense_fp32_kernel(TraceArgs a) {
     __shared__ GroupLds<true> lds;
     __shared__ int64_t claimed[2];
     __shared__ int claims_left;
-    const GroupWeights gw = stage_group(a.m, a.dec, &lds);
+    GroupWeights gw = stage_group(a.m, a.dec, &lds);
     const float b1 = a.m.b1[a.dec][0];
     const uint32_t lane = lane_id();
     const bool first = threadIdx.x < 64;
@@ -71,9 +79,21 @@ __global__ __launch_bounds__(kGroupThreads, 4) void trace_dense_fp32_kernel(Trac
         }
         const bool busy = s.phase != PH_IDLE;
         const uint32_t act = (uint32_t)__ballot(busy);
+        if (TAIL ? feed.empty() && __popc(act) <= kFewQueries : act == 0) break;
+        const float d = group_sdf<POSINV, FEW, false>(a.m, a.lod, &lds, gw, b1, act, busy ? s.qx : 0.0f, busy ? s.qy : 0.0f,
+                                                      busy ? s.qz : 0.0f);
+        if (busy) {
+            ++nevals;
+            s.consume(a, d);
+        }
+    }
+    if (TAIL) few_weights(gw);
+    while (TAIL) {
+        const bool busy = s.phase != PH_IDLE;
+        const uint32_t act = (uint32_t)__ballot(busy);
         if (act == 0) break;
-        const float d = group_sdf<POSINV, FEW>(a.m, a.lod, &lds, gw, b1, act, busy ? s.qx : 0.0f, busy ? s.qy : 0.0f,
-                                          busy ? s.qz : 0.0f);
+        const float d = group_sdf<POSINV, true, true>(a.m, a.lod, &lds, gw, b1, act, busy ? s.qx : 0.0f, busy ? s.qy : 0.0f,
+                                                      busy ? s.qz : 0.0f);
         if (busy) {
             ++nevals;
             s.consume(a, d);
@@ -87,20 +107,22 @@ __global__ __launch_bounds__(kGroupThreads, 4) void trace_dense_fp32_kernel(Trac
 }
 
 template <bool POSINV>
-static void launch_dense(const TraceArgs& a, dim3 grid, hipStream_t s) {
-    if (a.lod >= 3)
-        hipLaunchKernelGGL((trace_dense_fp32_kernel<POSINV, true>), grid, dim3(kGroupThreads), 0, s, a);
+static void launch_dense(const TraceArgs& a, int64_t n, dim3 grid, hipStream_t s) {
+    if (n <= kTailRays)
+        hipLaunchKernelGGL((trace_dense_fp32_kernel<POSINV, true, false>), grid, dim3(kGroupThreads), 0, s, a);
+    else if (a.lod >= 3)
+        hipLaunchKernelGGL((trace_dense_fp32_kernel<POSINV, false, true>), grid, dim3(kGroupThreads), 0, s, a);
     else
-        hipLaunchKernelGGL((trace_dense_fp32_kernel<POSINV, false>), grid, dim3(kGroupThreads), 0, s, a);
+        hipLaunchKernelGGL((trace_dense_fp32_kernel<POSINV, false, false>), grid, dim3(kGroupThreads), 0, s, a);
 }
 
 int launch_trace_fp32(const TraceArgs& a, int64_t n, hipStream_t s) {
     const int64_t blocks = (n + kGroup - 1) / kGroup, cap = (int64_t)device_cu_count() * 4;
     const dim3 grid((unsigned)(blocks < cap ? blocks : cap));
     if (a.m.pos_inv)
-        launch_dense<true>(a, grid, s);
+        launch_dense<true>(a, n, grid, s);
     else
-        launch_dense<false>(a, grid, s);
+        launch_dense<false>(a, n, grid, s);
     return check_launch("trace_dense_fp32_kernel");
 }
 
@@ -119,7 +141,7 @@ __global__ __launch_bounds__(kGroupThreads, 6) void sdf_group_fp32_kernel(ModelA
     const int64_t stride = (int64_t)gridDim.x * kGroup;
     for (int64_t first = (int64_t)blockIdx.x * kGroup; first < n; first += stride) {
         const int64_t i = first + (threadIdx.x & 31u), j = i < n ? i : n - 1;
-        const float d = group_sdf<POSINV, false>(m, lod, &lds, gw, b1, ~0u, x[3 * j], x[3 * j + 1], x[3 * j + 2]);
+        const float d = group_sdf<POSINV, false, false>(m, lod, &lds, gw, b1, ~0u, x[3 * j], x[3 * j + 1], x[3 * j + 2]);
         if (threadIdx.x < kGroup && i < n) out[i] = d;
     }
 }

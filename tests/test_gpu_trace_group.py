@@ -75,3 +75,27 @@ def test_same_bits_as_whole_batch_steps(dev, n, base_lod, num_lods, pos_invarian
         assert (rb.normal[hit] - _normals(net, x[hit], lod)).abs().max() <= 4e-7
     if n > 1000:
         assert n // 10 < hit.sum() < n
+
+
+@pytest.mark.parametrize("n, num_lods, pos_invariant",
+                         [(15, 5, False), (16, 1, False), (17, 5, True), (47, 3, False), (100, 8, True),
+                          ((1 << 18) + 33, 2, False), ((1 << 19) + 1, 4, True)])
+def test_few_rays_and_long_frames(dev, n, num_lods, pos_invariant):
+    """Around the 16 and 8 rays from which a block's last trips go other ways, and
+    frames long enough to go without them: the same bits."""
+    base_lod = 1 if num_lods == 8 else 2
+    net = workloads.make_sphere_model(radius=0.6, num_lods=num_lods, base_lod=base_lod, pos_invariant=pos_invariant,
+                                      device="cpu").to(dev)
+    o, d = rand_rays(n, 7 + n)
+    o[::5] *= 0.2
+    o, d = torch.from_numpy(o).to(dev), torch.from_numpy(d).to(dev)
+    net.lod = num_lods - 1
+    steps = torch.full((n,), -1, dtype=torch.int32, device=dev)
+    rb = SphereTracer(num_steps=24, min_dis=MIN_DIS)(net, o, d, ray_steps=steps)
+    x, t, hit, count = _step_all(net, o, d, num_lods - 1, 24)
+    assert torch.equal(rb.hit.reshape(-1), hit)
+    assert torch.equal(rb.x, x)
+    assert torch.equal(rb.depth.reshape(-1), t)
+    assert torch.equal(steps, count)
+    if hit.any():
+        assert (rb.normal[hit] - _normals(net, x[hit], num_lods - 1)).abs().max() <= 4e-7
