@@ -386,9 +386,8 @@ def train_bench(dev, reps=5):
     e[3].record()
     torch.cuda.synchronize()
     m2s = e[0].elapsed_time(e[1]) / reps
-    pairs = n * md.nf / (m2s * 1e-3)
+    pairs = n * md.nf / (m2s * 1e-3)  # point-triangle pairs decided (most by their box alone) per second
     return {"samples": n, "triangles": int(md.nf), "mesh2sdf_ms": m2s, "mesh2sdf_pairs_per_s": pairs,
-            "mesh2sdf_fp64_TFLOPs_nominal": pairs * 200 / 1e12,  # ~200 FP64 FLOP per pair; peak 78.6
             "batch_ms": e[1].elapsed_time(e[2]) / reps, "step_ms": e[2].elapsed_time(e[3]) / reps,
             "loss": float(tr.last_loss.item())}
 
