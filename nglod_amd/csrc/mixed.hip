@@ -22,6 +22,7 @@
 // append counter hit by every wave serialised the march kernels measurably.
 #include "api_common.hpp"
 #include "fp32_wave.hpp"
+#include "group_eval.hpp"
 #include "mixed_device.hpp"
 #include "split_wave.hpp"
 #include "trace_common.hpp"
@@ -291,6 +292,148 @@ __global__ __launch_bounds__(kMixedBlock) void trace_mixed_pass1_kernel(TraceArg
     add_evals(a, 1, nevals, lane);
 }
 
+struct alignas(16) Pass2Lds {
+    uint32_t frag[3][2][kGroup][12];  // [part][half][query][pair q]: channels 4 q + half and 4 q + 2 + half
+    float4 w[kGroup][2];              // corner weights
+    float pos[3][kGroup];
+    float part[4][64];
+    float b0[kH];
+    float w1[kH];
+    float wxyz[kH][4];
+    uint32_t base[kGroup];
+    uint32_t act;
+};
+
+// Pass 2 by groups: a block of four waves takes 32 rays, one evaluation of all of them
+// a trip (group_eval.hpp's split of the work, with the split-BF16 decoder, whose
+// rows of W0 stay in 24 registers).  The first wave keeps the rays' state in its lower
+// lanes, claims records and computes the cells; eight threads per ray gather its
+// corners and split the features; each wave decodes 32 hidden units.  The same sums in
+// the same order as trace_mixed_pass2_kernel: the same bits.
+//
+// Small frames are bound by the longest rays' trips, large ones by the owner wave's
+// serial part and the barriers, with four blocks a CU by registers.  Whole mixed frames
+// at LOD 1 / 2 (xyz) / 4 / 4 (xyz), 64 rays per wave -> this, us: 64x48 375 / 441 / 433 / 475 ->
+// 303 / 366 / 311 / 356; 128x96 356 / 434 / 428 / 480 -> 315 / 388 / 352 / 406; 320x180 395 / 487 /
+// 430 / 492 -> 355 / 437 / 368 / 425; 640x360 615 / 710 / 633 / 816 -> 546 / 656 / 568 / 690; 1280x720
+// 935 / 1270 / 1040 / 1198 -> 945 / 1160 / 995 / 1200; 1920x1080 1694 / 2016 / 1712 / 1998 -> 1679 / 2059 /
+// 1747 / 2081: hence the line at kPass2GroupRays.  A queue of records with their rays
+// in LDS, so that a refill does not wait for memory, gave nothing.
+constexpr int64_t kPass2GroupRays = 1 << 20;
+
+template <bool POSINV, bool RETURNS>
+__global__ __launch_bounds__(kGroupThreads, 4) void trace_mixed_pass2_group_kernel(TraceArgs a) {
+    __shared__ Pass2Lds lds;
+    const uint32_t lane = lane_id(), n = lane & 31u, half = lane >> 5;
+    const int h = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const bool owner = h == 0;
+    const float b1 = a.m.b1[a.dec][0];
+    bf16x8 ah[2], am[2], al[2];
+    {
+        const float* W0 = a.m.w0[a.dec];
+        const int off = POSINV ? 0 : 3, din = kC + off;
+        const float* row = W0 + (32 * h + (int)n) * din + off + (int)half;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            uint32_t ph[4], pm[4], pl[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                split3_pair(row[2 * (8 * kb + 2 * q)], row[2 * (8 * kb + 2 * q + 1)], ph[q], pm[q], pl[q]);
+            ah[kb] = __builtin_bit_cast(bf16x8, make_uint4(ph[0], ph[1], ph[2], ph[3]));
+            am[kb] = __builtin_bit_cast(bf16x8, make_uint4(pm[0], pm[1], pm[2], pm[3]));
+            al[kb] = __builtin_bit_cast(bf16x8, make_uint4(pl[0], pl[1], pl[2], pl[3]));
+        }
+        for (int j = threadIdx.x; j < kH; j += kGroupThreads) {
+            lds.b0[j] = a.m.b0[a.dec][j];
+            lds.w1[j] = a.m.w1[a.dec][j];
+            for (int k = 0; k < 3; ++k) lds.wxyz[j][k] = POSINV ? 0.0f : W0[j * din + k];
+            lds.wxyz[j][3] = 0.0f;
+        }
+    }
+    const int r = a.m.res[0], S = r + 1;
+    const float* grid = a.m.grid[0];
+    RayFeed feed;
+    feed.init(a.nrays, a.queue_stride);
+    RayState s;
+    s.ray = -1;
+    s.phase = PH_IDLE;
+    uint32_t nevals = 0;
+    for (;;) {
+        if (owner) {
+            const int64_t id =
+                feed.next_flagged<true>(a.handoff_queue, a.hflag, lane, lane < kGroup && s.phase == PH_IDLE);
+            if (id >= 0) s.resume(a, a.handoff[id]);
+            const bool busy = s.phase != PH_IDLE;
+            const uint32_t act = (uint32_t)__ballot(busy);
+            if (lane < kGroup) {
+                const float px = busy ? s.qx : 0.0f, py = busy ? s.qy : 0.0f, pz = busy ? s.qz : 0.0f;
+                const AxisW ax = axis_weights(px, r);
+                const AxisW ay = axis_weights(py, r);
+                const AxisW az = axis_weights(pz, r);
+                const float wxy00 = ax.w0 * ay.w0, wxy10 = ax.w1 * ay.w0;
+                const float wxy01 = ax.w0 * ay.w1, wxy11 = ax.w1 * ay.w1;
+                lds.base[n] = (uint32_t)((az.i0 * S + ay.i0) * S + ax.i0);
+                lds.w[n][0] = make_float4(wxy00 * az.w0, wxy10 * az.w0, wxy01 * az.w0, wxy11 * az.w0);
+                lds.w[n][1] = make_float4(wxy00 * az.w1, wxy10 * az.w1, wxy01 * az.w1, wxy11 * az.w1);
+                if (!POSINV) {
+                    lds.pos[0][n] = px;
+                    lds.pos[1][n] = py;
+                    lds.pos[2][n] = pz;
+                }
+                if (lane == 0) lds.act = act;
+            }
+        }
+        __syncthreads();
+        const uint32_t act = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.act);
+        if (act == 0) break;
+        {
+            const uint32_t query = threadIdx.x >> 3, q = threadIdx.x & 7u;
+            if ((act >> query) & 1u) {
+                float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                float4 g[8];
+                group_rows(grid, S, lds.base[query], q, g);
+                group_corners(g, lds.w[query], f);
+                uint32_t p[3];
+                split3_pair(f.x, f.z, p[0], p[1], p[2]);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) lds.frag[k][0][query][q] = p[k];
+                split3_pair(f.y, f.w, p[0], p[1], p[2]);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) lds.frag[k][1][query][q] = p[k];
+            }
+        }
+        __syncthreads();
+        {
+            bf16x8 b[3][2];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+                    b[k][kb] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&lds.frag[k][half][n][4 * kb]));
+            }
+            const f32x16 c = split_tile(ah, am, al, b[0], b[1], b[2], bias_tile(h, half, &lds));
+            lds.part[h][lane] = layer2_partial(c, h, half, &lds, !POSINV, POSINV ? 0.0f : lds.pos[0][n],
+                                               POSINV ? 0.0f : lds.pos[1][n], POSINV ? 0.0f : lds.pos[2][n]);
+        }
+        __syncthreads();
+        if (owner) {
+            float p = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) p += lds.part[k][lane];
+            const float d = halves_sum(p, p) + b1;
+            if (s.phase != PH_IDLE) {
+                ++nevals;
+                s.consume(a, d);
+                // hand back only a ray that moves away from the surface (step growing)
+                if (RETURNS && s.phase == PH_MARCH && fabsf(s.D) > a.return_dist && fabsf(s.D) > fabsf(s.Dp))
+                    s.hand_off_to(a.ret, a.rflag);
+            }
+        }
+    }
+    if (owner) add_evals(a, 0, nevals, lane);
+}
+
+// Pass 2 of frames of more than kPass2GroupRays rays, 64 a wave.
 // RETURNS: near misses may be handed back to a later pass 1 (not in the last
 // round); a separate instantiation, as for pass 1.
 template <bool POSINV, bool RETURNS>
@@ -735,6 +878,17 @@ static int grid_for(K kernel, int64_t n, int block) {
     return (int)(want < cap ? (want < 1 ? 1 : want) : cap);
 }
 
+template <bool POSINV, bool RETURNS>
+static void launch_pass2(const TraceArgs& a, int64_t n, hipStream_t s) {
+    if (n <= kPass2GroupRays) {
+        const int64_t blocks = (n + kGroup - 1) / kGroup, cap = (int64_t)device_cu_count() * 4;
+        hipLaunchKernelGGL((trace_mixed_pass2_group_kernel<POSINV, RETURNS>), dim3((unsigned)(blocks < cap ? blocks : cap)),
+                           dim3(kGroupThreads), 0, s, a);
+    } else {
+        const int blocks = grid_for(trace_mixed_pass2_kernel<POSINV, RETURNS>, n, kPass2Block);
+        hipLaunchKernelGGL((trace_mixed_pass2_kernel<POSINV, RETURNS>), dim3(blocks), dim3(kPass2Block), 0, s, a);
+    }
+}
 
 __global__ void clear_words_kernel(uint32_t* p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -762,7 +916,6 @@ template <bool POSINV>
 static int trace_mixed_rounds(TraceArgs a, int64_t n, hipStream_t s, PassTimer& timer) {
     const int g1 = grid_for(trace_mixed_pass1_kernel<POSINV, false>, n, kMixedBlock);
     const int g1r = grid_for(trace_mixed_pass1_kernel<POSINV, true>, n, kMixedBlock);
-    const int g2 = grid_for(trace_mixed_pass2_kernel<POSINV, false>, n, kPass2Block);
     const int words = (int)((n + 3) / 4);
     const dim3 cg((unsigned)((words + 255) / 256));
     const int rounds = a.return_dist > 0.0f ? kMixedRounds : 1;
@@ -789,9 +942,9 @@ static int trace_mixed_rounds(TraceArgs a, int64_t n, hipStream_t s, PassTimer& 
             timer.mark(kPassOther);
         }
         if (allow_return)
-            hipLaunchKernelGGL((trace_mixed_pass2_kernel<POSINV, true>), dim3(g2), dim3(kPass2Block), 0, s, a2);
+            launch_pass2<POSINV, true>(a2, n, s);
         else
-            hipLaunchKernelGGL((trace_mixed_pass2_kernel<POSINV, false>), dim3(g2), dim3(kPass2Block), 0, s, a2);
+            launch_pass2<POSINV, false>(a2, n, s);
         rc = check_launch("trace_mixed_pass2_kernel");
         if (rc) return rc;
         timer.mark(kPassFp32);

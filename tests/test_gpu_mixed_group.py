@@ -1,0 +1,37 @@
+"""The mixed trace's FP32 pass by groups of 32 rays (up to 2^20 rays) against the
+one with 64 rays a wave (above): a ray's result does not depend on the others, so
+the rays of a small batch have the same bits when they are part of a large one."""
+import pytest
+import torch
+
+from nglod_amd import workloads
+from nglod_amd.tracer import SphereTracer
+
+from helpers import rand_rays
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n, num_lods, pos_invariant, return_dist",
+                         [(1, 5, True, 0.0), (31, 3, False, 0.0), (33, 5, False, 2e-3), (4099, 5, True, 2e-3),
+                          (4099, 1, True, 0.0), (200001, 5, False, 0.0)])
+def test_small_batch_same_bits_as_in_a_large_one(dev, n, num_lods, pos_invariant, return_dist):
+    net = workloads.make_sphere_model(radius=0.6, num_lods=num_lods, base_lod=2, pos_invariant=pos_invariant,
+                                      device="cpu").to(dev)
+    net.lod = num_lods - 1
+    o, d = rand_rays(n, 11 + n)
+    o[::7] *= 0.2
+    o, d = torch.from_numpy(o).to(dev), torch.from_numpy(d).to(dev)
+    many = (1 << 20) // n + 1
+
+    def trace(o, d):
+        steps = torch.full((len(o),), -1, dtype=torch.int32, device=dev)
+        tracer = SphereTracer(form="mixed", near_dist=1e-2, return_dist=return_dist)
+        rb = tracer(net, o, d, ray_steps=steps)
+        return rb.x, rb.depth.reshape(-1), rb.hit.reshape(-1), rb.normal, steps
+
+    small, large = trace(o, d), trace(o.repeat(many, 1), d.repeat(many, 1))
+    for a, b in zip(small, large):
+        assert torch.equal(a, b[:n]) and torch.equal(a, b[-n:])
+    if n > 1000:
+        assert n // 10 < small[2].sum() < n
