@@ -159,15 +159,4 @@ struct SoloLevels {
     int res[NGLOD_MAX_LODS];
 };
 
-// Every thread of the block calls this before the block's __syncthreads().
-__device__ __forceinline__ void stage_solo_levels(const ModelArgs& m, SoloLevels* lv) {
-#pragma unroll
-    for (int l = 0; l < NGLOD_MAX_LODS; ++l) {
-        if ((int)threadIdx.x == l) {
-            lv->grid[l] = m.grid[l];
-            lv->res[l] = m.res[l];
-        }
-    }
-}
-
 }  // namespace nglod

@@ -31,19 +31,9 @@ namespace nglod {
 
 // Pass 1 reads its grid from global memory: with LDS copies of coarse levels
 // (when it gathered every level) it measured 10-20% slower on the 1280x720
-// LOD-4 frame.  Pass 2 gathers one FP32 cumulative grid per query and keeps
-// only the decoder in LDS (134 VGPRs); 512-thread blocks measured faster than
-// 256 for it (0.51 against 0.59 ms, before it took the normal taps), and more
-// waves per SIMD did not help.
+// LOD-4 frame.
 constexpr int kMixedBlock = 256;
-#ifndef NGLOD_MIXED_FP32_BLOCK
-#define NGLOD_MIXED_FP32_BLOCK 512
-#endif
-#ifndef NGLOD_MIXED_FP32_WAVES
-#define NGLOD_MIXED_FP32_WAVES 2
-#endif
-constexpr int kPass2Block = NGLOD_MIXED_FP32_BLOCK;
-constexpr int kMixedFp32Waves = NGLOD_MIXED_FP32_WAVES;
+constexpr int kPass2Rays = 64;  // of a block of kGroupThreads
 // Pass 1 claims rays 32 ids at a time (the FP32 march claims per idle lane):
 // measured faster for the mixed march, slightly slower for the FP32 one.  On
 // the 1280x720 LOD-4 frame with the claim counters one line apart: 16 ids
@@ -207,8 +197,8 @@ __device__ __forceinline__ void add_evals(const TraceArgs& a, int slot, uint32_t
 // RESUME: a later round, over the rays pass 2 handed back (ret, rflag)
 // instead of the frame's rays.  A separate instantiation: compiled into the
 // first-round kernel, the resume path slowed its march by half even unused.
-// Up to this many busy lanes, a drained wave of the FP32 passes and of the
-// pooled march gathers cooperatively (16 lanes per query).
+// Up to this many busy lanes, a drained wave of the pooled passes
+// gathers cooperatively (16 lanes per query).
 constexpr int kCoopLanes = 4;
 // Pass 1's tail: up to 8 busy lanes, 16 lanes per query up to 4 of them
 // (gather_fp16_coop) and 8 lanes per query above (gather_fp16_coop8); on
@@ -293,36 +283,37 @@ __global__ __launch_bounds__(kMixedBlock) void trace_mixed_pass1_kernel(TraceArg
 }
 
 struct alignas(16) Pass2Lds {
-    uint32_t frag[3][2][kGroup][12];  // [part][half][query][pair q]: channels 4 q + half and 4 q + 2 + half
-    float4 w[kGroup][2];              // corner weights
-    float pos[3][kGroup];
-    float part[4][64];
+    uint32_t frag[3][2][kPass2Rays][12];  // [part][half][query][pair q]: channels 4 q + half and 4 q + 2 + half
+    float4 w[kPass2Rays][2];              // corner weights
+    float pos[3][kPass2Rays];
+    float part[4][2][64];
     float b0[kH];
     float w1[kH];
     float wxyz[kH][4];
-    uint32_t base[kGroup];
-    uint32_t act;
+    uint32_t base[kPass2Rays];
+    uint64_t act;
 };
 
-// Pass 2 by groups: a block of four waves takes 32 rays, one evaluation of all of them
-// a trip (group_eval.hpp's split of the work, with the split-BF16 decoder, whose
-// rows of W0 stay in 24 registers).  The first wave keeps the rays' state in its lower
-// lanes, claims records and computes the cells; eight threads per ray gather its
-// corners and split the features; each wave decodes 32 hidden units.  The same sums in
-// the same order as trace_mixed_pass2_kernel: the same bits.
+// Pass 2: a block of four waves takes 64 rays, one evaluation of all of them a trip
+// (group_eval.hpp's split of the work, two tiles of 32, with the split-BF16 decoder,
+// whose rows of W0 stay in 24 registers).  The first wave keeps the rays' state,
+// claims records and computes the cells; eight threads per ray gather its corners and
+// split the features; each wave decodes 32 hidden units.  The sums have the order of
+// decode_split_wave.
 //
-// Small frames are bound by the longest rays' trips, large ones by the owner wave's
-// serial part and the barriers, with four blocks a CU by registers.  Whole mixed frames
-// at LOD 1 / 2 (xyz) / 4 / 4 (xyz), 64 rays per wave -> this, us: 64x48 375 / 441 / 433 / 475 ->
-// 303 / 366 / 311 / 356; 128x96 356 / 434 / 428 / 480 -> 315 / 388 / 352 / 406; 320x180 395 / 487 /
-// 430 / 492 -> 355 / 437 / 368 / 425; 640x360 615 / 710 / 633 / 816 -> 546 / 656 / 568 / 690; 1280x720
-// 935 / 1270 / 1040 / 1198 -> 945 / 1160 / 995 / 1200; 1920x1080 1694 / 2016 / 1712 / 1998 -> 1679 / 2059 /
-// 1747 / 2081: hence the line at kPass2GroupRays.  A queue of records with their rays
-// in LDS, so that a refill does not wait for memory, gave nothing.
-constexpr int64_t kPass2GroupRays = 1 << 20;
-
+// Small frames are bound by the longest rays' trips, large ones by the vector ALU and the
+// owner wave's serial part, with four blocks a CU by registers.  Whole mixed frames at LOD 1 / 2
+// (xyz) / 4 / 4 (xyz), us, a ray per lane and 64 rays a wave -> this: 64x48 377 / 443 / 433 / 476
+// -> 296 / 358 / 300 / 348; 128x96 358 / 435 / 428 / 483 -> 314 / 381 / 344 / 403; 320x180 398 /
+// 495 / 430 / 490 -> 363 / 442 / 372 / 431; 640x360 627 / 706 / 627 / 826 -> 561 / 659 / 585 / 721;
+// 1280x720 942 / 1278 / 1040 / 1211 -> 918 / 1207 / 1004 / 1183; 1920x1080 1697 / 2029 / 1700 / 2003
+// -> 1674 / 2000 / 1690 / 2034.  32 rays a block: the same up to 640x360, 2% slower above.
+// A queue of records with their rays in LDS, so that a refill does not wait for
+// memory, gave nothing.
+// RETURNS: near misses may be handed back to a later pass 1 (not in the last
+// round); a separate instantiation, as for pass 1.
 template <bool POSINV, bool RETURNS>
-__global__ __launch_bounds__(kGroupThreads, 4) void trace_mixed_pass2_group_kernel(TraceArgs a) {
+__global__ __launch_bounds__(kGroupThreads, 4) void trace_mixed_pass2_kernel(TraceArgs a) {
     __shared__ Pass2Lds lds;
     const uint32_t lane = lane_id(), n = lane & 31u, half = lane >> 5;
     const int h = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -361,33 +352,34 @@ __global__ __launch_bounds__(kGroupThreads, 4) void trace_mixed_pass2_group_kern
     for (;;) {
         if (owner) {
             const int64_t id =
-                feed.next_flagged<true>(a.handoff_queue, a.hflag, lane, lane < kGroup && s.phase == PH_IDLE);
+                feed.next_flagged<true>(a.handoff_queue, a.hflag, lane, s.phase == PH_IDLE);
             if (id >= 0) s.resume(a, a.handoff[id]);
             const bool busy = s.phase != PH_IDLE;
-            const uint32_t act = (uint32_t)__ballot(busy);
-            if (lane < kGroup) {
+            const uint64_t act = __ballot(busy);
+            {
                 const float px = busy ? s.qx : 0.0f, py = busy ? s.qy : 0.0f, pz = busy ? s.qz : 0.0f;
                 const AxisW ax = axis_weights(px, r);
                 const AxisW ay = axis_weights(py, r);
                 const AxisW az = axis_weights(pz, r);
                 const float wxy00 = ax.w0 * ay.w0, wxy10 = ax.w1 * ay.w0;
                 const float wxy01 = ax.w0 * ay.w1, wxy11 = ax.w1 * ay.w1;
-                lds.base[n] = (uint32_t)((az.i0 * S + ay.i0) * S + ax.i0);
-                lds.w[n][0] = make_float4(wxy00 * az.w0, wxy10 * az.w0, wxy01 * az.w0, wxy11 * az.w0);
-                lds.w[n][1] = make_float4(wxy00 * az.w1, wxy10 * az.w1, wxy01 * az.w1, wxy11 * az.w1);
+                lds.base[lane] = (uint32_t)((az.i0 * S + ay.i0) * S + ax.i0);
+                lds.w[lane][0] = make_float4(wxy00 * az.w0, wxy10 * az.w0, wxy01 * az.w0, wxy11 * az.w0);
+                lds.w[lane][1] = make_float4(wxy00 * az.w1, wxy10 * az.w1, wxy01 * az.w1, wxy11 * az.w1);
                 if (!POSINV) {
-                    lds.pos[0][n] = px;
-                    lds.pos[1][n] = py;
-                    lds.pos[2][n] = pz;
+                    lds.pos[0][lane] = px;
+                    lds.pos[1][lane] = py;
+                    lds.pos[2][lane] = pz;
                 }
                 if (lane == 0) lds.act = act;
             }
         }
         __syncthreads();
-        const uint32_t act = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.act);
+        const uint64_t act = lds.act;
         if (act == 0) break;
-        {
-            const uint32_t query = threadIdx.x >> 3, q = threadIdx.x & 7u;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const uint32_t query = 32u * t + (threadIdx.x >> 3), q = threadIdx.x & 7u;
             if ((act >> query) & 1u) {
                 float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 float4 g[8];
@@ -403,24 +395,31 @@ __global__ __launch_bounds__(kGroupThreads, 4) void trace_mixed_pass2_group_kern
             }
         }
         __syncthreads();
-        {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const uint32_t query = 32u * t + n;
             bf16x8 b[3][2];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb)
-                    b[k][kb] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&lds.frag[k][half][n][4 * kb]));
+                    b[k][kb] =
+                        __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&lds.frag[k][half][query][4 * kb]));
             }
             const f32x16 c = split_tile(ah, am, al, b[0], b[1], b[2], bias_tile(h, half, &lds));
-            lds.part[h][lane] = layer2_partial(c, h, half, &lds, !POSINV, POSINV ? 0.0f : lds.pos[0][n],
-                                               POSINV ? 0.0f : lds.pos[1][n], POSINV ? 0.0f : lds.pos[2][n]);
+            lds.part[h][t][lane] =
+                layer2_partial(c, h, half, &lds, !POSINV, POSINV ? 0.0f : lds.pos[0][query],
+                               POSINV ? 0.0f : lds.pos[1][query], POSINV ? 0.0f : lds.pos[2][query]);
         }
         __syncthreads();
         if (owner) {
-            float p = 0.0f;
+            float p[2] = {0.0f, 0.0f};
 #pragma unroll
-            for (int k = 0; k < 4; ++k) p += lds.part[k][lane];
-            const float d = halves_sum(p, p) + b1;
+            for (int k = 0; k < 4; ++k) {
+                p[0] += lds.part[k][0][lane];
+                p[1] += lds.part[k][1][lane];
+            }
+            const float d = halves_sum(p[0], p[1]) + b1;
             if (s.phase != PH_IDLE) {
                 ++nevals;
                 s.consume(a, d);
@@ -432,66 +431,6 @@ __global__ __launch_bounds__(kGroupThreads, 4) void trace_mixed_pass2_group_kern
     }
     if (owner) add_evals(a, 0, nevals, lane);
 }
-
-// Pass 2 of frames of more than kPass2GroupRays rays, 64 a wave.
-// RETURNS: near misses may be handed back to a later pass 1 (not in the last
-// round); a separate instantiation, as for pass 1.
-template <bool POSINV, bool RETURNS>
-__global__ __launch_bounds__(kPass2Block, kMixedFp32Waves) void trace_mixed_pass2_kernel(TraceArgs a) {
-    __shared__ SplitLds lds;
-    __shared__ SoloLevels solo_lv;
-    stage_split_lds(a.m, a.dec, &lds);
-    stage_solo_levels(a.m, &solo_lv);
-    __syncthreads();
-    const float b1 = a.m.b1[a.dec][0];
-    const uint32_t lane = lane_id();
-    RayFeed feed;
-    feed.init(a.nrays, a.queue_stride);
-    RayState s;
-    s.ray = -1;
-    s.phase = PH_IDLE;
-    uint32_t nevals = 0;
-    const int coop = a.solo_lanes < kCoopLanes ? a.solo_lanes : kCoopLanes;
-    bool tail = false;
-    for (;;) {
-        const int64_t id = feed.next_flagged<true>(a.handoff_queue, a.hflag, lane, s.phase == PH_IDLE);
-        if (id >= 0) s.resume(a, a.handoff[id]);
-        const uint64_t act = __ballot(s.phase != PH_IDLE);
-        if (act == 0) break;
-        if (feed.drained && feed.fmask == 0 && __popcll(act) <= coop) {
-            tail = true;
-            break;
-        }
-        const bool busy = s.phase != PH_IDLE;
-        const float d = sdf_split_wave<POSINV>(a.m, &lds, b1, lane, busy, s.qx, s.qy, s.qz);
-        if (busy) {
-            ++nevals;
-            s.consume(a, d);
-            // hand back only a ray that moves away from the surface (step growing)
-            if (RETURNS && s.phase == PH_MARCH && fabsf(s.D) > a.return_dist && fabsf(s.D) > fabsf(s.Dp))
-                s.hand_off_to(a.ret, a.rflag);
-        }
-    }
-    // The wave's last few rays: the same steps with the gather spread over the
-    // idle lanes (same bits).  A separate loop, so that its registers do not
-    // weigh on the main loop's.
-    while (tail) {
-        const uint64_t act = __ballot(s.phase != PH_IDLE);
-        if (act == 0) break;
-        const bool busy = s.phase != PH_IDLE;
-        float f[kC];
-        gather_fp32_coop(&solo_lv, lane, act, s.qx, s.qy, s.qz, f);
-        const float d = decode_split_wave_few<POSINV>(f, &lds, b1, lane, busy, s.qx, s.qy, s.qz);
-        if (busy) {
-            ++nevals;
-            s.consume(a, d);
-            if (RETURNS && s.phase == PH_MARCH && fabsf(s.D) > a.return_dist && fabsf(s.D) > fabsf(s.Dp))
-                s.hand_off_to(a.ret, a.rflag);
-        }
-    }
-    add_evals(a, 0, nevals, lane);
-}
-
 
 // ---------------------------------------------------------------------------
 // Pooled trace: the rays of several requests (each its own model and LOD) in
@@ -878,18 +817,6 @@ static int grid_for(K kernel, int64_t n, int block) {
     return (int)(want < cap ? (want < 1 ? 1 : want) : cap);
 }
 
-template <bool POSINV, bool RETURNS>
-static void launch_pass2(const TraceArgs& a, int64_t n, hipStream_t s) {
-    if (n <= kPass2GroupRays) {
-        const int64_t blocks = (n + kGroup - 1) / kGroup, cap = (int64_t)device_cu_count() * 4;
-        hipLaunchKernelGGL((trace_mixed_pass2_group_kernel<POSINV, RETURNS>), dim3((unsigned)(blocks < cap ? blocks : cap)),
-                           dim3(kGroupThreads), 0, s, a);
-    } else {
-        const int blocks = grid_for(trace_mixed_pass2_kernel<POSINV, RETURNS>, n, kPass2Block);
-        hipLaunchKernelGGL((trace_mixed_pass2_kernel<POSINV, RETURNS>), dim3(blocks), dim3(kPass2Block), 0, s, a);
-    }
-}
-
 __global__ void clear_words_kernel(uint32_t* p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0u;
@@ -916,6 +843,8 @@ template <bool POSINV>
 static int trace_mixed_rounds(TraceArgs a, int64_t n, hipStream_t s, PassTimer& timer) {
     const int g1 = grid_for(trace_mixed_pass1_kernel<POSINV, false>, n, kMixedBlock);
     const int g1r = grid_for(trace_mixed_pass1_kernel<POSINV, true>, n, kMixedBlock);
+    const int64_t want2 = (n + kPass2Rays - 1) / kPass2Rays, cap2 = (int64_t)device_cu_count() * 4;
+    const unsigned g2 = (unsigned)(want2 < cap2 ? want2 : cap2);
     const int words = (int)((n + 3) / 4);
     const dim3 cg((unsigned)((words + 255) / 256));
     const int rounds = a.return_dist > 0.0f ? kMixedRounds : 1;
@@ -942,9 +871,9 @@ static int trace_mixed_rounds(TraceArgs a, int64_t n, hipStream_t s, PassTimer& 
             timer.mark(kPassOther);
         }
         if (allow_return)
-            launch_pass2<POSINV, true>(a2, n, s);
+            hipLaunchKernelGGL((trace_mixed_pass2_kernel<POSINV, true>), dim3(g2), dim3(kGroupThreads), 0, s, a2);
         else
-            launch_pass2<POSINV, false>(a2, n, s);
+            hipLaunchKernelGGL((trace_mixed_pass2_kernel<POSINV, false>), dim3(g2), dim3(kGroupThreads), 0, s, a2);
         rc = check_launch("trace_mixed_pass2_kernel");
         if (rc) return rc;
         timer.mark(kPassFp32);

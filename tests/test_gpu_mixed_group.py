@@ -1,6 +1,6 @@
-"""The mixed trace's FP32 pass by groups of 32 rays (up to 2^20 rays) against the
-one with 64 rays a wave (above): a ray's result does not depend on the others, so
-the rays of a small batch have the same bits when they are part of a large one."""
+"""The mixed trace's FP32 pass, a block of four waves per 64 rays: a ray's result
+does not depend on the others, so the rays of a small batch (part-filled groups)
+have the same bits when they are part of one that fills the GPU."""
 import pytest
 import torch
 
