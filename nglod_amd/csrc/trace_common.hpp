@@ -86,8 +86,8 @@ struct TraceArgs {
     float return_dist;        // FP32 step length above which a ray goes back to mixed
     int defer_normals;        // 0: a finished hit takes its normal taps in-lane; 1: it is handed to the FP32
                               // pass (hand-off record in phase PH_N0), which takes the taps
-    int solo_lanes;           // mixed passes: a wave with no rays left to claim and at most min(this, 4) busy
-                              // lanes (pass 1: 8 unless 0) spreads their gathers over the idle lanes
+    int solo_lanes;           // pooled passes: a wave with no rays left to claim and at most min(this, 4) busy
+                              // lanes (pass 1 of a frame: 8 unless 0) spreads their gathers over the idle lanes
     int64_t nrays;  // the frame is split into kQueues ranges [nrays*q/kQueues, nrays*(q+1)/kQueues)
 };
 
