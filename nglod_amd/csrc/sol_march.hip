@@ -288,9 +288,13 @@ __global__ __launch_bounds__(kGroupThreads, 4) void trace_sparse_group_kernel(So
         // the next trip's).  Block-uniform: every wave sees the same phases.
         const uint32_t need = (uint32_t)__ballot(s.phase == SG_IDLE);
         if (need != 0 && !(drained && next >= queued)) {
-            if (next >= queued) {
-                if (first) group_claim(a, &lds, feed, lane);
-                __syncthreads();
+            const bool claims = next >= queued;
+            if (claims && first) group_claim(a, &lds, feed, lane);
+            // Wave 0 starts a ray by writing its origin, direction and list; until this
+            // barrier another wave may still be moving the lane's last ray by the old ones
+            // (consume in the last trip, walked in a trip that ended without an evaluation).
+            __syncthreads();
+            if (claims) {
                 next = 0;
                 queued = lds.queued;
                 drained = lds.drained != 0;
