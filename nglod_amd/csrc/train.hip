@@ -609,23 +609,29 @@ __device__ __forceinline__ float piece_of(const float* grad, const float* partia
     return p == 0 ? grad[c] : partial[(size_t)((first + p * kRunPiece) / kRunPiece) * kC + c];
 }
 
-// One thread per (corner, channel): sums the run's pieces in order.
+// A thread per (corner, channel) and turn: sums the run's pieces in order.  The
+// grid is capped: 8 levels of up to 512^3 cells are 4.9e9 (corner, channel) pairs,
+// and a launch holds fewer than 2^32 threads.
+constexpr uint32_t kFinalBlocks = 1u << 20;
+static_assert((uint64_t)kFinalBlocks * 256 < ((uint64_t)1 << 32), "threads of a launch");
+
 __global__ __launch_bounds__(256) void bwd_run_final_kernel(CornerLevels L, const uint2* __restrict__ runs,
                                                             const float* __restrict__ partial) {
-    const uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    const uint32_t k = (uint32_t)(t / kC);
-    const int c = (int)(t % kC);
-    if (k >= L.base[L.count]) return;
-    const uint2 run = runs[k];
-    const uint32_t cnt = run.y - run.x;
-    if (cnt <= (uint32_t)kRunPiece) return;
-    const int li = level_of(L, k);
-    if ((L.strided >> li) & 1u) return;
-    float* grad = L.grad[li] + (size_t)(k - L.base[li]) * kC;
-    const uint32_t np = (cnt + kRunPiece - 1) / kRunPiece;
-    float s = 0.0f;
-    for (uint32_t p = 0; p < np; ++p) s += piece_of(grad, partial, run.x, p, c);
-    grad[c] = s;
+    const uint64_t end = (uint64_t)L.base[L.count] * kC;
+    for (uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x; t < end; t += (uint64_t)gridDim.x * 256) {
+        const uint32_t k = (uint32_t)(t / kC);
+        const int c = (int)(t % kC);
+        const uint2 run = runs[k];
+        const uint32_t cnt = run.y - run.x;
+        if (cnt <= (uint32_t)kRunPiece) continue;
+        const int li = level_of(L, k);
+        if ((L.strided >> li) & 1u) continue;
+        float* grad = L.grad[li] + (size_t)(k - L.base[li]) * kC;
+        const uint32_t np = (cnt + kRunPiece - 1) / kRunPiece;
+        float s = 0.0f;
+        for (uint32_t p = 0; p < np; ++p) s += piece_of(grad, partial, run.x, p, c);
+        grad[c] = s;
+    }
 }
 
 // The same sums for levels whose runs hold many pieces (the coarse grids:
@@ -633,15 +639,23 @@ __global__ __launch_bounds__(256) void bwd_run_final_kernel(CornerLevels L, cons
 // kRunGroups x kC threads per run; thread (g, c) sums pieces g, g + kRunGroups,
 // ... of channel c in order (a row of kC partials is one coalesced load for
 // the block's 32 channels), then thread (0, c) adds the kRunGroups group sums
-// in group order.  A fixed order, so the result is the same every run.
+// in group order.  A fixed order, so the result is the same every run.  A
+// strided level has at most n / 64 corners, so all of them below 2^22 blocks.
 constexpr int kRunGroups = 8;
 
 __global__ __launch_bounds__(kRunGroups * kC) void bwd_run_strided_kernel(CornerLevels L, const uint2* __restrict__ runs,
                                                                           const float* __restrict__ partial) {
     __shared__ float gs[kRunGroups][kC];
-    const uint32_t k = blockIdx.x;
-    const int li = level_of(L, k);
-    if (!((L.strided >> li) & 1u)) return;  // block-uniform
+    // block b: corner b of the strided levels, counted through them alone
+    uint32_t k = blockIdx.x;
+    int li = 0;
+    for (;; ++li) {
+        if (!((L.strided >> li) & 1u)) continue;
+        const uint32_t corners = L.base[li + 1] - L.base[li];
+        if (k < corners) break;
+        k -= corners;
+    }
+    k += L.base[li];
     const uint2 run = runs[k];
     const uint32_t cnt = run.y - run.x;
     if (cnt == 0) return;
@@ -972,13 +986,15 @@ static int backward(const nglod_model_t* model, const float* x, int64_t n, int32
         const uint32_t windows = (mm + size - 1) / size;
         hipLaunchKernelGGL(bwd_pieces_kernel, dim3((windows + 7) / 8 * 8), dim3(256), 0, s, a, C, kout, vout, mm, size,
                            runs, partial);
-        if (C.strided != (1u << C.count) - 1u)
-            hipLaunchKernelGGL(bwd_run_final_kernel, dim3((unsigned)(((uint64_t)corners * kC + 255) / 256)), dim3(256),
-                               0, s, C, runs, partial);
+        if (C.strided != (1u << C.count) - 1u) {
+            const uint64_t blocks = ((uint64_t)corners * kC + 255) / 256;
+            hipLaunchKernelGGL(bwd_run_final_kernel, dim3((unsigned)(blocks < kFinalBlocks ? blocks : kFinalBlocks)),
+                               dim3(256), 0, s, C, runs, partial);
+        }
         if (C.strided) {
-            uint32_t last = 0;
-            for (int i = 0; i < C.count; ++i) last = (C.strided >> i) & 1u ? C.base[i + 1] : last;
-            hipLaunchKernelGGL(bwd_run_strided_kernel, dim3(last), dim3(kRunGroups * kC), 0, s, C, runs, partial);
+            uint32_t blocks = 0;
+            for (int i = 0; i < C.count; ++i) blocks += (C.strided >> i) & 1u ? C.base[i + 1] - C.base[i] : 0u;
+            hipLaunchKernelGGL(bwd_run_strided_kernel, dim3(blocks), dim3(kRunGroups * kC), 0, s, C, runs, partial);
         }
         return check_launch("bwd_pieces_kernel");
     };
