@@ -717,12 +717,12 @@ static uint64_t corners_of(int r) { return (uint64_t)(r + 1) * (r + 1) * (r + 1)
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// One sort of all levels' contributions while they can be numbered with 32
-// bits, else a sort per level.  Fewer launches against more sorting passes
-// over a level's contributions: a training step takes 1.35 ms against 1.48
-// with 512 queries and 5 levels, 1.43 against 1.70 with 2^16, 3.14 against 3.17
-// with 2^19.
-constexpr int64_t kTogether = (int64_t)1 << 31;
+// One sort of all levels' contributions up to this many, else a sort per level:
+// fewer launches against more sorting passes over a level's contributions (and
+// buffers of one level's size).  Steps in us, together / per level: 3 levels 774 / 867 with
+// 2^18 queries, 1353 / 1398 with 2^19, 2647 / 2628 with 2^20 (3 << 23 contributions), 10870 /
+// 10520 with 2^22; 5 levels 1381 / 1509, 2384 / 2388, 4614 / 4428, 18740 / 17190.
+constexpr int64_t kTogether = (int64_t)3 << 23;
 
 static void saved_layout(int64_t n, int lod, SavedLayout* L) {
     const size_t levels = (size_t)lod + 1;
@@ -757,7 +757,7 @@ static int bwd_layout(int64_t n, int lod, int din, const int32_t* res, bool save
         corners += corners_of(res[l]);
         most = corners_of(res[l]) > most ? corners_of(res[l]) : most;
     }
-    L->together = (int64_t)levels * n * 8 <= kTogether && corners < ((uint64_t)1 << 31);
+    L->together = (int64_t)levels * n * 8 < kTogether && corners < ((uint64_t)1 << 31);
     const size_t m = (size_t)n * 8 * (L->together ? levels : 1);
     SavedLayout S;
     saved_layout(n, lod, &S);

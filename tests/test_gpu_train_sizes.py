@@ -112,6 +112,22 @@ def test_levels_in_any_order(dev, res, n):
             _close(got, want, "decoder")
 
 
+@pytest.mark.parametrize("n", [390000, 393216, 400001])
+def test_one_sort_or_a_sort_per_level(dev, n):
+    """Eight levels: below 393216 queries one sort of all contributions, from there on a sort per
+    level, on the same buffers one after the other."""
+    res = [4, 2, 8, 16, 64, 32, 1, 24]
+    g = torch.Generator().manual_seed(n)
+    x = (torch.rand(n, 3, generator=g) * 2 - 1).to(dev)
+    levels, decs = _backward(res, x, 4)
+    for r, (used, got, want, grad) in zip(res, levels):
+        _close(got, want, r)
+        assert torch.isin((grad != 0).any(1).nonzero()[:, 0], used).all()
+    for d in decs:
+        for got, want in d:
+            _close(got, want, "decoder")
+
+
 @pytest.mark.parametrize("num_lods", [6, 7, 8])
 @pytest.mark.parametrize("pos_invariant", [True, False])
 @pytest.mark.parametrize("n", [500, 20000])
