@@ -11,15 +11,33 @@ from . import _lib
 
 
 def _param_slots(net, params):
-    """(kind, index) of each parameter; (None, -1) for one the kernels do not read."""
-    slots = {id(f.fm): ("grid", i) for i, f in enumerate(net.features)}
+    """(kind, index) of each parameter; (None, -1) for one outside the grids and
+    decoders.  Found by identity; one that is not read as it is (a grid's under a
+    parametrization or a pruning mask) by its name, as its level's grid.  A decoder's
+    raises: the gradient is that of the weight it is turned into."""
+    slots = {}
+    for i, f in enumerate(net.features):
+        slots.setdefault(id(f.fm), ("grid", i))
     for i, l in enumerate(net.louts):
         first, _, last = l
-        slots[id(first.weight)] = ("w0", i)
-        slots[id(first.bias)] = ("b0", i)
-        slots[id(last.weight)] = ("w1", i)
-        slots[id(last.bias)] = ("b1", i)
-    return [slots.get(id(p), (None, -1)) for p in params]
+        slots.setdefault(id(first.weight), ("w0", i))
+        slots.setdefault(id(first.bias), ("b0", i))
+        slots.setdefault(id(last.weight), ("w1", i))
+        slots.setdefault(id(last.bias), ("b1", i))
+    found = [slots.get(id(p)) for p in params]
+    if None in found:
+        names = {id(p): name for name, p in net.named_parameters()}
+        found = [s if s is not None else _slot_of(names[id(p)]) for s, p in zip(found, params)]
+    return found
+
+
+def _slot_of(name):
+    parts = name.split(".")
+    if parts[0] == "features":
+        return "grid", int(parts[1])
+    if parts[0] == "louts":
+        raise KeyError(f"no gradient for {name}: not a weight or bias of its decoder")
+    return None, -1
 
 
 # The forward of every level keeps its features for the backward (164 bytes per
