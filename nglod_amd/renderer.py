@@ -43,8 +43,9 @@ def _on_device(rows, device):
     """FP32 tensors of rows of numbers.  To the GPU by one asynchronous copy from
     pinned memory: a copy from pageable memory waits for the stream, that is for
     the frame before."""
-    if (torch.device(device).type == "cuda" and all(type(r) in (list, tuple) and len(r) == len(rows[0]) and
-                                                    all(isinstance(v, (int, float)) for v in r) for r in rows)
+    if (device is not None and torch.device(device).type == "cuda"
+            and all(type(r) in (list, tuple) and len(r) == len(rows[0]) and
+                    all(isinstance(v, (int, float)) for v in r) for r in rows)
             and not torch.cuda.is_current_stream_capturing()):
         host = torch.tensor(rows, dtype=torch.float32, pin_memory=True)
         return host.to(device, non_blocking=True).unbind(0)
