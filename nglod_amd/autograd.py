@@ -40,8 +40,11 @@ def _slot_of(name):
     return None, -1
 
 
-# The forward of every level keeps its features for the backward (164 bytes per
-# query and level) up to this many bytes; a larger batch computes them again.
+# A forward of every level whose caller runs the backward itself, with nothing in
+# between, keeps its features for it (164 bytes per query and level) up to this many
+# bytes; a larger batch computes them again, and so does any other backward: a
+# program may write the weights in between, and a write through .data leaves no mark
+# to know it by.
 SAVE_LIMIT = 4 << 30
 
 
@@ -51,7 +54,7 @@ def _versions(params):
 
 class _SdfFunction(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, net, x, lod, all_levels, *params):
+    def forward(ctx, net, x, lod, all_levels, keep_features, *params):
         ctx.net = net
         ctx.lod = lod
         ctx.all_levels = all_levels
@@ -59,7 +62,7 @@ class _SdfFunction(torch.autograd.Function):
         ctx.x_shape = x.shape
         ctx.x_dtype = x.dtype
         n = xf.shape[0]
-        if all_levels and n > 0 and any(ctx.needs_input_grad[4:]):
+        if keep_features and all_levels and n > 0 and any(ctx.needs_input_grad[5:]):
             lib = _lib.load()
             m = net.descriptor(_lib.FP32)
             nbytes = lib.nglod_sdf_fwd_save_bytes(m, n, lod)
@@ -99,8 +102,8 @@ class _SdfFunction(torch.autograd.Function):
                 if (mask >> lvl) & 1:
                     grad_x.addcmul_(g[lvl][:, None], net.sdf_grad_hip(x, lvl)[1])
             grad_x = grad_x.to(ctx.x_dtype).reshape(ctx.x_shape)
-        if not any(ctx.needs_input_grad[4:]):
-            return (None, grad_x, None, None, *([None] * len(ctx.needs_input_grad[4:])))
+        if not any(ctx.needs_input_grad[5:]):
+            return (None, grad_x, None, None, None, *([None] * len(ctx.needs_input_grad[5:])))
         used_dec = {0} if net.num_decoder == 1 else {i for i in range(L + 1) if (mask >> i) & 1}
         G = _lib.NglodModelGrads()
         out = {}
@@ -137,15 +140,16 @@ class _SdfFunction(torch.autograd.Function):
                 grads.append(out[(kind, idx)])
             else:
                 grads.append(None)
-        return (None, grad_x, None, None, *grads)
+        return (None, grad_x, None, None, None, *grads)
 
 
-def sdf_with_grad(net, x, lod, all_levels, stacked=False, params=None):
+def sdf_with_grad(net, x, lod, all_levels, stacked=False, params=None, keep_features=False):
     """stacked: the levels' predictions as one [lod + 1, n, 1] tensor; params:
-    net's parameters, if the caller has them."""
+    net's parameters, if the caller has them; keep_features: the caller runs the
+    backward before anything can write the weights."""
     if params is None:
         params = _lib.parameter_list(net)
-    out = _SdfFunction.apply(net, x, lod, all_levels, *params)
+    out = _SdfFunction.apply(net, x, lod, all_levels, keep_features, *params)
     if all_levels and not stacked:
         return [out[i] for i in range(out.shape[0])]
     return out

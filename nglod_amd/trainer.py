@@ -54,7 +54,8 @@ class Trainer:
                 p.grad = None
         batch_size = pts.shape[0]
         if self._fused(pts, gts, params):
-            stacked = sdf_with_grad(net, pts, net.num_lods - 1, all_levels=True, stacked=True, params=params)
+            stacked = sdf_with_grad(net, pts, net.num_lods - 1, all_levels=True, stacked=True, params=params,
+                                    keep_features=True)
             net.loss_preds = list(stacked.unbind(0))
             gt = gts.contiguous()
             grad = torch.empty_like(stacked)
