@@ -51,14 +51,16 @@ struct AdamArgs {
     int64_t n[kAdamTensors];
     uint32_t first[kAdamTensors + 1];
     int count;
-    float w1, beta2, w2, bias2_sqrt, eps, step;
+    float w1, w1_rest, beta2, w2, bias2_sqrt, eps, step;
 };
 
 // One element, rounding as torch's multi-tensor Adam on this GPU does (checked
-// bit for bit): m by an FMA (lerp), v = fma(1 - beta2, g g, v beta2), the update
-// p = fma(-lr / bias1, m / (sqrt(v) / bias2_sqrt + eps), p).
+// bit for bit): m by an FMA (lerp, which starts from the nearer end: beta1 = 0 gives g
+// itself), v = fma(1 - beta2, g g, v beta2), the update p = fma(-lr / bias1, m /
+// (sqrt(v) / bias2_sqrt + eps), p).
 __device__ __forceinline__ void adam_one(const AdamArgs& a, float& p, float g, float& m, float& v) {
-    m = __builtin_fmaf(a.w1, g - m, m);
+    const float d1 = g - m;
+    m = a.w1 < 0.5f ? __builtin_fmaf(a.w1, d1, m) : __builtin_fmaf(-d1, a.w1_rest, g);
     v = __builtin_fmaf(a.w2, g * g, v * a.beta2);
     const float d = sqrtf(v) / a.bias2_sqrt + a.eps;
     p = __builtin_fmaf(a.step, m / d, p);
@@ -136,6 +138,7 @@ int nglod_adam_step(float* const* p, const float* const* g, float* const* m, flo
     if (count > 0 && (!p || !g || !m || !v || !n)) return fail(NGLOD_ERR_ARG, "NULL pointer");
     AdamArgs a;
     a.w1 = (float)(1.0 - beta1);
+    a.w1_rest = 1.0f - a.w1;
     a.beta2 = (float)beta2;
     a.w2 = (float)(1.0 - beta2);
     a.bias2_sqrt = (float)pow(1.0 - pow(beta2, (double)step), 0.5);
