@@ -35,8 +35,9 @@ class Trainer:
         OctreeSDF's every-level predictions against one FP32 value per point."""
         net = self.net
         return (type(net) is OctreeSDF and "sdf" not in net.__dict__ and net.lod is None and pts.dim() == 2
-                and pts.is_cuda and pts.shape[0] > 0 and torch.is_tensor(gts) and gts.shape == (pts.shape[0], 1) and gts.dtype == torch.float32
-                and gts.device == pts.device and not gts.requires_grad and torch.is_grad_enabled()
+                and pts.is_cuda and pts.shape[0] > 0 and torch.is_tensor(gts) and gts.shape == (pts.shape[0], 1)
+                and gts.dtype == torch.float32 and gts.device == pts.device and not gts.requires_grad
+                and torch.is_grad_enabled()
                 and all(0 <= i < net.num_lods for i in self.loss_lods)
                 and len(set(self.loss_lods)) == len(self.loss_lods) > 0
                 and all(p.requires_grad for p in params))
