@@ -3,16 +3,17 @@
 //
 // The distance is the minimum over the triangles, and a point is inside iff
 // each of 13 lines through it meets a triangle on both sides.  Both need few
-// of the triangles, so each call sorts the triangles along a Morton curve and
-// builds a tree of boxes over them (8 children per node, consecutive in that
-// order).  Boxes are FP32 and wide enough for every rounding of the FP64 tests
-// below them, so the triangles that are skipped could not have changed a
-// result: the distance is the same minimum over the same FP64 values and the
-// flags are the same flags as those of a loop over all triangles.
+// of the triangles, so a call of more than a few pairs (pair_lanes) sorts the
+// triangles along a Morton curve and builds a tree of boxes over them (8
+// children per node, consecutive in that order).  Boxes are FP32 and wide
+// enough for every rounding of the FP64 tests below them, so the triangles
+// that are skipped could not have changed a result: the distance is the same
+// minimum over the same FP64 values and the flags are the same flags as those
+// of a loop over all triangles.
 //
 // 2^19 points (a third uniform in the box, the rest near the surface) and 5120
-// triangles: 2.2 ms, of it 0.10 ms for the tree, 0.08 ms for the order of the
-// points, 0.84 ms for the distances and 1.32 ms for the lines; 30.3 ms with
+// triangles: 2.25 ms, of it 0.10 ms for the tree, 0.08 ms for the order of the
+// points, 0.77 ms for the distances and 1.31 ms for the lines; 30.3 ms with
 // every point against every triangle (FP64 issue, 2.7 G pairs).
 #include "api_common.hpp"
 #include "radix_sort.hpp"
@@ -103,6 +104,50 @@ __device__ __forceinline__ double d2axmb(const double* a, double x, const double
     NGLOD_FP64_CONTRACT
     const double t0 = a[0] * x - b[0], t1 = a[1] * x - b[1], t2 = a[2] * x - b[2];
     return t0 * t0 + t1 * t1 + t2 * t2;
+}
+
+// The two records of a triangle (its nine floats), and its longest edge's square and
+// 1 / its smallest determinant that is not taken for 0.
+struct TriScale {
+    double ee, worst;
+};
+
+__device__ __forceinline__ TriScale tri_records(const float* t, TriNear& N, TriLine& L) {
+    NGLOD_FP64_CONTRACT
+    double A[3], B[3], C[3], v10[3], v21[3], v02[3], nor[3];
+    for (int k = 0; k < 3; ++k) {
+        A[k] = t[k];
+        B[k] = t[3 + k];
+        C[k] = t[6 + k];
+    }
+    for (int k = 0; k < 3; ++k) {
+        v10[k] = B[k] - A[k];
+        v21[k] = C[k] - B[k];
+        v02[k] = A[k] - C[k];
+    }
+    cross3(v10, v02, nor);
+    for (int k = 0; k < 9; ++k) N.v[k] = t[k];
+    N.i10 = 1.0 / dot3(v10, v10);
+    N.i21 = 1.0 / dot3(v21, v21);
+    N.i02 = 1.0 / dot3(v02, v02);
+    N.inor = 1.0 / dot3(nor, nor);
+    N.degenerate = (nor[0] == 0.0 && nor[1] == 0.0 && nor[2] == 0.0) ? 1u : 0u;
+    for (int k = 0; k < 3; ++k) {
+        L.a[k] = A[k];
+        L.v10[k] = v10[k];
+        L.e2[k] = -v02[k];
+    }
+    TriScale s;
+    s.worst = 0.0;
+    for (int i = 0; i < kDirs; ++i) {
+        const double dir[3] = {kStab[i][0], kStab[i][1], kStab[i][2]};
+        cross3(dir, L.e2, L.dir[i].pvec);
+        const double det = dot3(v10, L.dir[i].pvec);
+        L.dir[i].idet = (det > -1e-8 && det < 1e-8) ? 0.0 : 1.0 / det;
+        s.worst = fmax(s.worst, fabs(L.dir[i].idet));
+    }
+    s.ee = fmax(dot3(v10, v10), fmax(dot3(v21, v21), dot3(v02, v02)));
+    return s;
 }
 
 // ---------------------------------------------------------------------------
@@ -303,53 +348,22 @@ __global__ __launch_bounds__(128) void tri_prep_kernel(const float* __restrict__
         return;
     }
     const float* t = mesh + 9 * (size_t)order[s];
-    double A[3], B[3], C[3], v10[3], v21[3], v02[3], nor[3];
-    for (int k = 0; k < 3; ++k) {
-        A[k] = t[k];
-        B[k] = t[3 + k];
-        C[k] = t[6 + k];
-    }
-    for (int k = 0; k < 3; ++k) {
-        v10[k] = B[k] - A[k];
-        v21[k] = C[k] - B[k];
-        v02[k] = A[k] - C[k];
-    }
-    cross3(v10, v02, nor);
     TriNear N;
-    for (int k = 0; k < 9; ++k) N.v[k] = t[k];
-    N.i10 = 1.0 / dot3(v10, v10);
-    N.i21 = 1.0 / dot3(v21, v21);
-    N.i02 = 1.0 / dot3(v02, v02);
-    N.inor = 1.0 / dot3(nor, nor);
-    N.degenerate = (nor[0] == 0.0 && nor[1] == 0.0 && nor[2] == 0.0) ? 1u : 0u;
-    near[s] = N;
     TriLine L;
-    for (int k = 0; k < 3; ++k) {
-        L.a[k] = A[k];
-        L.v10[k] = v10[k];
-        L.e2[k] = -v02[k];
-    }
-    double worst = 0.0;  // 1 / the smallest determinant
-    for (int i = 0; i < kDirs; ++i) {
-        const double dir[3] = {kStab[i][0], kStab[i][1], kStab[i][2]};
-        cross3(dir, L.e2, L.dir[i].pvec);
-        const double det = dot3(v10, L.dir[i].pvec);
-        L.dir[i].idet = (det > -1e-8 && det < 1e-8) ? 0.0 : 1.0 / det;
-        worst = fmax(worst, fabs(L.dir[i].idet));
-    }
+    const TriScale sc = tri_records(t, N, L);
+    near[s] = N;
     line[s] = L;
     float S = 0.0f, diag = 0.0f;
     for (int k = 0; k < 3; ++k) {
         S = fmaxf(S, fmaxf(fabsf(bd.lo[k]), fabsf(bd.hi[k])));
         diag += bd.hi[k] - bd.lo[k];
     }
-    const double ee = fmax(dot3(v10, v10), fmax(dot3(v21, v21), dot3(v02, v02)));
-    const float pad = 4e-6f * S + (float)(6e-15 * worst * ee * (sqrt(ee) + (double)diag));
+    const float pad = 4e-6f * S + (float)(6e-15 * sc.worst * sc.ee * (sqrt(sc.ee) + (double)diag));
     float va[kForms], vb[kForms], vc[kForms];
     point_forms(t[0], t[1], t[2], va);
     point_forms(t[3], t[4], t[5], vb);
     point_forms(t[6], t[7], t[8], vc);
-    bool finite = fabsf(pad) < INFINITY && 6.7e-16 * worst * ee < 0.25;
+    bool finite = fabsf(pad) < INFINITY && 6.7e-16 * sc.worst * sc.ee < 0.25;
     for (int k = 0; k < 9; ++k) finite &= fabsf(t[k]) < INFINITY;
     Slabs& sl = slabs[s >> 3];
     for (int k = 0; k < kForms; ++k) {
@@ -424,24 +438,16 @@ __global__ __launch_bounds__(1024) void tree_top_kernel(Tree t, int l0) {
 }
 
 // ---------------------------------------------------------------------------
-// Squared distance from p to triangle T by the reference's edge/face rule,
-// with the FP64 operations of the whole-mesh loop; INFINITY for a degenerate
-// triangle, NaN where the arithmetic gives it (the minimum drops both).
-__device__ __forceinline__ double tri_dist2(const TriNear& T, const double* p) {
+// Squared distance from p (p0 = p - the first vertex) to a triangle by the
+// reference's edge/face rule, with the FP64 operations of a loop over the whole mesh.
+// T: its vertices and reciprocals.
+template <typename Tri>
+__device__ __forceinline__ double edge_face_dist2(const Tri& T, const double* p0, const double* p, const double* v10,
+                                                  const double* v21, const double* v02, const double* nor,
+                                                  const double* c10, const double* c21, const double* c02) {
     NGLOD_FP64_CONTRACT
-    if (T.degenerate) return INFINITY;
-    const double A[3] = {T.v[0], T.v[1], T.v[2]}, B[3] = {T.v[3], T.v[4], T.v[5]}, C[3] = {T.v[6], T.v[7], T.v[8]};
-    const double v10[3] = {B[0] - A[0], B[1] - A[1], B[2] - A[2]};
-    const double v21[3] = {C[0] - B[0], C[1] - B[1], C[2] - B[2]};
-    const double v02[3] = {A[0] - C[0], A[1] - C[1], A[2] - C[2]};
-    const double p0[3] = {p[0] - A[0], p[1] - A[1], p[2] - A[2]};
-    const double p1[3] = {p[0] - B[0], p[1] - B[1], p[2] - B[2]};
-    const double p2[3] = {p[0] - C[0], p[1] - C[1], p[2] - C[2]};
-    double nor[3], c10[3], c21[3], c02[3];
-    cross3(v10, v02, nor);
-    cross3(v10, nor, c10);
-    cross3(v21, nor, c21);
-    cross3(v02, nor, c02);
+    const double p1[3] = {p[0] - T.v[3], p[1] - T.v[4], p[2] - T.v[5]};
+    const double p2[3] = {p[0] - T.v[6], p[1] - T.v[7], p[2] - T.v[8]};
     const double s = copysign(1.0, dot3(c10, p0)) + copysign(1.0, dot3(c21, p1)) + copysign(1.0, dot3(c02, p2));
     double d2;
     if (s < 2.0) {
@@ -454,6 +460,24 @@ __device__ __forceinline__ double tri_dist2(const TriNear& T, const double* p) {
         d2 = dn * dn * T.inor;
     }
     return d2 < 0.0 ? 0.0 : d2;
+}
+
+// The distance for a triangle of the tree; INFINITY for a degenerate
+// triangle, NaN where the arithmetic gives it (the minimum drops both).
+__device__ __forceinline__ double tri_dist2(const TriNear& T, const double* p) {
+    NGLOD_FP64_CONTRACT
+    if (T.degenerate) return INFINITY;
+    const double A[3] = {T.v[0], T.v[1], T.v[2]}, B[3] = {T.v[3], T.v[4], T.v[5]}, C[3] = {T.v[6], T.v[7], T.v[8]};
+    const double v10[3] = {B[0] - A[0], B[1] - A[1], B[2] - A[2]};
+    const double v21[3] = {C[0] - B[0], C[1] - B[1], C[2] - B[2]};
+    const double v02[3] = {A[0] - C[0], A[1] - C[1], A[2] - C[2]};
+    double nor[3], c10[3], c21[3], c02[3];
+    cross3(v10, v02, nor);
+    cross3(v10, nor, c10);
+    cross3(v21, nor, c21);
+    cross3(v02, nor, c02);
+    const double p0[3] = {p[0] - A[0], p[1] - A[1], p[2] - A[2]};
+    return edge_face_dist2(T, p0, p, v10, v21, v02, nor, c10, c21, c02);
 }
 
 // The bound a box must beat, from the best squared distance so far: FP32
@@ -490,7 +514,7 @@ constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kMirror8 = 0x141, kRotate8 = 0x128;
 // nearest on top; an entry that no point needs any more is dropped unvisited.
 // The vector memory path bounds it: a node is two 16-byte loads and a triangle
 // five (1.11 ms with a load per bound and the products of the edges stored,
-// 0.84 ms so, 2^19 points and 5120 triangles).
+// 0.77 ms so, 2^19 points and 5120 triangles).
 //
 // 64 points per wave against one child after another (wave-uniform, no
 // divergence) took 4.1 ms instead: a few waves, those of points in the middle
@@ -580,7 +604,7 @@ __device__ __forceinline__ u16x2_t as_u16x2(uint32_t w) { return __builtin_bit_c
 // sides have a hit.  Lanes of their own follow their lines' few nodes: a wave
 // that walks its 64 points' 13 lines together enters the union of them.  The
 // group loads bound it (vector memory path): 16-bit intervals halve them
-// against FP32 ones (1.76 -> 1.32 ms at 2^19 points, 5120 triangles).
+// against FP32 ones (1.76 -> 1.31 ms at 2^19 points, 5120 triangles).
 struct LineStack {
     uint32_t group[kMaxLevels][256];
     uint32_t mask[kMaxLevels][256];
@@ -700,6 +724,107 @@ __global__ __launch_bounds__(256) void mesh_sign_kernel(const float* __restrict_
 }
 
 // ---------------------------------------------------------------------------
+// Every point against every triangle, for few of either: no order, no tree, two
+// launches.  `lanes` lanes of a wave take a point, each every lanes-th triangle of a
+// tile in LDS; the minimum and the flags do not depend on the order.
+//
+// Bound: FP64 issue (11 ps a pair) where the points fill the GPU, else the chain of a
+// lane's triangles (2.4 us each).  The tree's sorts and levels cost 100 us and more before
+// its first triangle: 12 triangles and 10^4 points 158 us by the tree, 16 so.
+struct PairTri {
+    float v[9];
+    uint32_t degenerate;
+    double v10[3], v02[3], nor[3], c10[3], c21[3], c02[3], i10, i21, i02, inor;
+    double pvec[kDirs][3], idet[kDirs];
+};
+constexpr int kPairTile = 64, kPairWords = sizeof(PairTri) / 8, kPairStride = kPairWords + 1;  // odd: over the banks
+// the records take the place of the tree's
+static_assert(8 * sizeof(PairTri) <= 8 * (sizeof(TriNear) + sizeof(TriLine) + sizeof(Box)) + sizeof(Slabs), "room");
+
+__global__ __launch_bounds__(128) void pair_records_kernel(const float* __restrict__ mesh, uint32_t nf,
+                                                           PairTri* __restrict__ out) {
+    NGLOD_FP64_CONTRACT
+    const uint32_t f = blockIdx.x * 128 + threadIdx.x;
+    if (f >= nf) return;
+    TriNear N;
+    TriLine L;
+    tri_records(mesh + 9 * (size_t)f, N, L);
+    PairTri T;
+    for (int k = 0; k < 9; ++k) T.v[k] = N.v[k];
+    T.degenerate = N.degenerate;
+    double v21[3];
+    for (int k = 0; k < 3; ++k) {
+        T.v10[k] = L.v10[k];
+        v21[k] = (double)N.v[6 + k] - (double)N.v[3 + k];
+        T.v02[k] = -L.e2[k];
+    }
+    cross3(T.v10, T.v02, T.nor);
+    cross3(T.v10, T.nor, T.c10);
+    cross3(v21, T.nor, T.c21);
+    cross3(T.v02, T.nor, T.c02);
+    T.i10 = N.i10;
+    T.i21 = N.i21;
+    T.i02 = N.i02;
+    T.inor = N.inor;
+    for (int d = 0; d < kDirs; ++d) {
+        for (int k = 0; k < 3; ++k) T.pvec[d][k] = L.dir[d].pvec[k];
+        T.idet[d] = L.dir[d].idet;
+    }
+    out[f] = T;
+}
+
+__global__ __launch_bounds__(256) void mesh_pairs_kernel(const float* __restrict__ pts, int64_t n, uint32_t nf,
+                                                         uint32_t lanes, const PairTri* __restrict__ tris,
+                                                         float* __restrict__ dist, double* __restrict__ dist64) {
+    NGLOD_FP64_CONTRACT
+    __shared__ double tile[kPairTile * kPairStride];
+    const uint32_t q = threadIdx.x % lanes;
+    const int64_t i = (int64_t)blockIdx.x * (256 / lanes) + threadIdx.x / lanes;
+    const int64_t at = i < n ? i : n - 1;
+    const double p[3] = {pts[3 * at], pts[3 * at + 1], pts[3 * at + 2]};
+    double best = INFINITY;
+    uint32_t flags = 0;
+    for (uint32_t f0 = 0; f0 < nf; f0 += kPairTile) {
+        const uint32_t cnt = min((uint32_t)kPairTile, nf - f0);
+        const double* src = reinterpret_cast<const double*>(tris + f0);
+        __syncthreads();
+        for (uint32_t w = threadIdx.x; w < cnt * kPairWords; w += 256)
+            tile[w / kPairWords * kPairStride + w % kPairWords] = src[w];
+        __syncthreads();
+        for (uint32_t k = q; k < cnt; k += lanes) {
+            const PairTri& T = *reinterpret_cast<const PairTri*>(tile + k * kPairStride);
+            const double p0[3] = {p[0] - T.v[0], p[1] - T.v[1], p[2] - T.v[2]};
+            const double v21[3] = {(double)T.v[6] - T.v[3], (double)T.v[7] - T.v[4], (double)T.v[8] - T.v[5]};
+            if (!T.degenerate)
+                best = fmin(best, edge_face_dist2(T, p0, p, T.v10, v21, T.v02, T.nor, T.c10, T.c21, T.c02));
+            double qvec[3];
+            cross3(p0, T.v10, qvec);
+            const double e2[3] = {-T.v02[0], -T.v02[1], -T.v02[2]};
+            const double tnum = dot3(e2, qvec);
+#pragma unroll
+            for (int d = 0; d < kDirs; ++d) {
+                const double inv = T.idet[d];
+                if (inv == 0.0) continue;
+                const double u = dot3(p0, T.pvec[d]) * inv;
+                if (u < 0.0 || u > 1.0) continue;
+                const double dir[3] = {kStab[d][0], kStab[d][1], kStab[d][2]};
+                const double w = dot3(dir, qvec) * inv;
+                if (w < 0.0 || u + w > 1.0) continue;
+                flags |= tnum * inv >= 0.0 ? 1u << d : 1u << (kDirs + d);
+            }
+        }
+    }
+    for (uint32_t o = lanes / 2; o > 0; o >>= 1) {
+        best = fmin(best, __shfl_xor(best, (int)o));
+        flags |= (uint32_t)__shfl_xor((int)flags, (int)o);
+    }
+    if (i >= n || q != 0) return;
+    const double d = flags == (1u << 2 * kDirs) - 1u ? -sqrt(best) : sqrt(best);
+    dist[i] = (float)d;
+    if (dist64) dist64[i] = d;
+}
+
+// ---------------------------------------------------------------------------
 static size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
 struct SdfLayout {
@@ -743,6 +868,19 @@ static void sdf_layout(int64_t n, int64_t nf, SdfLayout* L) {
 constexpr int64_t kMaxFaces = (int64_t)1 << 30;
 constexpr int64_t kMaxOrdered = (int64_t)1 << 31;
 
+// Lanes per point for every point against every triangle; 0: the tree.  Icospheres and a
+// cube, us, tree / pairs: 12 triangles 110 / 13 with 1000 points, 274 / 72 with 2^19, 687 /
+// 247 with 2^21; 20 triangles 687 / 475; 80 triangles 240 / 22 with 1000, 342 / 273 with
+// 2^18, 485 / 513 with 2^19; 320 triangles 414 / 61 with 1000, 411 / 229 with 16000, 407 / 399
+// with 64000; 1280 triangles 681 / 214 with 1000, 730 / 459 with 4000, 700 / 858 with 16000 (5120:
+// 1286 / 821 and 1218 / 1795 with 1000 and 4000, and one point 400 / 814).  Lanes, 80 triangles: 4000
+// points 41 with 64, 63 with 4, 190 with 1; 16000 130, 64, 190; 64000 467, 111, 192; 2^18
+// 1848, 399, 273: beyond 4 the lanes' different triangles are bank conflicts.
+static uint32_t pair_lanes(int64_t n, int64_t nf) {
+    if (n <= 4096 ? nf > 1280 : nf > 24 && (nf > 320 || n * nf > (int64_t)1 << 24)) return 0;
+    return n <= 4096 ? 64 : n <= 1 << 16 ? 4 : n <= 1 << 17 ? 2 : 1;
+}
+
 }  // namespace nglod
 
 using namespace nglod;
@@ -785,6 +923,13 @@ int nglod_mesh2sdf_f64(const float* points, int64_t n, const float* mesh, int64_
     t.slabs = (Slabs*)(w + L.slabs);
     float* bounds = (float*)(w + L.bounds);
     const uint32_t nt = (uint32_t)nf;
+    if (const uint32_t lanes = pair_lanes(n, nf)) {
+        hipLaunchKernelGGL(pair_records_kernel, dim3((nt + 127) / 128), dim3(128), 0, s, mesh, nt, (PairTri*)w);
+        const int64_t per = 256 / lanes;
+        hipLaunchKernelGGL(mesh_pairs_kernel, dim3((unsigned)((n + per - 1) / per)), dim3(256), 0, s, points, n, nt,
+                           lanes, (const PairTri*)w, dist, dist64);
+        return check_launch("mesh_pairs_kernel");
+    }
     const SortBuffers ts = sort_buffers(w + L.sort, nf);
     hipLaunchKernelGGL(mesh_bounds_kernel, dim3(kBoundsBlocks), dim3(256), 0, s, mesh, nf, bounds);
     hipLaunchKernelGGL(tri_keys_kernel, dim3((nt + 255) / 256), dim3(256), 0, s, mesh, nt, bounds, ts.keys[0]);
