@@ -597,7 +597,8 @@ int nglod_shadow_rays(const float* ray_o, const float* ray_d, int64_t n, float g
                       const float* noise, float* x, float* t, uint8_t* hit, float* normal, uint8_t* plane_hit,
                       float* shadow_o, float* shadow_d, uint8_t* light_hit, void* stream);
 
-/* Workspace bytes of nglod_ao (one claim counter; reset by every call). */
+/* Workspace bytes of nglod_ao (claim counters; reset by every call).  From 256
+ * bytes on a smaller one will do, with a single counter. */
 size_t nglod_ao_workspace_size(void);
 
 /* Ambient occlusion (sdf-net/lib/renderer.py:184-209): per ray with hit[i]
