@@ -258,9 +258,10 @@ struct SolRay {
     }
 };
 
-// Persistent sparse march of structures with more than kSolGroupLevels levels or
-// tables off their vectors' alignment (the others: launch_trace_sparse_group): one ray per lane (SolRay), refilled from kQueues
-// ray ranges (RayFeed); the features come from the sparse corner table, the
+// Persistent sparse march with a ray per lane (SolRay), refilled from kQueues ray ranges
+// (RayFeed), for the frames that march_by_lanes names, for structures with more than
+// kSolGroupLevels levels and for tables off their vectors' alignment (the others:
+// launch_trace_sparse_group).  The features come from the sparse corner table, the
 // decoder is the FP32 MFMA one of the dense form (fp32_wave.hpp), staged in
 // LDS once per block.  512-thread blocks, as the dense FP32 march.
 // 512 and 256 threads measured the same (3.23 / 3.25 ms on the 1280x720 LOD-4
@@ -548,6 +549,17 @@ int nglod_sol_trinkets(const int16_t* points, const int32_t* pyramid, int32_t le
     return NGLOD_OK;
 }
 
+// Whether a frame of a coarse level is large enough for a ray per lane: an evaluation of
+// few levels is cheap, and the groups' barriers and fourfold state are not.  The object seen
+// from far / filling the view, us, groups / lanes: LOD 0 with 480x270 rays 435 / 629 and
+// 284 / 208, 640x360 594 / 700 and 455 / 346, 1280x720 1713 / 1444 and 1540 / 1131; LOD 1 with
+// 640x360 612 / 788 and 491 / 431, 960x540 1032 / 1130 and 1007 / 838, 1280x720 1644 / 1633 and
+// 1717 / 1383; LOD 2 with 1280x720 1673 / 1896 and 1827 / 1623, 1920x1080 3400 / 3588 and
+// 4048 / 3484; LOD 3 with 1920x1080 3390 / 4177 and 4396 / 4352.
+static bool march_by_lanes(int lod, int64_t n) {
+    return lod == 0 ? n > 1 << 17 : lod == 1 ? n > 1 << 18 : lod == 2 && n > 1 << 20;
+}
+
 static int sol_args(const nglod_sol_t* sol, SolArgs& a) {
     if (!sol) return fail(NGLOD_ERR_ARG, "sol is NULL");
     if (sol->target < 2 || sol->target > 12 || sol->lod != sol->target - 2)
@@ -621,7 +633,7 @@ int nglod_trace_sparse(const nglod_sol_t* sol, const float* ray_o, const float* 
     rc = check_launch("clear_counters_kernel");
     if (rc) return rc;
     const bool posinv = a.din == kC;
-    if (a.lod < kSolGroupLevels && ((uintptr_t)a.points & 7u) == 0 && aligned16(a.cf))
+    if (a.lod < kSolGroupLevels && ((uintptr_t)a.points & 7u) == 0 && aligned16(a.cf) && !march_by_lanes(a.lod, n))
         return launch_trace_sparse_group(a, s);
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
