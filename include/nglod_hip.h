@@ -420,8 +420,8 @@ int nglod_sdf_bwd(const nglod_model_t* model, const float* x, int64_t n, int32_t
                   void* workspace, size_t workspace_bytes, void* stream);
 
 /* The training forward: nglod_sdf_fwd_all's predictions (the same bits), and
- * in `saved` (nglod_sdf_fwd_save_bytes bytes, 16-byte aligned: 164 bytes per
- * query and level at most) what nglod_sdf_bwd_saved then need not compute again:
+ * in `saved` (nglod_sdf_fwd_save_bytes bytes, 16-byte aligned: up to 164 bytes per
+ * query and level, and 256 for each of its parts' alignment) what nglod_sdf_bwd_saved then need not compute again:
  * the spatial order of the queries, their features and the signs of the
  * decoders' pre-activations.  n <= 2^28. */
 size_t nglod_sdf_fwd_save_bytes(const nglod_model_t* model, int64_t n, int32_t lod);

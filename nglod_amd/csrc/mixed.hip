@@ -194,9 +194,6 @@ __device__ __forceinline__ void add_evals(const TraceArgs& a, int slot, uint32_t
     if (lane == 0 && tot) atomicAdd(a.evals + slot, tot);
 }
 
-// RESUME: a later round, over the rays pass 2 handed back (ret, rflag)
-// instead of the frame's rays.  A separate instantiation: compiled into the
-// first-round kernel, the resume path slowed its march by half even unused.
 // Up to this many busy lanes, a drained wave of the pooled passes
 // gathers cooperatively (16 lanes per query).
 constexpr int kCoopLanes = 4;
@@ -206,6 +203,9 @@ constexpr int kCoopLanes = 4;
 // against 0.69 ms on the 1280x720 frame.
 constexpr int kPass1CoopLanes = 8;
 
+// RESUME: a later round, over the rays pass 2 handed back (ret, rflag)
+// instead of the frame's rays.  A separate instantiation: compiled into the
+// first-round kernel, the resume path slowed its march by half even unused.
 template <bool POSINV, bool RESUME>
 __global__ __launch_bounds__(kMixedBlock) void trace_mixed_pass1_kernel(TraceArgs a) {
     __shared__ MixedLds lds;
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(kMixedBlock) void trace_mixed_pass1_kernel(TraceArg
         const bool busy = s.phase != PH_IDLE;
         __half2 acc[kC / 2];
         gather_fp16_cum(a.m, busy, s.qx, s.qy, s.qz, acc);
-        const float d = decode_mixed_wave<POSINV>(acc, &lds, b1, lane, busy, s.qx, s.qy, s.qz);
+        const float d = decode_mixed_wave<POSINV>(acc, &lds, b1, lane, s.qx, s.qy, s.qz);
         if (busy) {
             ++nevals;
             hist.push(s);
@@ -506,8 +506,7 @@ struct PoolMixedSlot {
     float b1;
 };
 
-// A wave's LDS slot in the pooled FP32 passes: decoder, level table, b1 and
-// the one-query-at-a-time tail's hidden vector.
+// A wave's LDS slot in the pooled FP32 passes: decoder, level table and b1.
 struct PoolFp32Slot {
     Fp32Lds dec;
     SoloLevels lv;
@@ -722,8 +721,8 @@ __device__ __forceinline__ int64_t pool_next_flagged(RayFeed& f, const PoolArgs&
 }
 
 // Pass 2 over the pool: FP32 continuation of the handed-off rays, claimed in
-// virtual-id order (flags indexed by pool slot), with the one-query-at-a-time
-// tail of the single-request pass.
+// virtual-id order (flags indexed by pool slot); a wave's last few rays spread
+// their gathers over the idle lanes.
 template <bool POSINV>
 __global__ __launch_bounds__(kPoolFp32Block) void pool_pass2_kernel(TraceArgs a, PoolArgs p) {
     __shared__ PoolFp32Slot slots[kPoolFp32Block / 64];

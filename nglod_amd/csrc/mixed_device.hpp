@@ -169,16 +169,15 @@ __device__ __forceinline__ float layer2_partial(f32x16 c, int h, uint32_t half, 
     return acc;
 }
 
-// SDF of the 64 lanes' query points.  Every lane of the wave must call this
-// (no divergent branch around it): the MFMAs and lane swaps are wave-wide.
-// Lanes without a query pass active = false: they load nothing, and a
-// 32-query tile with no active lane skips its MFMAs.  Each output column
-// depends only on its own query.
 // The decoder on the 64 lanes' FP16 feature sums acc (zero on inactive
-// lanes); wave-wide, as sdf_mixed_wave.
+// lanes).  Every lane of the wave must call this (no divergent branch around it):
+// the MFMAs and lane swaps are wave-wide, for both 32-query tiles whether used or
+// not (in one block a tile's ReLU runs beside the other's products;
+// decode_mixed_wave_few skips an unused tile).  Each output column depends only
+// on its own query.
 template <bool POSINV>
 __device__ __forceinline__ float decode_mixed_wave(const __half2 (&acc)[kC / 2], const MixedLds* s, float b1,
-                                                   uint32_t lane, bool active, float px, float py, float pz) {
+                                                   uint32_t lane, float px, float py, float pz) {
     const uint32_t half = lane >> 5;
     // own channels 16kb + 0..7 (Y) and 16kb + 8..15 (X) as bf16; one
     // v_permlane32_swap per word gives tile 0 (own Y | X of lane l-32) and
@@ -262,12 +261,14 @@ __device__ __forceinline__ float decode_mixed_wave_few(const __half2 (&acc)[kC /
     return halves_sum(part[0], part[1]) + b1;
 }
 
+// SDF of the 64 lanes' query points, wave-wide as decode_mixed_wave.  Lanes without a
+// query pass active = false: they load nothing.
 template <bool POSINV, typename LV>
 __device__ __forceinline__ float sdf_mixed_wave(const LV& m, const MixedLds* s, float b1, uint32_t lane,
                                                 bool active, float px, float py, float pz) {
     __half2 acc[kC / 2];
     gather_fp16_cum(m, active, px, py, pz, acc);
-    return decode_mixed_wave<POSINV>(acc, s, b1, lane, active, px, py, pz);
+    return decode_mixed_wave<POSINV>(acc, s, b1, lane, px, py, pz);
 }
 
 // FP16 grid pointers and resolutions, copied to LDS so that the cooperative

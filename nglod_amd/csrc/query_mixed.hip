@@ -26,7 +26,7 @@ __global__ __launch_bounds__(256) void sdf_mixed_kernel(ModelArgs m, int dec, co
     if (__ballot(valid) == 0) return;  // whole wave past the end (no barrier follows)
     __half2 acc[kC / 2];
     gather_fp16_cum(m, valid, px, py, pz, acc);
-    const float d = decode_mixed_wave<POSINV>(acc, &lds, b1, lane, valid, px, py, pz);
+    const float d = decode_mixed_wave<POSINV>(acc, &lds, b1, lane, px, py, pz);
     if (valid) out[i] = d;
 }
 

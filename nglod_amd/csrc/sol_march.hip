@@ -257,11 +257,11 @@ __device__ __forceinline__ void group_claim(const SolArgs& a, SolGroupLds* s, Ra
 // units per wave.  The rows of a ray's corners are looked up only when its voxel
 // changes, those of the coarser levels only when its parent does (most
 // evaluations, the six normal taps among them, stay in theirs), and a corner's
-// coordinates come from its voxel's.  Bound: the latency of a trip's dependent
-// loads and barriers (waves wait half of their cycles), vector ALU 48%; four
-// blocks a CU by registers and LDS.  1280x720, LOD 4, 5.4 M evaluations: one ray
-// per lane 2.71 ms; by groups, corners and voxels looked up in every trip 2.60;
-// this 1.84.
+// coordinates come from its voxel's.  Bound: the vector memory path (TA busy 56%, TD
+// 68% of the cycles) and the vector ALU (47%), in trips of dependent loads and
+// barriers (waves wait for memory 28% of theirs); four blocks a CU by registers.
+// 1280x720, LOD 4, 5.4 M evaluations: one ray per lane 2.71 ms; by groups, corners
+// and voxels looked up in every trip 2.60; this 1.84.
 template <bool POSINV>
 __global__ __launch_bounds__(kGroupThreads, 4) void trace_sparse_group_kernel(SolArgs a) {
     __shared__ SolGroupLds lds;

@@ -146,12 +146,13 @@ __device__ __forceinline__ f32x16 split_tile(const bf16x8 (&ah)[2], const bf16x8
 
 // The decoder on the 64 lanes' FP32 feature vectors f (zero on inactive
 // lanes).  Every lane of the wave must call this (no divergent branch around
-// it): the MFMAs and lane swaps are wave-wide.  A 32-query tile with no
-// active lane skips its MFMAs; each output column depends only on its own
-// query, so a lane's result is the same whatever the other lanes hold.
+// it): the MFMAs and lane swaps are wave-wide, for both 32-query tiles whether
+// used or not (in one block a tile's ReLU runs beside the other's products;
+// decode_split_wave_few skips an unused tile).  Each output column depends only on
+// its own query, so a lane's result is the same whatever the other lanes hold.
 template <bool POSINV, typename LDS>
-__device__ __forceinline__ float decode_split_wave(const float (&f)[kC], const LDS* s, float b1, uint32_t lane,
-                                                   bool active, float px, float py, float pz) {
+__device__ __forceinline__ float decode_split_wave(const float (&f)[kC], const LDS* s, float b1, uint32_t lane, float px,
+                                                   float py, float pz) {
     const uint32_t half = lane >> 5;
     // [tile][kb] B operands of the three parts
     bf16x8 Bh[2][2], Bm[2][2], Bl[2][2];
@@ -290,7 +291,7 @@ __device__ __forceinline__ float sdf_split_wave(const LV& lv, const LDS* s, floa
                                                 float px, float py, float pz) {
     float f[kC];
     gather_fp32_cum(lv, active, px, py, pz, f);
-    return decode_split_wave<POSINV, LDS>(f, s, b1, lane, active, px, py, pz);
+    return decode_split_wave<POSINV, LDS>(f, s, b1, lane, px, py, pz);
 }
 
 // gather_fp32_cum for the busy lanes of a wave with at most 4 of them (act,

@@ -15,8 +15,9 @@ namespace nglod {
 //
 // Bound: small frames by the length of the longest ray times a trip's latency
 // (about 2 us: the dependent loads, three barriers, 16 MFMAs in a row), large ones
-// by the corner rows through the vector L1 (56% of its cycles at 1280x720, vector
-// ALU 50%, matrix cores 27%) and by the four blocks a CU that the registers
+// by the corner rows through the vector L1 (TA busy 59%, TD 67% of the cycles at
+// 1280x720), the FP32 units (vector ALU 47%, matrix cores 27%: not beside each other on a
+// SIMD) and by the four blocks a CU that the registers
 // allow: three measured a quarter slower, also with a second level's rows in
 // flight.  A whole frame, 5 LODs, against one ray per lane and 64 rays a wave:
 // 64x48 1339 -> 365 us, 128x96 1367 -> 430, 320x180 1445 -> 677, 1280x720 4091 ->

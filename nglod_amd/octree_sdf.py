@@ -255,9 +255,10 @@ class OctreeSDF(nn.Module):
         SphereTracer.forward applies to its normals.  No autograd graph.
         ordered: None picks by batch size, True / False forces the evaluation in
         cell / input order (the same results; a frame's points are neighbours
-        already).  Uniform points at LOD 4, both ways in us: autodiff 117 / 105
-        with 2^16 points, 140 / 174 with 2^17; finite differences 212 / 251 with
-        2^13, at LOD 1 148 / 221 with 2^17; tetrahedron 181 / 185 with 2^15."""
+        already).  Uniform points, cell / input order in us: autodiff at LOD 4 117 /
+        105 with 2^16 points, 140 / 174 with 2^17.  The taps' line is no crossing: with
+        2^13, 2^15 points finite differences take 210 / 247, 225 / 266 at LOD 4 and 103 /
+        117, 112 / 119 at LOD 1, the tetrahedron 157 / 171, 176 / 183 and 82 / 85, 97 / 86."""
         if method not in _lib.GRAD_METHODS:
             raise NotImplementedError(f"gradient method {method!r}")
         xf = x.detach().reshape(-1, 3).float().contiguous()
