@@ -19,7 +19,7 @@ def _param_slots(net, params):
     for i, f in enumerate(net.features):
         slots.setdefault(id(f.fm), ("grid", i))
     for i, l in enumerate(net.louts):
-        first, _, last = list(l)[:3]
+        first, _, last, *_ = l
         slots.setdefault(id(first.weight), ("w0", i))
         slots.setdefault(id(first.bias), ("b0", i))
         slots.setdefault(id(last.weight), ("w1", i))

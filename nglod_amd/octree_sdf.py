@@ -174,7 +174,7 @@ class OctreeSDF(nn.Module):
             res[i] = f.fsize
             grid[i] = address(f.fm, True)
         for i, l in enumerate(self.louts):
-            first, _, last = list(l)[:3]
+            first, _, last, *_ = l
             w0[i] = address(first.weight, False)
             b0[i] = address(first.bias, False)
             w1[i] = address(last.weight, False)
