@@ -430,7 +430,7 @@ int nglod_sdf_fwd_save(const nglod_model_t* model, const float* x, int64_t n, in
                        size_t saved_bytes, void* workspace, size_t workspace_bytes, void* stream);
 
 /* nglod_sdf_bwd on what nglod_sdf_fwd_save left for the same model, x, n and
- * lod; the same gradients, bit for bit. */
+ * lod (the weights as they were then); the same gradients, bit for bit. */
 size_t nglod_sdf_bwd_saved_workspace_size(const nglod_model_t* model, int64_t n, int32_t lod);
 int nglod_sdf_bwd_saved(const nglod_model_t* model, const float* x, int64_t n, int32_t lod, const float* grad_out,
                         int32_t level_mask, const nglod_model_grads_t* grads, void* saved, size_t saved_bytes,
@@ -468,7 +468,8 @@ size_t nglod_mesh2sdf_ordered_workspace_size(int64_t n, int64_t nf);
  * (:341-353) have a hit on both sides of the point (:479-529, :584-602).
  * dist [n] fp32; dist64 [n] fp64 (may be NULL).  workspace: 8-byte aligned, at
  * least nglod_mesh2sdf_workspace_size(nf) bytes; the points are ordered when it
- * has nglod_mesh2sdf_ordered_workspace_size(n, nf). */
+ * has nglod_mesh2sdf_ordered_workspace_size(n, nf), unless there are so few pairs of
+ * points and triangles that each is tested. */
 int nglod_mesh2sdf_f64(const float* points, int64_t n, const float* mesh, int64_t nf, float* dist,
                        double* dist64, void* workspace, size_t workspace_bytes, void* stream);
 
