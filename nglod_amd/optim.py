@@ -76,6 +76,8 @@ class Adam(torch.optim.Adam):
                     return None
                 rows.append((p, g, avg, sq, step))
             found.append((group, rows))
+        if not fresh and not any(rows for _, rows in found):
+            return None  # no gradients: nothing on any device
         if torch.cuda.is_current_stream_capturing():
             return None  # torch's step says what capture needs
         plans = []
